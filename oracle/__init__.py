@@ -31,10 +31,10 @@ _F = ctypes.c_float
 
 
 def build(ref: bool | None = None) -> None:
-    """Compile liboracle.so (and _ref/libytref.so when the reference exists)."""
+    """Compile liboracle.so (and _ref/libytref.so when the reference's sources are there)."""
     subprocess.check_call(["make", "-s", "-C", HERE, "all"])
     if ref is None:
-        ref = os.path.isdir(REF_ROOT)
+        ref = os.path.isfile(os.path.join(REF_ROOT, "ytensor.hpp"))
     if ref:
         subprocess.check_call(["make", "-s", "-C", HERE, "ref"])
 
