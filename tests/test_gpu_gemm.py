@@ -403,3 +403,70 @@ def test_one_phase_tiles_c_row_strides(yt, m, n, k, layout):
     yt.gemm(a, b, out, alpha=0.5)
     torch.cuda.synchronize()
     assert torch.equal(out.view(torch.int16), ref.contiguous().view(torch.int16))
+
+
+# Edges of the any-layout kernel and of the short first k step: k below, at and past
+# a 16-byte chunk (8 / 4 elements) and a k step (64 / 32), m and n below a group of
+# 4 rows, at and past the 64- and 128-wide tiles (3000 x 3100: 128-wide ones).
+ANY_SHAPES = [(1, 1, 1), (2, 3, 5), (5, 3, 7), (3, 66, 8), (64, 64, 64), (65, 63, 65), (67, 130, 31), (130, 68, 33),
+              (1, 1003, 779), (17, 40, 1000), (129, 257, 136), (120, 200, 72), (3000, 3100, 45), (3000, 3104, 72)]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN", "TT", "SN", "NS", "offset", "c_cols", "c_strided"])
+@pytest.mark.parametrize("shape", ANY_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_any_layout_edges(yt, shape, layout, dtype):
+    """Every operand layout (row-major, transposed, every other element "S",
+    one element past an aligned base, a column-major and a strided C) at the
+    edge sizes, with alpha / beta and a batch of two, against float64 on the same
+    16-bit / fp32 inputs. Bound: the 32-bit sum of k products in any order,
+    (k + 2) 2^-24 sum|a||b|, plus the rounding of the result."""
+    m, n, k = shape
+    td = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[dtype]
+    g = torch.Generator(device="cuda").manual_seed(m * 31 + n * 7 + k)
+
+    def operand(rows, cols, how):
+        if how == "T":
+            return torch.randn(2, cols, rows, device="cuda", generator=g).to(td).transpose(1, 2)
+        if how == "S":
+            return torch.randn(2, rows, 2 * cols, device="cuda", generator=g).to(td)[:, :, ::2]
+        if how == "offset":
+            flat = torch.randn(2 * rows * cols + 1, device="cuda", generator=g).to(td)
+            return flat[1:].view(2, rows, cols)
+        return torch.randn(2, rows, cols, device="cuda", generator=g).to(td)
+
+    how = layout if len(layout) == 2 else (["offset"] * 2 if layout == "offset" else "NN")
+    A, B = operand(m, k, how[0]), operand(k, n, how[1])
+    C = operand(m, n, {"c_cols": "T", "c_strided": "S", "offset": "offset"}.get(layout, "N"))
+    C0 = C.clone()
+    yt.gemm(A, B, C, 0.5, 2.0)
+    prod = A.double() @ B.double()
+    mass = A.double().abs() @ B.double().abs()
+    want = 0.5 * prod + 2.0 * C0.double()
+    ulp = {"f32": 2.0 ** -23, "bf16": 2.0 ** -8, "f16": 2.0 ** -10}[dtype]
+    bound = (k + 2) * 2.0 ** -24 * mass + ulp * want.abs() + 4 * 2.0 ** -23 * C0.double().abs() + 1e-7
+    assert ((C.double() - want).abs() <= bound).all(), ((C.double() - want).abs() - bound).max().item()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("layout", ["NN", "NT", "NT_odd"])
+def test_ragged_k_reads_nothing_past_it(yt, layout, dtype):
+    """What lies past k in a padded row, past n in a padded k-row and after the
+    operands' last element is NaN here: the short first k step takes zeros for it
+    in both operands, so the product is that of the clean operands bit for bit."""
+    td = {"f32": torch.float32, "bf16": torch.bfloat16}[dtype]
+    for m, n, k in [(70, 72, 40), (129, 136, 72), (64, 200, 1000), (20, 24, 8)]:
+        k -= layout == "NT_odd"
+        g = torch.Generator(device="cuda").manual_seed(m + n + k)
+        pad = 8
+        A = torch.full((m + 1, k + pad), float("nan"), device="cuda", dtype=td)
+        A[:m, :k] = torch.randn(m, k, device="cuda", generator=g).to(td)
+        rows, cols = (k, n) if layout == "NN" else (n, k)
+        B = torch.full((rows + 1, cols + pad), float("nan"), device="cuda", dtype=td)
+        B[:rows, :cols] = torch.randn(rows, cols, device="cuda", generator=g).to(td)
+        Bv = B[:rows, :cols] if layout == "NN" else B[:rows, :cols].t()
+        C = torch.empty(m, n, device="cuda", dtype=td)
+        yt.gemm(A[:m, :k], Bv, C)
+        Ac, Bc = A[:m, :k].contiguous(), B[:rows, :cols].contiguous()
+        want = yt.matmul(Ac, Bc if layout == "NN" else Bc.t())
+        assert torch.isfinite(C).all() and torch.equal(C, want)

@@ -23,8 +23,8 @@
 //  * Tiles are assigned XCD-aware: the hardware places workgroup w on XCD
 //    w % 8; each XCD receives a contiguous, M-grouped range of tiles so its
 //    32 CUs share A and B panels in their own L2.
-//  * The register-staged kernel (gemm_mfma_kernel) serves layouts the DMA path
-//    cannot take (k not a multiple of the k step, 4-byte-aligned NN rows).
+//  * What the DMA cannot take (rows that are not 16-byte aligned, k or n that are
+//    no whole chunks, a transposed A, other strides) runs in gemm_any.hip.
 
 #include "common.hpp"
 #include "launch.hpp"
@@ -44,8 +44,6 @@ struct GemmArgs {
     int c_line_ok;  // 16-bit C: 16-byte aligned base and rows (the ping-pong kernel's line stores)
 };
 
-__device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row ^ (row >> 3)) & 7); }
-
 // Swizzles of the DMA-staged kernel, chosen by measuring gfx950's LDS read rate
 // per access pattern (64 banks; ds_read_b128 and ds_read_b64_tr_b16):
 //  * K-major tiles [row][8 x 16 B]: chunk c of row r at c ^ ((r >> 1) & 7). Rows
@@ -57,210 +55,6 @@ __device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row ^ 
 //    k-rows r and r + 8 (served together) land in different blocks.
 __device__ __forceinline__ int swz_dma(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 __device__ __forceinline__ int nn_blk(int row, int blk, int mask) { return blk ^ ((row ^ ((row >> 3) << 2)) & mask); }
-
-template <class T, class TO, int BM, int BN, int WM, int WN, bool NN>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(GemmArgs a) {
-    using raw = typename T::raw;
-    constexpr int THREADS = 64 * WM * WN;
-    constexpr int VEC = 16 / sizeof(raw);      // elements per 16-byte chunk
-    constexpr int BK = 8 * VEC;                 // elements per k step (128 bytes)
-    constexpr int WTM = BM / WM, WTN = BN / WN; // wave tile
-    constexpr int FM = WTM / 16, FN = WTN / 16;
-    constexpr int A_CHUNKS = BM * 8, B_CHUNKS = BN * 8;
-    constexpr int A_PT = (A_CHUNKS + THREADS - 1) / THREADS;
-    constexpr int B_PT = (B_CHUNKS + THREADS - 1) / THREADS;
-    constexpr int NN_GROUPS = 8 * (BN / 4);     // VEC k-rows x 4 columns each
-    constexpr int NN_PT = (NN_GROUPS + THREADS - 1) / THREADS;
-    constexpr int STAGE = (BM + BN) * 8;        // u32x4 slots per stage
-
-    __shared__ u32x4 lds[2 * STAGE];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int wm = wave / WN, wn = wave % WN;
-
-    int tm, tn;
-    tile_coords(blockIdx.x, a.tiles_m, a.tiles_n, tm, tn);
-    const int m0 = tm * BM, n0 = tn * BN;
-    const int bz = blockIdx.y;
-
-    const raw* __restrict__ Ap = static_cast<const raw*>(a.A) + bz * a.sa_b;
-    const raw* __restrict__ Bp = static_cast<const raw*>(a.B) + bz * a.sb_b;
-
-    const int KT = (a.k + BK - 1) / BK;
-
-    u32x4 ra[A_PT];
-    u32x4 rb[NN ? 1 : B_PT];
-    // NN staging: VEC rows of 4 columns each (8 bytes for 16-bit, 16 bytes for fp32)
-    using nn_row_t = typename std::conditional<sizeof(raw) == 2, u32x2, u32x4>::type;
-    nn_row_t rn[NN ? NN_PT : 1][NN ? VEC : 1];
-
-    auto load_global = [&](int kt) {
-        const int k0 = kt * BK;
-#pragma unroll
-        for (int i = 0; i < A_PT; ++i) {
-            const int id = tid + i * THREADS;
-            const int r = id >> 3, c = id & 7;
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if ((A_CHUNKS % THREADS == 0 || id < A_CHUNKS) && m0 + r < a.m && k0 + c * VEC < a.k)
-                v = *reinterpret_cast<const u32x4*>(Ap + (int64_t)(m0 + r) * a.rsa + (k0 + c * VEC));
-            ra[i] = v;
-        }
-        if constexpr (!NN) {
-#pragma unroll
-            for (int i = 0; i < B_PT; ++i) {
-                const int id = tid + i * THREADS;
-                const int r = id >> 3, c = id & 7;
-                u32x4 v = {0u, 0u, 0u, 0u};
-                if ((B_CHUNKS % THREADS == 0 || id < B_CHUNKS) && n0 + r < a.n && k0 + c * VEC < a.k)
-                    v = *reinterpret_cast<const u32x4*>(Bp + (int64_t)(n0 + r) * a.csb + (k0 + c * VEC));
-                rb[i] = v;
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < NN_PT; ++i) {
-                const int id = tid + i * THREADS;
-                const int g = id % (BN / 4), kc = id / (BN / 4);
-                const int col = n0 + g * 4;
-                const bool ok = (NN_GROUPS % THREADS == 0 || id < NN_GROUPS) && col < a.n;
-#pragma unroll
-                for (int r = 0; r < VEC; ++r) {
-                    const int kk = k0 + kc * VEC + r;
-                    nn_row_t v = {};
-                    if (ok && kk < a.k) v = *reinterpret_cast<const nn_row_t*>(Bp + (int64_t)kk * a.rsb + col);
-                    rn[i][r] = v;
-                }
-            }
-        }
-    };
-
-    auto store_lds = [&](int stage) {
-        u32x4* sA = lds + stage * STAGE;
-        u32x4* sB = sA + BM * 8;
-#pragma unroll
-        for (int i = 0; i < A_PT; ++i) {
-            const int id = tid + i * THREADS;
-            if (A_CHUNKS % THREADS == 0 || id < A_CHUNKS) {
-                const int r = id >> 3, c = id & 7;
-                sA[r * 8 + swz(r, c)] = ra[i];
-            }
-        }
-        if constexpr (!NN) {
-#pragma unroll
-            for (int i = 0; i < B_PT; ++i) {
-                const int id = tid + i * THREADS;
-                if (B_CHUNKS % THREADS == 0 || id < B_CHUNKS) {
-                    const int r = id >> 3, c = id & 7;
-                    sB[r * 8 + swz(r, c)] = rb[i];
-                }
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < NN_PT; ++i) {
-                const int id = tid + i * THREADS;
-                if (NN_GROUPS % THREADS == 0 || id < NN_GROUPS) {
-                    const int g = id % (BN / 4), kc = id / (BN / 4);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        u32x4 o;
-                        if constexpr (sizeof(raw) == 2) {
-                            // out[j] = column j's VEC k-values: half-word j of each row, paired.
-#pragma unroll
-                            for (int q = 0; q < 4; ++q) {
-                                const uint32_t lo = rn[i][2 * q][j >> 1];
-                                const uint32_t hi = rn[i][2 * q + 1][j >> 1];
-                                o[q] = (j & 1) ? ((lo >> 16) | (hi & 0xffff0000u)) : ((lo & 0xffffu) | (hi << 16));
-                            }
-                        } else {
-#pragma unroll
-                            for (int q = 0; q < 4; ++q) o[q] = rn[i][q][j];
-                        }
-                        const int row = g * 4 + j;
-                        sB[row * 8 + swz(row, kc)] = o;
-                    }
-                }
-            }
-        }
-    };
-
-    f32x4 acc[FM][FN];
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    load_global(0);
-    store_lds(0);
-    __syncthreads();
-
-    const int lrow = lane & 15;
-    const int lgrp = lane >> 4;
-
-    for (int kt = 0; kt < KT; ++kt) {
-        const int cur = kt & 1;
-        if (kt + 1 < KT) load_global(kt + 1);
-        const u32x4* sA = lds + cur * STAGE;
-        const u32x4* sB = sA + BM * 8;
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const int chunk = ks * 4 + lgrp;
-            u32x4 fa[FM], fb[FN];
-#pragma unroll
-            for (int i = 0; i < FM; ++i) {
-                const int r = wm * WTM + i * 16 + lrow;
-                fa[i] = sA[r * 8 + swz(r, chunk)];
-            }
-#pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                const int r = wn * WTN + j * 16 + lrow;
-                fb[j] = sB[r * 8 + swz(r, chunk)];
-            }
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j) acc[i][j] = mfma_chunk(T{}, fb[j], fa[i], acc[i][j]);
-        }
-        if (kt + 1 < KT) store_lds(cur ^ 1);
-        __syncthreads();
-    }
-
-    // Epilogue: lane holds C[m][n..n+3] for m = row lrow, n = 4*lgrp + r.
-    using oraw = typename TO::raw;
-    oraw* Cp = static_cast<oraw*>(a.C) + bz * a.sc_b;
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-        const int m = m0 + wm * WTM + i * 16 + lrow;
-        if (m >= a.m) continue;
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            const int n = n0 + wn * WTN + j * 16 + lgrp * 4;
-            if (n >= a.n) continue;
-            oraw* crow = Cp + (int64_t)m * a.rsc;
-            float v[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = a.alpha * acc[i][j][r];
-            const bool full = a.c_vec_ok && (n + 3 < a.n);
-            if (a.beta != 0.0f) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (n + r < a.n) v[r] += a.beta * load_as_f32<TO>(crow, n + r);
-            }
-            if (full) {
-                if constexpr (sizeof(oraw) == 2) {
-                    u32x2 p = {pack2<TO>(v[0], v[1]), pack2<TO>(v[2], v[3])};
-                    *reinterpret_cast<u32x2*>(crow + n) = p;
-                } else {
-                    *reinterpret_cast<f32x4*>(crow + n) = f32x4{v[0], v[1], v[2], v[3]};
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (n + r < a.n) store_from_f32<TO>(crow, n + r, v[r]);
-            }
-        }
-    }
-}
 
 // ---------------------------------------------------------------------------
 // DMA-staged variant (the fast path). Tiles go global -> LDS with
@@ -275,10 +69,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(GemmArgs a) {
 //   ds_read_b64_tr_b16: within each 16-lane group, lane j addresses the 4
 //   columns 4*(j%4).. of k-row j/4 and lane i receives column i of those 4
 //   k-rows -- exactly the MFMA B operand (two reads per 16x32 fragment).
-// Requirements (checked on the host): k % BK == 0, 16-byte aligned rows, and
-// for NN: n % 16 == 0. Rows past M / N are clamped (their outputs are never
-// stored); K has no tail.
+// Requirements (checked on the host): k % VEC == 0, 16-byte aligned rows, and
+// for NN: n % 8 == 0. Rows past M / N are clamped (their outputs are never
+// stored).
 // ---------------------------------------------------------------------------
+
+// What the DMA reads in place of k past the end.
+static __device__ const u32x4 dma_zero[1] = {{0u, 0u, 0u, 0u}};
 
 // SOFF: every operand spans less than 2^31 bytes (checked on the host): the DMA
 // then goes from a wave-uniform base, moved by scalar adds per k step, plus a
@@ -318,21 +115,27 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
     const int bz = blockIdx.y;
     const raw* __restrict__ Ap = static_cast<const raw*>(a.A) + bz * a.sa_b;
     const raw* __restrict__ Bp = static_cast<const raw*>(a.B) + bz * a.sb_b;
-    const int KT = a.k / BK;
+    // A ragged k makes the FIRST step short, [0, first): its missing chunks come
+    // from 16 bytes of zeros (dma_zero), and the loop has whole steps only.
+    const int KT = (a.k + BK - 1) / BK;
+    const int first = a.k - (KT - 1) * BK;
 
+    // Step 0 of a ragged k, and every step of operands too large for SOFF.
     auto issue_a = [&](int kt, u32x4* sA) {
-        const int k0 = kt * BK;
+        const int k0 = kt == 0 ? 0 : kt * BK - (BK - first);
 #pragma unroll
         for (int i = 0; i < A_PT; ++i) {
             const int slot = i * THREADS + wave * 64 + lane;
             const int r = slot >> 3;
             const int c = swz_dma(r, slot & 7);  // the swizzle is an involution on the chunk index
             const int row = min(m0 + r, a.m - 1);
-            dma16_async(Ap + (int64_t)row * a.rsa + k0 + c * VEC, &sA[i * THREADS + wave * 64]);
+            const raw* g = Ap + (int64_t)row * a.rsa + k0 + c * VEC;
+            if (kt == 0 && c * VEC >= first) g = reinterpret_cast<const raw*>(dma_zero);
+            dma16_async(g, &sA[i * THREADS + wave * 64]);
         }
     };
     auto issue_b = [&](int kt, u32x4* sB) {
-        const int k0 = kt * BK;
+        const int k0 = kt == 0 ? 0 : kt * BK - (BK - first);
 #pragma unroll
         for (int i = 0; i < B_PT; ++i) {
             const int slot = i * THREADS + wave * 64 + lane;
@@ -342,10 +145,12 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
                 const int c = swz_dma(r, slot & 7);
                 const int row = min(n0 + r, a.n - 1);
                 g = Bp + (int64_t)row * a.csb + k0 + c * VEC;
+                if (kt == 0 && c * VEC >= first) g = reinterpret_cast<const raw*>(dma_zero);
             } else {
                 const int r = slot / (2 * NBLK), ps = slot % (2 * NBLK);
                 const int lb = nn_blk(r, ps >> 1, BLK_MASK);
-                g = Bp + (int64_t)(k0 + r) * a.rsb + min(n0 + lb * 16, a.n - 16) + (ps & 1) * 8;
+                g = Bp + (int64_t)(k0 + r) * a.rsb + min(n0 + lb * 16 + (ps & 1) * 8, a.n - 8);
+                if (kt == 0 && r >= first) g = reinterpret_cast<const raw*>(dma_zero);
             }
             dma16_async(g, &sB[i * THREADS + wave * 64]);
         }
@@ -373,7 +178,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
             } else {
                 const int r = slot / (2 * NBLK), ps = slot % (2 * NBLK);
                 const int lb = nn_blk(r, ps >> 1, BLK_MASK);
-                e = (int64_t)r * a.rsb + min(n0 + lb * 16, a.n - 16) + (ps & 1) * 8;
+                e = (int64_t)r * a.rsb + min(n0 + lb * 16 + (ps & 1) * 8, a.n - 8);
             }
             offB[i] = (uint32_t)(e * (int64_t)sizeof(raw));
         }
@@ -382,10 +187,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
     }
     // DMA of k step kt into stage st
     auto issue_st = [&](int kt, int st) {
-        if constexpr (SOFF) {
-            const char* bA = reinterpret_cast<const char*>(Ap) + (int64_t)kt * BK * (int64_t)sizeof(raw);
-            const char* bB = reinterpret_cast<const char*>(Bp) +
-                             (int64_t)kt * BK * (NN ? a.rsb : (int64_t)1) * (int64_t)sizeof(raw);
+        if (SOFF && (kt > 0 || first == BK)) {
+            const int64_t k0 = (int64_t)kt * BK - (BK - first);
+            const char* bA = reinterpret_cast<const char*>(Ap) + k0 * (int64_t)sizeof(raw);
+            const char* bB = reinterpret_cast<const char*>(Bp) + k0 * (NN ? a.rsb : (int64_t)1) * (int64_t)sizeof(raw);
 #pragma unroll
             for (int i = 0; i < A_PT; ++i) dma16_soff(bA, offA[i], ldsA0 + (uint32_t)(st * STA + i * THREADS) * 16u);
 #pragma unroll
@@ -838,60 +643,6 @@ __global__ __launch_bounds__(512, 1) void gemm_pingpong_kernel(GemmArgs a) {
 //   row loads, 8 waves split K, LDS reduction.
 // ---------------------------------------------------------------------------
 constexpr int SKINNY_M = 16;
-constexpr int SKINNY_WAVES = 8;
-
-template <class T, class TO>
-__global__ __launch_bounds__(64 * SKINNY_WAVES) void gemm_skinny_nn_kernel(GemmArgs a) {
-    using raw = typename T::raw;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n = blockIdx.x * 64 + lane;
-    const int bz = blockIdx.y;
-    const raw* __restrict__ Ap = static_cast<const raw*>(a.A) + bz * a.sa_b;
-    const raw* __restrict__ Bp = static_cast<const raw*>(a.B) + bz * a.sb_b;
-    const int per_wave = (a.k + SKINNY_WAVES - 1) / SKINNY_WAVES;
-    const int k_begin = wave * per_wave, k_end = min(a.k, k_begin + per_wave);
-    float acc[SKINNY_M];
-#pragma unroll
-    for (int i = 0; i < SKINNY_M; ++i) acc[i] = 0.f;
-    const bool col = n < a.n;
-    const raw* bp = Bp + (col ? n : 0);
-    constexpr int UNR = 8;
-    int k = k_begin;
-    for (; k + UNR <= k_end; k += UNR) {
-        float b[UNR];
-#pragma unroll
-        for (int u = 0; u < UNR; ++u) b[u] = col ? load_as_f32<T>(bp, (int64_t)(k + u) * a.rsb) : 0.f;
-#pragma unroll
-        for (int i = 0; i < SKINNY_M; ++i) {
-            if (i < a.m) {
-#pragma unroll
-                for (int u = 0; u < UNR; ++u) acc[i] = fmaf(load_as_f32<T>(Ap, (int64_t)i * a.rsa + k + u), b[u], acc[i]);
-            }
-        }
-    }
-    for (; k < k_end; ++k) {
-        const float b = col ? load_as_f32<T>(bp, (int64_t)k * a.rsb) : 0.f;
-#pragma unroll
-        for (int i = 0; i < SKINNY_M; ++i)
-            if (i < a.m) acc[i] = fmaf(load_as_f32<T>(Ap, (int64_t)i * a.rsa + k), b, acc[i]);
-    }
-    __shared__ float red[SKINNY_WAVES][SKINNY_M][64];
-#pragma unroll
-    for (int i = 0; i < SKINNY_M; ++i) red[wave][i][lane] = acc[i];
-    __syncthreads();
-    if (wave != 0 || !col) return;
-    using oraw = typename TO::raw;
-    for (int i = 0; i < a.m; ++i) {
-        float t = 0.f;
-#pragma unroll
-        for (int w = 0; w < SKINNY_WAVES; ++w) t += red[w][i][lane];
-        oraw* crow = static_cast<oraw*>(a.C) + bz * a.sc_b + (int64_t)i * a.rsc;
-        float v = a.alpha * t;
-        if (a.beta != 0.0f) v += a.beta * load_as_f32<TO>(crow, n);
-        store_from_f32<TO>(crow, n, v);
-    }
-}
-
 // M == 1 with row-major B [K][N] (the configs' weight layout): a workgroup owns
 // CPR * VEC consecutive columns (CPR 16-byte chunks of a k-row); its 16 waves
 // split K, and within a wave lane (r, c) = (lane / CPR, lane % CPR) reads chunk c
@@ -984,7 +735,7 @@ __global__ __launch_bounds__(1024) void gemv_nn_kernel(GemmArgs a) {
 //     c ^ (((r >> 2) & 3) << 2); MFMA step j of lane group g reads k-row
 //     16 kb + 4 g + j, one ds_read_b32 of n = 16 fn + l % 16: the four groups'
 //     rows land in four bank ranges.
-// Rows of A / B past m / n re-read the last row (never stored); k % 32 == 0.
+// Rows of A / B past m / n re-read the last row (never stored); k % 4 == 0.
 template <int BM, int BN, int WM, int WN, bool NN, int STAGES>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(GemmArgs a) {
     constexpr int THREADS = 64 * WM * WN;
@@ -1038,16 +789,25 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(GemmArgs a) {
             boff[i] = (c ^ (row & 7)) * 4;
         }
     }
+    // A ragged k makes the first step short, as in gemm_mfma_dma_kernel.
+    const int nks = (a.k + BK - 1) / BK;
+    const int first = a.k - (nks - 1) * BK;
     auto issue = [&](int ks) {
-        const int k0 = ks * BK;
+        const int k0 = ks == 0 ? 0 : ks * BK - (BK - first);
         u32x4* dA = sA + (ks % STAGES) * STA;
         u32x4* dB = sB + (ks % STAGES) * STB;
 #pragma unroll
-        for (int i = 0; i < A_PT; ++i) dma16_async(Ap + arow[i] + k0 + aoff[i] * 4, &dA[i * THREADS + wave * 64]);
+        for (int i = 0; i < A_PT; ++i) {
+            const float* p = Ap + arow[i] + k0 + aoff[i] * 4;
+            if (ks == 0 && aoff[i] * 4 >= first) p = reinterpret_cast<const float*>(dma_zero);
+            dma16_async(p, &dA[i * THREADS + wave * 64]);
+        }
 #pragma unroll
         for (int i = 0; i < B_PT; ++i) {
-            if constexpr (NN) dma16_async(Bp + bbase[i] + (int64_t)k0 * a.rsb, &dB[i * THREADS + wave * 64]);
-            else dma16_async(Bp + bbase[i] + k0 + boff[i], &dB[i * THREADS + wave * 64]);
+            const float* p = Bp + bbase[i] + (NN ? (int64_t)k0 * a.rsb : (int64_t)k0 + boff[i]);
+            const int bk = NN ? (i * THREADS + tid) / (BN / 4) : boff[i];  // the chunk's (first) k in the step
+            if (ks == 0 && bk >= first) p = reinterpret_cast<const float*>(dma_zero);
+            dma16_async(p, &dB[i * THREADS + wave * 64]);
         }
     };
 
@@ -1057,7 +817,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(GemmArgs a) {
 #pragma unroll
         for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int nks = a.k / BK;
     constexpr int AHEAD = STAGES - 1;  // steps issued before the first one is computed
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i)
@@ -1138,32 +897,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(GemmArgs a) {
     }
 }
 
-// Any-stride fallback: one output per thread, fp32 accumulation in k order.
-struct GenericArgs {
-    const void* A;
-    const void* B;
-    void* C;
-    int m, n, k;
-    int64_t rsa, csa, rsb, csb, rsc, csc, sa_b, sb_b, sc_b;
-    float alpha, beta;
-};
-
-template <class T, class TO>
-__global__ __launch_bounds__(256) void gemm_generic_kernel(GenericArgs a) {
-    const int j = blockIdx.x * 16 + (threadIdx.x & 15);
-    const int i = blockIdx.y * 16 + (threadIdx.x >> 4);
-    const int b = blockIdx.z;
-    if (i >= a.m || j >= a.n) return;
-    const int64_t ao = b * a.sa_b + i * a.rsa, bo = b * a.sb_b + j * a.csb;
-    float acc = 0.0f;
-    for (int p = 0; p < a.k; ++p)
-        acc = fmaf(load_as_f32<T>(a.A, ao + p * a.csa), load_as_f32<T>(a.B, bo + p * a.rsb), acc);
-    const int64_t co = b * a.sc_b + i * a.rsc + j * a.csc;
-    float v = a.alpha * acc;
-    if (a.beta != 0.0f) v += a.beta * load_as_f32<TO>(a.C, co);
-    store_from_f32<TO>(a.C, co, v);
-}
-
 // C = beta * C (k == 0 or alpha == 0), sgemm.inl:594-604.
 template <class TO>
 __global__ __launch_bounds__(256) void gemm_scale_kernel(void* C, int m, int n, int64_t rsc, int64_t csc,
@@ -1180,20 +913,6 @@ __global__ __launch_bounds__(256) void gemm_scale_kernel(void* C, int m, int n, 
 // Host side
 // ---------------------------------------------------------------------------
 namespace {
-
-template <class T, class TO, int BM, int BN, int WM, int WN>
-hipError_t launch_tile(const GemmArgs& a0, bool nn, int batch, hipStream_t s) {
-    GemmArgs a = a0;
-    a.tiles_m = (a.m + BM - 1) / BM;
-    a.tiles_n = (a.n + BN - 1) / BN;
-    dim3 grid(a.tiles_m * a.tiles_n, batch);
-    dim3 block(64 * WM * WN);
-    if (nn)
-        gemm_mfma_kernel<T, TO, BM, BN, WM, WN, true><<<grid, block, 0, s>>>(a);
-    else
-        gemm_mfma_kernel<T, TO, BM, BN, WM, WN, false><<<grid, block, 0, s>>>(a);
-    return hipGetLastError();
-}
 
 template <class T, class TO, int BM, int BN, int WM, int WN, int STAGES>
 hipError_t launch_dma_tile(const GemmArgs& a0, bool nn, int batch, hipStream_t s) {
@@ -1237,7 +956,7 @@ hipError_t launch_dma(const GemmArgs& a, bool nn, int batch, hipStream_t s) {
             // NT with a partial last column of tiles: the whole tiles on the
             // ping-pong kernel, the last N % 256 columns as a product of their own
             // (disjoint columns of C; B rows and C columns offset).
-            if (!nn && a.m % 256 == 0 && a.n % 256 != 0 && a.n > 256 && span_a < (int64_t(1) << 31) &&
+            if (!nn && a.m % 256 == 0 && a.k % 64 == 0 && a.n % 256 != 0 && a.n > 256 && span_a < (int64_t(1) << 31) &&
                 span_b < (int64_t(1) << 31)) {
                 using oraw = typename TO::raw;
                 GemmArgs g = a;
@@ -1253,7 +972,7 @@ hipError_t launch_dma(const GemmArgs& a, bool nn, int batch, hipStream_t s) {
                 r.C = static_cast<oraw*>(a.C) + g.n;
                 return launch_dma<T, TO>(r, nn, batch, s);
             }
-            if (a.m % 256 == 0 && (nn ? a.n % 16 == 0 : a.n % 256 == 0) && span_a < (int64_t(1) << 31) &&
+            if (a.m % 256 == 0 && a.k % 64 == 0 && (nn ? a.n % 16 == 0 : a.n % 256 == 0) && span_a < (int64_t(1) << 31) &&
                 span_b < (int64_t(1) << 31)) {
                 GemmArgs g = a;
                 g.tiles_m = a.m / 256;
@@ -1273,23 +992,6 @@ hipError_t launch_dma(const GemmArgs& a, bool nn, int batch, hipStream_t s) {
     // projections with weights coming from HBM).
     if (tiles(64, 64) < 256) return launch_dma_tile<T, TO, 64, 32, 2, 1, 4>(a, nn, batch, s);
     return launch_dma_tile<T, TO, 64, 64, 2, 2, 4>(a, nn, batch, s);
-}
-
-template <class T, class TO>
-hipError_t launch_mfma(const GemmArgs& a, bool nn, int batch, hipStream_t s) {
-    auto tiles = [&](int bm, int bn) {
-        return (int64_t)((a.m + bm - 1) / bm) * ((a.n + bn - 1) / bn) * batch;
-    };
-    if (tiles(256, 256) >= 160) return launch_tile<T, TO, 256, 256, 2, 4>(a, nn, batch, s);
-    if (tiles(128, 128) >= 96) return launch_tile<T, TO, 128, 128, 2, 2>(a, nn, batch, s);
-    return launch_tile<T, TO, 64, 64, 2, 2>(a, nn, batch, s);
-}
-
-template <class T, class TO>
-hipError_t launch_generic(const GenericArgs& a, int batch, hipStream_t s) {
-    dim3 grid((a.n + 15) / 16, (a.m + 15) / 16, batch);
-    gemm_generic_kernel<T, TO><<<grid, 256, 0, s>>>(a);
-    return hipGetLastError();
 }
 
 template <class TO>
@@ -1349,17 +1051,15 @@ int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int6
             // 64-row tile per column tile) streams B at full width; the column-per-
             // lane kernel below re-reads A per k and issues 2-byte loads of B
             // ((16, 3072, 1024): ~100 us there)
-            if (es == 2 && (k % (8 * VEC)) == 0 && (rsb % VEC) == 0 && (sb_b % VEC) == 0 && (n % 16) == 0 &&
-                aligned(B, 16))
+            if (es == 2 && (rsb % VEC) == 0 && (sb_b % VEC) == 0 && (n % VEC) == 0 && aligned(B, 16))
                 return status_of(launch_dma<T, TO>(g, true, batch, s));
-            gemm_skinny_nn_kernel<T, TO><<<dim3((n + 63) / 64, batch), 64 * SKINNY_WAVES, 0, s>>>(g);
-            return status_of(hipGetLastError());
         }
         if constexpr (std::is_same_v<T, F32> && std::is_same_v<TO, F32>) {
-            // fp32 on the DMA-staged fp32 MFMA kernel: k a multiple of its 32-wide
-            // step, 16-byte aligned rows of A and of B (NT) or B's k-rows (NN)
+            // fp32 on the DMA-staged fp32 MFMA kernel: 16-byte aligned rows of A and
+            // of B (NT) or B's k-rows (NN). 1000^3: 37.8 us on the register-staged
+            // kernel that took k % 32 != 0 before, 24.6 us here
             const bool f_nn = nn && (rsb % 4) == 0 && (sb_b % 4) == 0 && aligned(B, 16) && n >= 4;
-            if (k % 32 == 0 && (nt || f_nn)) {
+            if (nt || f_nn) {
                 auto ntiles = [&](int bm, int bn) { return (int64_t)((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batch; };
                 const bool big = ntiles(128, 128) >= 512;
                 GemmArgs f = g;
@@ -1378,16 +1078,15 @@ int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int6
                 return status_of(hipGetLastError());
             }
         }
-        // DMA-staged fast path: whole k steps, 16-byte aligned rows everywhere.
-        const bool dma_k = (k % (8 * VEC)) == 0;
-        const bool dma_nt = nt;
-        const bool dma_nn = nn && es == 2 && (rsb % VEC) == 0 && (sb_b % VEC) == 0 && (n % 16) == 0 &&
+        // DMA-staged fast path: 16-byte aligned rows everywhere, k in whole chunks
+        // (k % 64 != 0, 4096 x 4096 x 4072 NN: 228 -> 119 us, 1000^3 17.3 -> 7.8 us
+        // against the register-staged kernel that took those before).
+        const bool dma_nn = nn && es == 2 && (rsb % VEC) == 0 && (sb_b % VEC) == 0 && (n % VEC) == 0 &&
                             aligned(B, 16);
-        if (dma_k && (dma_nt || dma_nn)) return status_of(launch_dma<T, TO>(g, nn, batch, s));
-        return status_of(launch_mfma<T, TO>(g, nn, batch, s));
+        if (nt || dma_nn) return status_of(launch_dma<T, TO>(g, nn, batch, s));
     }
-    GenericArgs g{A, B, C, m, n, k, rsa, csa, rsb, csb, rsc, csc, sa_b, sb_b, sc_b, alpha, beta};
-    return status_of(launch_generic<T, TO>(g, batch, s));
+    return gemm_any_dispatch(T::code, TO::code, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b, rsc, csc,
+                             alpha, beta, s);
 }
 
 }  // namespace

@@ -19,6 +19,11 @@ int gemm_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, c
                   int64_t rsa, int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C,
                   int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, hipStream_t s);
 
+// Any layout, size and alignment (gemm_any.hip); k > 0.
+int gemm_any_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, const void* A, int64_t sa_b,
+                      int64_t rsa, int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C,
+                      int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, hipStream_t s);
+
 // Skinny GEMM / fused decode GEMV (gemv.hip): C[m, n] = alpha * A' . W^T + beta * C
 // with A' built by the prologue (0: A as is, 1: RMSNorm of fp32 rows, 2: SwiGLU
 // of [gate | up] rows).
