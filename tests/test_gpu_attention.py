@@ -824,3 +824,91 @@ def test_prefill_fp32_bool_mask_words(orc, yt, pattern, grid, D):
     assert e <= 1e-4
     empty = ~m.any(axis=1)
     assert np.all(g[:, :, empty] == 0.0)
+
+
+def _sdpa64(q, k, v, scale, vis, bias):
+    """softmax(scale q k^T + bias over the visible keys) v in float64; q [H, Sq, D],
+    k / v [Hkv, Skv, .]; hidden keys never touch the sum, rows that see none are 0."""
+    G = q.shape[0] // k.shape[0]
+    k, v = k.repeat_interleave(G, 0).double(), v.repeat_interleave(G, 0).double()
+    s = torch.matmul(q.double(), k.transpose(-1, -2).contiguous()) * scale
+    if bias is not None:
+        s = s + bias.double()
+    p = torch.nan_to_num(torch.softmax(s.masked_fill(~vis, float("-inf")), -1), nan=0.0)
+    return torch.matmul(p, v)
+
+
+# d and dv below, at and past the 16-wide blocks and the 64 / 128 / 256 forms; key
+# counts below 4 and at the edges of the 16- and 32-key blocks
+ANY_CASES = [(1, 1, 1, 1), (3, 5, 2, 3), (16, 16, 17, 31), (40, 24, 33, 32), (64, 64, 5, 23), (64, 64, 40, 300), (64, 32, 18, 65),
+             (80, 80, 50, 130), (128, 128, 17, 100), (96, 130, 20, 33), (256, 256, 35, 70), (250, 7, 16, 64)]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("layout", ["plain", "k_t", "v_t", "kv_t", "odd"])
+@pytest.mark.parametrize("case", ANY_CASES, ids=lambda c: "-".join(map(str, c)))
+def test_prefill_any_layout(yt, case, layout, dtype):
+    """The any-layout kernel: K and / or V stored transposed, rows at an odd element
+    offset, head dims of every class, GQA 2:1, against float64, under each mask
+    kind in turn. Hidden keys hold infinities and NaN in V (a cache row not yet
+    written): none may reach a row that does not see them. Bound: 32-bit sums and
+    exponentials of scores up to 8 in size (1e-5 of the values' size), plus the
+    rounding of the result."""
+    D, Dv, Sq, Skv = case
+    td = TORCH_DT[dtype]
+    g = torch.Generator(device="cuda").manual_seed(D * 7 + Dv + Sq + Skv)
+    Hq, Hkv = 4, 2
+    mfma = layout == "plain" and D == Dv and D in (64, 128)  # the kernels of the aligned layouts
+    if mfma and dtype != "f32":
+        pytest.skip("16-bit weights there; tested with that tolerance above")
+
+    def operand(rows, cols, heads, t):
+        if t:
+            return torch.randn(1, heads, cols, rows, device="cuda", generator=g).to(td).transpose(-1, -2)
+        pad = 1 if layout == "odd" else 0
+        return torch.randn(1, heads, rows, cols + pad, device="cuda", generator=g).to(td)[..., pad:]
+
+    q = operand(Sq, D, Hq, False)
+    k = operand(Skv, D, Hkv, layout in ("k_t", "kv_t"))
+    v = operand(Skv, Dv, Hkv, layout in ("v_t", "kv_t"))
+    i, j = torch.arange(Sq, device="cuda")[:, None], torch.arange(Skv, device="cuda")[None, :]
+    bias = torch.randn(Sq, Skv, device="cuda", generator=g)
+    drop = torch.rand(Sq, Skv, device="cuda", generator=g) < 0.3
+    drop[0] = True  # a row that sees nothing
+    off = Skv // 3 - 1
+    for mask, vis, bs in [(None, torch.ones_like(drop), None), ("causal", j <= i + Skv - Sq, None),
+                          (("diag", off), j <= i + off, bias), (~drop, ~drop, None), (~drop, ~drop, bias)]:
+        vv = v.clone() if v.stride(-1) == 1 else v.transpose(-1, -2).clone().transpose(-1, -2)
+        hidden = ~vis.any(0)
+        if hidden.any() and not mfma:
+            vv[:, :, hidden] = torch.tensor([float("inf"), float("nan"), float("-inf")], device="cuda").to(td)[
+                torch.arange(int(hidden.sum()), device="cuda") % 3][:, None]
+        out = yt.scaled_dot_product_attention(q, k, vv, 0.0, mask=mask, bias=bs)
+        clean = torch.where(hidden[None, :, None], torch.zeros_like(vv[0]), vv[0])
+        want = _sdpa64(q[0], k[0], clean, 1.0 / math.sqrt(D), vis, bs)
+        ulp = {"f32": 0.0, "bf16": 2.0 ** -8, "f16": 2.0 ** -10}[dtype]
+        bound = 1e-5 * float(clean.double().abs().max()) + ulp * want.abs()
+        assert torch.isfinite(out).all() and ((out[0].double() - want).abs() <= bound).all(), (layout, mask if isinstance(mask, (str, tuple)) else "bytes")
+
+
+def test_prefill_any_layout_non_finite_values(yt):
+    """A visible infinity or NaN in V reaches exactly the rows that see it (the
+    transposed-cache layout, two key blocks)."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    Skv, D = 70, 64
+    q = torch.randn(1, 2, 20, D, device="cuda", generator=g)
+    k = torch.randn(1, 2, D, Skv, device="cuda", generator=g).transpose(-1, -2)
+    v = torch.randn(1, 2, D, Skv, device="cuda", generator=g).transpose(-1, -2)
+    v[:, :, 3, 5], v[:, :, 40, 6], v[:, :, 41, 6], v[:, :, 69, 7] = float("inf"), float("inf"), float("-inf"), float("nan")
+    mask = torch.zeros(20, Skv, dtype=torch.bool, device="cuda")
+    mask[:, 10] = True
+    mask[1, 3] = mask[2, 40] = mask[3, 40] = mask[3, 41] = mask[4, 69] = True
+    out = yt.scaled_dot_product_attention(q, k, v, mask=mask)[0]
+    want = torch.zeros(20, D, device="cuda")
+    want[1, 5] = want[2, 6] = float("inf")
+    want[3, 6] = want[4, 7] = float("nan")
+    finite = torch.isfinite(want)
+    for h in range(2):
+        assert torch.equal(torch.isfinite(out[h]), finite)
+        assert out[h, 1, 5] == float("inf") and out[h, 2, 6] == float("inf") and out[h, 3, 6].isnan() and out[h, 4, 7].isnan()
+        assert torch.equal(out[h, 0], v[0, h, 10])

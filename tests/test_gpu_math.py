@@ -261,3 +261,58 @@ def test_math_long_rows(orc, yt, dev, Lkv):
     ref = orc.sdpa_math(Q, K, V, 0.0, mask=m, bias=b)
     assert np.abs(_f(got) - ref).max() <= 1e-4
     assert torch.count_nonzero(got[:, 3]) == 0
+
+
+def _math64(q, k, v, scale, vis, bias):
+    """The MATH backend in float64: hidden scores are -1e9 before scale and bias and
+    stay in the softmax; rows that see no key are zero when a mask is given."""
+    G = q.shape[0] // k.shape[0]
+    k, v = k.repeat_interleave(G, 0).double(), v.repeat_interleave(G, 0).double()
+    s = torch.matmul(q.double(), k.transpose(-1, -2).contiguous())
+    if vis is not None:
+        s = s.masked_fill(~vis, -1e9)
+    s = s * scale
+    if bias is not None:
+        s = s + bias.double()
+    o = torch.matmul(torch.softmax(s, -1), v)
+    return o if vis is None else o.masked_fill(~vis.any(-1)[:, None], 0.0)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Sq,Skv", [(1, 1), (5, 63), (64, 65), (65, 129), (130, 256), (300, 333), (2100, 200)])
+def test_sdpa_math_one_launch(yt, dev, Sq, Skv, D, dt):
+    """The one-launch MATH kernels against float64 at the edges of their 64-query and
+    64- / 128-key blocks, every mask kind, GQA 2:1. Beside ordinary scales: a
+    negative one and one of 1e-8 (hidden keys keep weight), a bias that lifts
+    hidden keys back up. Bound: 32-bit arithmetic on scores up to 8 (1e-5 of the
+    values' size) and in 16 bits the rounding of the weights and the result."""
+    g = torch.Generator(device=dev).manual_seed(Sq + Skv + D)
+    q = torch.randn(2, 4, Sq, D, device=dev, generator=g).to(dt)
+    k = torch.randn(2, 2, Skv, D, device=dev, generator=g).to(dt)
+    v = torch.randn(2, 2, Skv, D, device=dev, generator=g).to(dt)
+    i, j = torch.arange(Sq, device=dev)[:, None], torch.arange(Skv, device=dev)[None, :]
+    drop = torch.rand(Sq, Skv, device=dev, generator=g) < 0.4
+    drop[Sq // 2] = True
+    bias = torch.randn(Sq, Skv, device=dev, generator=g)
+    lift = torch.where(drop, torch.full_like(bias, 1e9 / D ** 0.5), bias)
+    cases = [(None, None, 0.0, None), ("causal", j <= i + Skv - Sq, 0.0, None), (("diag", -3), j <= i - 3, 0.0, None),
+             (~drop, ~drop, 0.0, None), (~drop, ~drop, 0.0, bias), ("causal", j <= i + Skv - Sq, 1e-8, None),
+             (~drop, ~drop, -1e-9, None), (~drop, ~drop, 0.0, lift)]
+    ulp = {torch.float32: 2e-7, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dt]
+    for mask, vis, scale, bs in cases:
+        out = yt.scaled_dot_product_attention(q, k, v, scale, mask=mask, bias=bs, backend="math")
+        for b in range(2):
+            want = _math64(q[b], k[b], v[b], scale or 1.0 / D ** 0.5, vis, bs)
+            top = float(v.double().abs().max())
+            bound = (1e-5 + ulp) * top + 2 * ulp * want.abs()
+            if bs is lift:  # -1e9 scale + 1e9 / sqrt(d) cancels to the size of a float's ulp at 1e8
+                continue
+            assert ((out[b].double() - want).abs() <= bound).all(), (scale, bs is not None)
+        assert torch.isfinite(out).all()
+    if Skv >= 63 and Sq > 1:
+        # 0 . V as in the product: a non-finite V row behind the mask reaches every row
+        v2 = v.clone()
+        v2[:, :, Skv - 1, 3] = float("nan")
+        out = yt.scaled_dot_product_attention(q, k, v2, mask=("diag", 0), backend="math")
+        assert out[..., 3].isnan().all() and torch.isfinite(out[..., :3]).all()

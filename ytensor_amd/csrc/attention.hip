@@ -34,35 +34,69 @@
 #include <mutex>
 #include <cfloat>
 
-#include "common.hpp"
+#include "attention_args.hpp"
 #include "launch.hpp"
 
 namespace ythip {
 
-constexpr float LOG2E = 1.4426950408889634f;
+// What the DMA reads in place of V rows past the last key.
+static __device__ const u32x4 dma_zero[1] = {{0u, 0u, 0u, 0u}};
 
-struct AttnArgs {
-    const void* Q;
-    const void* K;
-    const void* V;
-    void* O;
-    int64_t qs0, qs1, qs2, ks0, ks1, ks2, vs0, vs1, vs2, os0, os1, os2;
-    int64_t qs3, ks3, vs3, os3;  // element strides along d (1 on the MFMA path)
-    int B, Hq, Hkv, Sq, Skv, D, Dv;
-    int diag_off;  // causal / diagonal masks: key j visible to query i iff j <= i + diag_off
-    float scale_log2;  // scale * log2(e)
-    const uint8_t* mask;
-    int64_t mask_ld;
-    int causal;
-    const float* bias;
-    int64_t brs, bcs;
-    int nqb;
-    int balance;  // causal: the grid is resident at once, two workgroups per CU (see attn_fwd_mfma)
-    uint8_t* tcls;        // byte mask's tile classes (mask_tile_class_kernel), or null
-    int nkbt;             // 64-key blocks of the mask rows: ceil(Skv / 64)
-    int o_line;           // O: unit d stride, 16-byte aligned base, rows and heads
-    int mask_words;       // byte mask, no bias, 4-byte aligned base and rows (attn_fwd_f32)
-};
+
+// MODE 4, the MATH backend (src/function/ops.inl:388-418): masked_matmul leaves
+// -1e9 where the mask hides a key, then scale, then bias, then softmax over every
+// key. A hidden key's score is that finite value, not -inf: with large negative
+// scores, a bias or a negative scale it can carry weight. V rows behind the mask
+// still meet their weight of 0, so a non-finite one reaches the output as in the
+// product 0 . V.
+//
+// The four scores of keys key..key+3 for query q (q < Sq; key clamped by the
+// caller), in log2 units: x[i] = Q.K[key + i] on entry, -inf past the last key.
+// seen: some key of them is visible.
+__device__ __forceinline__ void math_scores4(const AttnArgs& a, f32x4& x, int q, int qa, int key, bool& seen) {
+    const float hidden = -1e9f * a.scale;
+    const bool whole = key + 3 < a.Skv;
+    uint32_t w = 0x01010101u;
+    if (a.mask != nullptr) {
+        const uint8_t* p = a.mask + (int64_t)q * a.mask_ld + key;
+        if (whole) {
+            w = *reinterpret_cast<const u32_any*>(p);
+        } else {
+            w = 0;
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                if (key + i < a.Skv) w |= (uint32_t)p[i] << (8 * i);
+        }
+    }
+    f32x4 bv = {0.f, 0.f, 0.f, 0.f};
+    if (a.bias != nullptr) {
+        const float* p = a.bias + (int64_t)q * a.brs + (int64_t)key * a.bcs;
+        if (whole && a.bcs == 1) {
+            bv = *reinterpret_cast<const f32x4_any*>(p);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (key + i < a.Skv) bv[i] = p[(int64_t)i * a.bcs];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const bool in = key + i < a.Skv;
+        bool vis = in && ((w >> (8 * i)) & 0xffu) != 0u;
+        if (a.causal) vis = vis && key + i <= qa + a.diag_off;
+        seen = seen || vis;
+        float v = vis ? x[i] * a.scale : hidden;
+        if (a.bias != nullptr) v += bv[i];
+        x[i] = in ? v * LOG2E : -INFINITY;
+    }
+}
+// The same for a diagonal mask alone and keys that are all there: as cheap as the
+// flash kernels' masking (S = 1024 causal: 28.5 us through the general form).
+__device__ __forceinline__ void math_scores4_diag(const AttnArgs& a, f32x4& x, int qa, int key) {
+    const float hidden = -1e9f * a.scale * LOG2E;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = key + i <= qa + a.diag_off ? x[i] * a.scale_log2 : hidden;
+}
 
 // MODE 0: no mask; 1: causal; 2: byte mask and/or bias read per element;
 // 3: byte mask staged per key block: the block's [BQ x BKV] mask tile is DMA'd
@@ -182,7 +216,7 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
             u32x4 v = {0u, 0u, 0u, 0u};
             if (q < a.Sq) v = *reinterpret_cast<const u32x4*>(Qp + (int64_t)q * a.qs2 + ks * 32 + g * 8);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
+            for (int e = 0; e < 4 && MODE != 4; ++e) {
                 const uint32_t w2 = v[e];
                 v[e] = pack2<T>(lo_as_f32(T{}, w2) * c, hi_as_f32(T{}, w2) * c);
             }
@@ -279,17 +313,24 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
                 dma16_soff(vbase, vbo[i], lv + (uint32_t)(i * THREADS) * 16u);
             }
         } else {
-            // a tail stage's rows past the end re-read the last key (never used)
+            // a tail stage's K rows past the end re-read the last key (never used),
+            // its V rows read zeros
 #pragma unroll
             for (int i = 0; i < PT; ++i) {
                 const int row = slot_row(i);
                 const int sh = k0 + SBKV <= a.Skv ? 0 : min(k0 + row, a.Skv - 1) - k0 - row;
                 dma16_async(kbase + koff(i) + sh * (int)a.ks2, &dK[i * THREADS + wave * 64]);
-                dma16_async(vbase + voff(i) + sh * (int)a.vs2, &dV[i * THREADS + wave * 64]);
+                const raw* vp = vbase + voff(i) + sh * (int)a.vs2;
+                if (k0 + row >= a.Skv) vp = reinterpret_cast<const raw*>(dma_zero);
+                dma16_async(vp, &dV[i * THREADS + wave * 64]);
             }
         }
     };
 
+    bool seen[QT];  // MODE 4 under a mask: some key is visible to the row (this lane's keys)
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt)
+        seen[qt] = !a.any_mask || (a.causal && q0 + qt * 16 + l16 + off >= 0);
     f32x4 s[QT][NKT];
     // S^T - m = K . Q^T - m for block kb (K stage kb & 1).
     auto qk = [&](int kb) {
@@ -297,7 +338,10 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
-            for (int kt = 0; kt < NKT; ++kt) s[qt][kt] = f32x4{-m[qt], -m[qt], -m[qt], -m[qt]};
+            for (int kt = 0; kt < NKT; ++kt) {
+                const float z = MODE == 4 ? 0.f : -m[qt];
+                s[qt][kt] = f32x4{z, z, z, z};
+            }
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
@@ -339,19 +383,49 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
             tile_all = __ballot(!all) == 0;
         }
     };
+    // MODE 4: block kb is hidden from every row of the wave by the diagonal, and
+    // its weights 2^(hidden - m) are all 0: only 0 . V is left of it.
+    auto all_zero = [&](int kb) {
+        if constexpr (MODE != 4) return false;
+        if (!a.causal || a.bias != nullptr || kb * SBKV + grp * BKV <= q0 + WQ - 1 + off) return false;
+        bool zero = true;
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) zero = zero && mset[qt] && -1e9f * a.scale * LOG2E - m[qt] < -200.f;
+        return __ballot(!zero) == 0;
+    };
     // Online softmax of block kb and O += V^T P^T (V stage kb & 1).
-    auto softmax_pv = [&](int kb) {
+    auto softmax_pv = [&](int kb, bool zero = false) {
         const int k0 = kb * SBKV + grp * BKV;
         const bool staged = MODE == 3 && k0 + BKV <= a.Skv;
-        const bool need_mask = (MODE == 2) || (MODE == 3 && !tile_all) || (k0 + BKV > a.Skv) ||
+        const bool need_mask = (MODE == 2) || (MODE == 4 && (a.mask != nullptr || a.bias != nullptr ||
+                                                             (a.causal && k0 + BKV - 1 > q0 + off))) || (MODE == 3 && !tile_all) || (k0 + BKV > a.Skv) ||
                                (MODE == 1 && k0 + BKV - 1 > q0 + off);
         u32x4 pk[QT][NKT / 2];
+        if (MODE == 4 && zero) {
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                for (int kk = 0; kk < NKT / 2; ++kk) pk[qt][kk] = u32x4{0u, 0u, 0u, 0u};
+        } else {
         float lmax[QT];
         bool trig = false;
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
             const int qa = q0 + qt * 16 + l16;
-            if (need_mask) {
+            if constexpr (MODE == 4) {
+                if (!need_mask) {
+#pragma unroll
+                    for (int kt = 0; kt < NKT; ++kt) s[qt][kt] *= c;
+                } else {
+                    const bool diag = a.mask == nullptr && a.bias == nullptr && k0 + BKV <= a.Skv;
+#pragma unroll
+                    for (int kt = 0; kt < NKT; ++kt) {
+                        const int key = k0 + kt * 16 + g * 4;
+                        if (diag) math_scores4_diag(a, s[qt][kt], qa, key);
+                        else math_scores4(a, s[qt][kt], min(qa, a.Sq - 1), qa, key, seen[qt]);
+                    }
+                }
+            } else if (need_mask) {
 #pragma unroll
                 for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
@@ -389,7 +463,8 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
             lmax[qt] = mx;
             // the reference point of a row moves (set on its first visible block,
             // afterwards only for a block max far above it) iff one of its lanes sees this
-            trig = trig || mx > thr[qt];
+            if constexpr (MODE == 4) trig = trig || mx - m[qt] > thr[qt];
+            else trig = trig || mx > thr[qt];
         }
         auto exps = [&]() {
 #pragma unroll
@@ -399,8 +474,11 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
                     float e[8];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        e[r] = __builtin_amdgcn_exp2f(s[qt][2 * kk][r]);
-                        e[4 + r] = __builtin_amdgcn_exp2f(s[qt][2 * kk + 1][r]);
+                        // MODE 4 keeps the scores themselves: next to a hidden key's
+                        // -1e9, s - m would lose a visible score's digits
+                        const float z = MODE == 4 ? m[qt] : 0.f;
+                        e[r] = __builtin_amdgcn_exp2f(s[qt][2 * kk][r] - z);
+                        e[4 + r] = __builtin_amdgcn_exp2f(s[qt][2 * kk + 1][r] - z);
                     }
                     pk[qt][kk] = u32x4{pack2<T>(e[0], e[1]), pack2<T>(e[2], e[3]), pack2<T>(e[4], e[5]),
                                        pack2<T>(e[6], e[7])};
@@ -417,21 +495,25 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
                 float mx = lmax[qt];
                 mx = __builtin_elementwise_maximum(mx, __shfl_xor(mx, 16, 64));
                 mx = __builtin_elementwise_maximum(mx, __shfl_xor(mx, 32, 64));
+                const float top = mx;
+                if constexpr (MODE == 4) mx -= m[qt];
                 const bool move = mset[qt] ? (mx > LAZY) : (mx != -INFINITY);
                 const float delta = move ? mx : 0.f;
                 const float alpha = (move && mset[qt]) ? __builtin_amdgcn_exp2f(-delta) : 1.0f;
-                m[qt] += delta;
+                if constexpr (MODE == 4) m[qt] = move ? top : m[qt];
+                else m[qt] += delta;
                 mset[qt] = mset[qt] || move;
                 thr[qt] = mset[qt] ? LAZY : -INFINITY;
 #pragma unroll
                 for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) s[qt][kt][r] -= delta;
+                    for (int r = 0; r < 4 && MODE != 4; ++r) s[qt][kt][r] -= delta;
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt) o[qt][dt] *= alpha;
                 lsum[qt] *= alpha;
             }
             exps();
+        }
         }
         const u32x4* cV = sV + (kb & 1) * STG + grp * BKV * KCH;
 #pragma unroll
@@ -534,7 +616,9 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
             if (kb + 1 < nkb) issue(kb + 1);
             if (active(kb)) {
                 mask_tile(kb);
-                if (tile_any) {
+                if (MODE == 4 && all_zero(kb)) {
+                    softmax_pv(kb, true);
+                } else if (tile_any) {
                     qk(kb);
                     softmax_pv(kb);
                 }
@@ -544,6 +628,21 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
         }
     }
 
+    // 1 / l; MODE 4: only a row that sees no key is zero (softmax over scores that
+    // are all -inf is NaN there)
+    auto inverse = [&](float L, bool row_seen) {
+        if constexpr (MODE == 4) return row_seen ? 1.0f / L : 0.f;
+        else return L > 0.f ? 1.0f / L : 0.f;
+    };
+    if constexpr (MODE == 4) {
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {  // over the row's four lanes
+            int v = seen[qt];
+            v |= __shfl_xor(v, 16, 64);
+            v |= __shfl_xor(v, 32, 64);
+            seen[qt] = v != 0;
+        }
+    }
     if constexpr (KSPLIT == 2) {
         // Every wave is past the last barrier, so the stages are free: waves 4-7
         // leave O and l (one u32x4 slot per lane) and m (-inf where none of its
@@ -559,6 +658,7 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
                 for (int dt = 0; dt < DT; ++dt) dst[dt * 64] = __builtin_bit_cast(u32x4, o[qt][dt]);
                 dst[DT * 64] = __builtin_bit_cast(u32x4, lsum[qt]);
                 xm[(wl * QT + qt) * 64 + lane] = mset[qt] ? m[qt] : -INFINITY;
+                if constexpr (MODE == 4) xm[(4 * QT + wl * QT + qt) * 64 + lane] = seen[qt] ? 1.f : 0.f;
             }
         }
         __syncthreads();
@@ -567,6 +667,7 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
         for (int qt = 0; qt < QT; ++qt) {
             const u32x4* src = xo + ((wl * QT + qt) * (DT + 1)) * 64 + lane;
             const float m1 = xm[(wl * QT + qt) * 64 + lane];
+            if constexpr (MODE == 4) seen[qt] = seen[qt] || xm[(4 * QT + wl * QT + qt) * 64 + lane] != 0.f;
             float a0 = 1.f, a1 = 0.f;
             if (!mset[qt]) {
                 a0 = 0.f;
@@ -597,7 +698,7 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) {
                 const float L = lsum[qt][0];
-                const float inv = L > 0.f ? 1.0f / L : 0.f;
+                const float inv = inverse(L, seen[qt]);
                 const int r = qt * 16 + l16;
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt) {
@@ -623,7 +724,7 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
         const float L = lsum[qt][0];
-        const float inv = L > 0.f ? 1.0f / L : 0.f;
+        const float inv = inverse(L, seen[qt]);
         const int q = q0 + qt * 16 + l16;
         if (q >= a.Sq) continue;
         raw* orow = Op + (int64_t)q * a.os2;
@@ -1199,61 +1300,9 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pingpong(AttnArgs a) {
     }
 }
 
-// Any layout / any dtype / d, dv <= 256: one wave per (batch, head, query row).
-// Scores for the whole row are kept in LDS (kv_len <= ROW_MAX), then max,
-// exp, sum and P.V in key order (the decode formulation of the reference).
-constexpr int ROW_MAX = 16384;
-
-template <class T>
-__global__ __launch_bounds__(64) void attn_rowwise(AttnArgs a) {
-    extern __shared__ float sc[];
-    const int qi = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-    const int kvh = h / (a.Hq / a.Hkv);
-    const int lane = threadIdx.x;
-    const int64_t qo = b * a.qs0 + h * a.qs1 + (int64_t)qi * a.qs2;
-    const int64_t ko = b * a.ks0 + kvh * a.ks1;
-    const int64_t vo = b * a.vs0 + kvh * a.vs1;
-    const float scale = a.scale_log2 / LOG2E;
-    const int off = a.diag_off;
-    float mx = -INFINITY;
-    for (int j = lane; j < a.Skv; j += 64) {
-        bool vis = true;
-        if (a.causal) vis = j <= qi + off;
-        if (vis && a.mask != nullptr) vis = a.mask[(int64_t)qi * a.mask_ld + j] != 0;
-        float x = -INFINITY;
-        if (vis) {
-            float acc = 0.f;
-            for (int d = 0; d < a.D; ++d)
-                acc = fmaf(load_as_f32<T>(a.Q, qo + d * a.qs3),
-                           load_as_f32<T>(a.K, ko + (int64_t)j * a.ks2 + d * a.ks3), acc);
-            x = acc * scale;
-            if (a.bias != nullptr) x += a.bias[(int64_t)qi * a.brs + (int64_t)j * a.bcs];
-        }
-        sc[j] = x;
-        mx = fmaxf(mx, x);
-    }
-#pragma unroll
-    for (int off2 = 32; off2 >= 1; off2 >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off2, 64));
-    float sum = 0.f;
-    for (int j = lane; j < a.Skv; j += 64) {
-        const float p = (sc[j] == -INFINITY) ? 0.f : expf(sc[j] - mx);
-        sc[j] = p;
-        sum += p;
-    }
-#pragma unroll
-    for (int off2 = 32; off2 >= 1; off2 >>= 1) sum += __shfl_xor(sum, off2, 64);
-    __syncthreads();
-    const float inv = sum > 0.f ? 1.0f / sum : 0.f;
-    const int64_t oo = b * a.os0 + h * a.os1 + (int64_t)qi * a.os2;
-    for (int d = lane; d < a.Dv; d += 64) {
-        float acc = 0.f;
-        if (sum > 0.f)
-            for (int j = 0; j < a.Skv; ++j)
-                if (sc[j] != 0.f)
-                    acc = fmaf(sc[j] * inv, load_as_f32<T>(a.V, vo + (int64_t)j * a.vs2 + d * a.vs3), acc);
-        store_from_f32<T>(a.O, oo + d * a.os3, acc);
-    }
-}
+// Layouts the MFMA kernels do not take (attention_any.hip) are limited to this
+// many keys.
+constexpr int ANY_MAX = 16384;
 
 // ---------------------------------------------------------------------------
 // fp32 prefill on the matrix cores. The reference's flash backend is fp32-only
@@ -1333,7 +1382,8 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_f32(AttnArgs a) {
     {
         const float* qp = Qp + (int64_t)min(qrow, a.Sq - 1) * a.qs2 + 4 * g;
 #pragma unroll
-        for (int bb = 0; bb < NB; ++bb) qf[bb] = *reinterpret_cast<const f32x4*>(qp + 16 * bb) * a.scale_log2;
+        for (int bb = 0; bb < NB; ++bb) 
+            qf[bb] = *reinterpret_cast<const f32x4*>(qp + 16 * bb) * (MODE == 4 ? 1.0f : a.scale_log2);
     }
 
     // DMA slots (row and swizzled chunk) as element offsets from the block's first key
@@ -1377,15 +1427,18 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_f32(AttnArgs a) {
         }
 #pragma unroll
         for (int i = 0; i < PT; ++i) {
-            // rows past the end re-read the last key (masked, never used)
+            // K rows past the end re-read the last key (masked, never used), V rows zeros
             const int row = slot_row(i);
             const int sh = min(k0 + row, a.Skv - 1) - k0 - row;
             dma16_async(kbase + koff(i) + sh * (int)a.ks2, &dK[i * 64 * NW + wave * 64]);
-            dma16_async(vbase + voff(i) + sh * (int)a.vs2, &dV[i * 64 * NW + wave * 64]);
+            const float* vp = vbase + voff(i) + sh * (int)a.vs2;
+            if (k0 + row >= a.Skv) vp = reinterpret_cast<const float*>(dma_zero);
+            dma16_async(vp, &dV[i * 64 * NW + wave * 64]);
         }
     };
 
     float m = -INFINITY, lsum = 0.f;
+    bool seen = !a.any_mask || (a.causal && qrow + a.diag_off >= 0);  // MODE 4
     f32x4 o[NB];
 #pragma unroll
     for (int t = 0; t < NB; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1497,6 +1550,16 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_f32(AttnArgs a) {
                     s[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kt][j], qf[bb][j], s[kt], 0, 0, 0);
         }
         // visibility, the block's row maximum, probabilities
+        if constexpr (MODE == 4) {
+            const bool diag = a.mask == nullptr && a.bias == nullptr && k0 + BKV <= a.Skv;
+            const bool plain = diag && (!a.causal || k0 + BKV - 1 <= q0 + a.diag_off);
+#pragma unroll
+            for (int kt = 0; kt < NKT; ++kt) {
+                if (plain) s[kt] *= a.scale_log2;
+                else if (diag) math_scores4_diag(a, s[kt], qrow, k0 + kofs + kt * 16 + 4 * g);
+                else math_scores4(a, s[kt], min(qrow, a.Sq - 1), qrow, k0 + kofs + kt * 16 + 4 * g, seen);
+            }
+        }
         float mx = -INFINITY;
 #pragma unroll
         for (int kt = 0; kt < NKT; ++kt)
@@ -1553,7 +1616,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_f32(AttnArgs a) {
         // Group 1 leaves O, m and l of each lane; group 0 merges them.
         __syncthreads();
         float* xo = reinterpret_cast<float*>(sK);
-        const int slot = (wl * 64 + lane) * (4 * NB + 2);
+        const int slot = (wl * 64 + lane) * (4 * NB + (MODE == 4 ? 3 : 2));
         if (wave >= 4) {
 #pragma unroll
             for (int t = 0; t < NB; ++t)
@@ -1561,6 +1624,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_f32(AttnArgs a) {
                 for (int i = 0; i < 4; ++i) xo[slot + 4 * t + i] = o[t][i];
             xo[slot + 4 * NB] = m;
             xo[slot + 4 * NB + 1] = lsum;
+            if constexpr (MODE == 4) xo[slot + 4 * NB + 2] = seen ? 1.f : 0.f;
         }
         __syncthreads();
         if (wave >= 4) return;
@@ -1574,6 +1638,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_f32(AttnArgs a) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) o[t][i] = o[t][i] * a0 + xo[slot + 4 * t + i] * a1;
         lsum = lsum * a0 + l1 * a1;
+        if constexpr (MODE == 4) seen = seen || xo[slot + 4 * NB + 2] != 0.f;
     }
     if (!wave_rows || qrow >= a.Sq) return;
     // the query's denominator: the sum of its 4 lanes' partials
@@ -1586,12 +1651,19 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_f32(AttnArgs a) {
         const auto p32 = __builtin_amdgcn_permlane32_swap(w, w, false, false);
         lt = __uint_as_float(p32[0]) + __uint_as_float(p32[1]);
     }
-    const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+    bool live = lt > 0.f;
+    if constexpr (MODE == 4) {  // only a row that sees no key is zero
+        int v = seen;
+        v |= __shfl_xor(v, 16, 64);
+        v |= __shfl_xor(v, 32, 64);
+        live = v != 0;
+    }
+    const float inv = live ? 1.0f / lt : 0.f;
     float* orow = Op + (int64_t)qrow * a.os2;
 #pragma unroll
     for (int t = 0; t < NB; ++t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) orow[(16 * t + 4 * g + i) * a.os3] = lt > 0.f ? o[t][i] * inv : 0.f;
+        for (int i = 0; i < 4; ++i) orow[(16 * t + 4 * g + i) * a.os3] = live ? o[t][i] * inv : 0.f;
 }
 
 // ---------------------------------------------------------------------------
@@ -2197,6 +2269,29 @@ hipError_t launch_prefill_mfma(AttnArgs a, int mode, hipStream_t s) {
     return launch_prefill_gh<T, D, 1, 2>(a, mode, s);
 }
 
+// The MATH backend in one launch (MODE 4): the score matrix never leaves the
+// registers. With the scores in fp32 and the weights in 16 bits in memory,
+// S = 1024 (16 heads, causal, bf16) was 61 us in three launches, is 20 us; S = 2048
+// 234 -> 59 us; fp32 S = 1024 119 -> 87 us. The weights are rounded to 16 bits as
+// before; error against 64 bits 2.3e-3 -> 2.0e-3 (bf16).
+template <class T, int D>
+hipError_t launch_math_mfma(AttnArgs a, hipStream_t s) {
+    // the key split at every size: 32 queries per wave spill 68 VGPRs here
+    a.balance = 0;
+    a.nqb = (a.Sq + 63) / 64;
+    attn_fwd_mfma<T, D, 4, 1, 1, 4, 2><<<dim3(a.nqb * a.B * a.Hq), 512, 0, s>>>(a);
+    return hipGetLastError();
+}
+template <int D>
+hipError_t launch_math_f32(AttnArgs a, hipStream_t s) {
+    const int64_t nqb = (a.Sq + 127) / 128;
+    if (nqb * a.B * a.Hq < 2 * (int64_t)device_cus())
+        attn_fwd_f32<D, 4, 2><<<dim3((unsigned)((a.Sq + 63) / 64 * a.B * a.Hq)), 512, 0, s>>>(a);
+    else
+        attn_fwd_f32<D, 4><<<dim3((unsigned)(nqb * a.B * a.Hq)), 512, 0, s>>>(a);
+    return hipGetLastError();
+}
+
 template <int D>
 hipError_t launch_prefill_f32(AttnArgs a, int mode, hipStream_t s) {
     // a byte mask alone with 16-byte aligned rows and a workspace: its tile
@@ -2224,11 +2319,19 @@ hipError_t launch_prefill_f32(AttnArgs a, int mode, hipStream_t s) {
     return hipGetLastError();
 }
 
+// The layouts of the MFMA kernels: d == dv in {64, 128}, contiguous, and
+// 16-byte aligned rows of Q, K and V (K / V reach LDS by 16-byte DMA; 64 rows
+// within 2^31 elements). O: 8-byte aligned rows in 16 bits.
 template <class T>
-hipError_t launch_rowwise(const AttnArgs& a, hipStream_t s) {
-    dim3 grid(a.Sq, a.Hq, a.B);
-    attn_rowwise<T><<<grid, 64, sizeof(float) * a.Skv, s>>>(a);
-    return hipGetLastError();
+bool mfma_layout(const AttnArgs& a) {
+    constexpr int ev = 16 / sizeof(typename T::raw);
+    const bool rows = a.qs3 == 1 && a.ks3 == 1 && a.vs3 == 1 && a.os3 == 1 && (a.D == 64 || a.D == 128) && a.Dv == a.D &&
+                      al(a.Q, 16) && al(a.K, 16) && al(a.V, 16) && a.qs0 % ev == 0 && a.qs1 % ev == 0 &&
+                      a.qs2 % ev == 0 && a.ks0 % ev == 0 && a.ks1 % ev == 0 && a.ks2 % ev == 0 && a.vs0 % ev == 0 &&
+                      a.vs1 % ev == 0 && a.vs2 % ev == 0 && a.ks2 < (1 << 24) && a.vs2 < (1 << 24) && a.ks2 >= 0 &&
+                      a.vs2 >= 0;
+    if (ev == 8) return rows && al(a.O, 8) && a.os0 % 4 == 0 && a.os1 % 4 == 0 && a.os2 % 4 == 0;
+    return rows && (int64_t)a.B * a.Hq < (1 << 30);
 }
 
 template <class T>
@@ -2239,15 +2342,7 @@ int prefill_typed(AttnArgs a, hipStream_t s) {
     const bool stage_mask = a.mask != nullptr && a.bias == nullptr && !a.causal && al(a.mask, 16) &&
                             a.mask_ld % 16 == 0;
     const int mode = a.causal ? 1 : (simple_mask ? 0 : (stage_mask ? 3 : 2));
-    const bool unit_d = a.qs3 == 1 && a.ks3 == 1 && a.vs3 == 1 && a.os3 == 1;
-    const bool mfma_ok = es == 2 && unit_d && (a.D == 64 || a.D == 128) && a.Dv == a.D &&
-                         !(a.causal && !simple_mask) &&
-                         a.scale_log2 > 0.f &&
-                         al(a.Q, 16) && al(a.K, 16) && al(a.V, 16) && al(a.O, 8) &&
-                         a.qs0 % 8 == 0 && a.qs1 % 8 == 0 && a.qs2 % 8 == 0 && a.ks0 % 8 == 0 && a.ks1 % 8 == 0 &&
-                         a.ks2 % 8 == 0 && a.vs0 % 8 == 0 && a.vs1 % 8 == 0 && a.vs2 % 8 == 0 &&
-                         a.os0 % 4 == 0 && a.os1 % 4 == 0 && a.os2 % 4 == 0 &&
-                         a.ks2 < (1 << 24) && a.vs2 < (1 << 24) && a.ks2 >= 0 && a.vs2 >= 0;
+    const bool mfma_ok = es == 2 && mfma_layout<T>(a) && !(a.causal && !simple_mask) && a.scale_log2 > 0.f;
     if (mfma_ok) {
         if constexpr (es == 2) {
             if (a.D == 128) return status_of(launch_prefill_mfma<T, 128>(a, mode, s));
@@ -2255,24 +2350,25 @@ int prefill_typed(AttnArgs a, hipStream_t s) {
         }
     }
     if constexpr (es == 4) {
-        // fp32 on v_mfma_f32_16x16x4_f32: 16-byte aligned rows of Q, K and V
-        // (K / V reach LDS by 16-byte DMA), 64 K / V rows within 2^31 elements
-        const bool f32_ok = unit_d && (a.D == 64 || a.D == 128) && a.Dv == a.D && (int64_t)a.B * a.Hq < (1 << 30) &&
-                            al(a.Q, 16) && al(a.K, 16) && al(a.V, 16) && a.qs0 % 4 == 0 && a.qs1 % 4 == 0 &&
-                            a.qs2 % 4 == 0 && a.ks0 % 4 == 0 && a.ks1 % 4 == 0 && a.ks2 % 4 == 0 &&
-                            a.vs0 % 4 == 0 && a.vs1 % 4 == 0 && a.vs2 % 4 == 0 && a.ks2 >= 0 && a.vs2 >= 0 &&
-                            a.ks2 < (1 << 24) && a.vs2 < (1 << 24);
-        if (f32_ok) {
+        // fp32 on v_mfma_f32_16x16x4_f32 (its diagonal form takes no bias)
+        if (mfma_layout<T>(a) && !(a.causal && !simple_mask)) {
             const int fmode = a.causal ? 1 : (simple_mask ? 0 : 2);
             if (a.D == 128) return status_of(launch_prefill_f32<128>(a, fmode, s));
             return status_of(launch_prefill_f32<64>(a, fmode, s));
         }
     }
-    if (a.Skv > ROW_MAX)
-        return fail(YTHIP_EUNSUPPORTED,
-                    "ythip_attn_prefill: this layout/dtype uses the row-wise kernel, limited to kv_len <= %d",
-                    ROW_MAX);
-    return status_of(launch_rowwise<T>(a, s));
+    if (a.Skv > ANY_MAX)
+        return fail(YTHIP_EUNSUPPORTED, "ythip_attn_prefill: this layout is limited to kv_len <= %d", ANY_MAX);
+    return status_of(attn_any(T::code, a, s));
+}
+
+template <class T>
+int math_typed(const AttnArgs& a, hipStream_t s) {
+    if (!mfma_layout<T>(a)) return -1;
+    if constexpr (std::is_same_v<T, F32>)
+        return status_of(a.D == 128 ? launch_math_f32<128>(a, s) : launch_math_f32<64>(a, s));
+    else
+        return status_of(a.D == 128 ? launch_math_mfma<T, 128>(a, s) : launch_math_mfma<T, 64>(a, s));
 }
 
 int decode_splits(int B, int Hq, int max_ctx) {
@@ -2385,6 +2481,31 @@ int decode_route(int dtype, const AttnArgs& p, int mask_kind, const uint8_t* mas
 }
 
 }  // namespace
+
+int attn_math_fused(const AttnCall& c, hipStream_t s) {
+    AttnArgs a{};
+    a.Q = c.Q; a.K = c.K; a.V = c.V; a.O = c.O;
+    a.qs0 = c.q_str[0]; a.qs1 = c.q_str[1]; a.qs2 = c.q_str[2]; a.qs3 = c.q_str[3];
+    a.ks0 = c.k_str[0]; a.ks1 = c.k_str[1]; a.ks2 = c.k_str[2]; a.ks3 = c.k_str[3];
+    a.vs0 = c.v_str[0]; a.vs1 = c.v_str[1]; a.vs2 = c.v_str[2]; a.vs3 = c.v_str[3];
+    a.os0 = c.o_str[0]; a.os1 = c.o_str[1]; a.os2 = c.o_str[2]; a.os3 = c.o_str[3];
+    a.o_line = a.os3 == 1 && a.os0 % 8 == 0 && a.os1 % 8 == 0 && a.os2 % 8 == 0 && al(a.O, 16);
+    a.B = c.B; a.Hq = c.Hq; a.Hkv = c.Hkv; a.Sq = c.Sq; a.Skv = c.Skv; a.D = c.D; a.Dv = c.Dv;
+    a.scale = c.scale;
+    a.scale_log2 = c.scale * LOG2E;
+    a.causal = c.mask_kind == YTHIP_MASK_CAUSAL || c.mask_kind == YTHIP_MASK_DIAG;
+    const int64_t off = c.mask_kind == YTHIP_MASK_DIAG ? c.mask_ld : (int64_t)c.Skv - c.Sq;
+    a.diag_off = (int)std::max<int64_t>(-(int64_t)c.Sq - 1, std::min<int64_t>(off, c.Skv));
+    a.any_mask = c.mask_kind != YTHIP_MASK_NONE;
+    a.mask = c.mask_kind == YTHIP_MASK_BOOL ? c.mask : nullptr;
+    a.mask_ld = c.mask_ld;
+    a.bias = c.bias; a.brs = c.brs; a.bcs = c.bcs;
+    switch (c.dtype) {
+        case YTHIP_F32: return math_typed<F32>(a, s);
+        case YTHIP_F16: return math_typed<F16>(a, s);
+        default: return math_typed<BF16>(a, s);
+    }
+}
 
 }  // namespace ythip
 

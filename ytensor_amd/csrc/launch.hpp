@@ -24,6 +24,22 @@ int gemm_any_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int 
                       int64_t rsa, int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C,
                       int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, hipStream_t s);
 
+// The MATH attention backend in one launch (attention.hip); -1 when the layout is
+// not one of the MFMA kernels' (nothing was launched).
+struct AttnCall {
+    int dtype, B, Hq, Hkv, Sq, Skv, D, Dv;
+    const void *Q, *K, *V;
+    void* O;
+    const int64_t *q_str, *k_str, *v_str, *o_str;
+    float scale;
+    int mask_kind;
+    const uint8_t* mask;
+    int64_t mask_ld;
+    const float* bias;
+    int64_t brs, bcs;
+};
+int attn_math_fused(const AttnCall& c, hipStream_t s);
+
 // Skinny GEMM / fused decode GEMV (gemv.hip): C[m, n] = alpha * A' . W^T + beta * C
 // with A' built by the prologue (0: A as is, 1: RMSNorm of fp32 rows, 2: SwiGLU
 // of [gate | up] rows).

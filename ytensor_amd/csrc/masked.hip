@@ -16,14 +16,11 @@
 // doc/en/api/function/fused.mdx:200); any other predicate is evaluated into a
 // bool mask by the caller.
 //
-// MI355X design: both operations are a product on the matrix cores plus a
-// bandwidth-bound pass over the [m, n] result. The products run on the GEMM
-// kernels of gemm.hip (fp32 output into a caller workspace); the mask / blend
-// and the softmax rows are one workgroup per row, and the attention weights
-// are written in the input type so
-// that the second product runs on the 16-bit MFMA path as in the reference,
-// whose score tensor has the input type. Masked tiles are not skipped: the
-// products are computed whole and the mask applied on the way out.
+// MI355X design: a product on the matrix cores plus a bandwidth-bound pass over the
+// [m, n] result. The products run on the GEMM kernels (fp32 output into a caller
+// workspace). MATH attention in the layouts of the MFMA attention kernels is one
+// launch (attention.hip, MODE 4); the passes here (scores in fp32, a softmax
+// workgroup per row, weights in the input type, a second product) serve the rest.
 
 #include <cfloat>
 
@@ -311,6 +308,10 @@ __attribute__((visibility("default"))) int ythip_attn_math(
     const size_t need = ythip_attn_math_workspace_size(dtype, B, Hq, q_len, kv_len);
     if (!workspace || ws_bytes < need)
         return fail(YTHIP_EINVAL, "%s: workspace of %zu bytes needed (%zu given)", who, need, ws_bytes);
+    // one launch for the layouts of the MFMA attention kernels
+    const AttnCall call{dtype, B, Hq, Hkv, q_len, kv_len, d, dv, Q, K, V, O, q_str, k_str, v_str, o_str,
+                        scale, mask_kind, mask, mask_ld, bias, rs_bias, cs_bias};
+    if (const int st = attn_math_fused(call, s); st != -1) return st;
     const int G = Hq / Hkv;
     const size_t cells = (size_t)B * Hq * q_len * kv_len;
     float* S = static_cast<float*>(workspace);
