@@ -316,3 +316,36 @@ def test_sdpa_math_one_launch(yt, dev, Sq, Skv, D, dt):
         v2[:, :, Skv - 1, 3] = float("nan")
         out = yt.scaled_dot_product_attention(q, k, v2, mask=("diag", 0), backend="math")
         assert out[..., 3].isnan().all() and torch.isfinite(out[..., :3]).all()
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("layout", ["NN", "NT", "odd", "c_cols"])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (5, 7, 3), (64, 64, 64), (130, 200, 72), (200, 136, 40), (257, 129, 100), (2048, 2056, 40)])
+def test_gemm_masked_layouts(yt, dev, m, n, k, layout, dt):
+    """The masked store of every product kernel (16-byte aligned rows NN / NT, odd
+    rows, a column-major C; 64- and 128-wide tiles, ragged edges): diagonals that
+    hide whole tiles, cut them and hide nothing, and bytes; kept or filled; alpha /
+    beta. Against float64: (k + 2) 2^-24 sum|a||b| plus the rounding of the result;
+    hidden entries exactly."""
+    g = torch.Generator(device=dev).manual_seed(m + n + k)
+    pad = 1 if layout == "odd" else 0
+    A = torch.randn(2, m, k + pad, device=dev, generator=g).to(dt)[:, :, pad:]
+    B = torch.randn(2, n, k, device=dev, generator=g).to(dt).transpose(1, 2) if layout == "NT" else \
+        torch.randn(2, k, n + pad, device=dev, generator=g).to(dt)[:, :, pad:]
+    prod = torch.matmul(A.double(), B.double().contiguous())
+    mass = torch.matmul(A.double().abs(), B.double().abs().contiguous())
+    i, j = torch.arange(m, device=dev)[:, None], torch.arange(n, device=dev)[None, :]
+    bytes_ = torch.rand(m, n, device=dev, generator=g) < 0.5
+    ulp = {torch.float32: 2.0 ** -23, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -10}[dt]
+    for mask, vis in [("causal", j <= i + n - m), (("diag", -70), j <= i - 70), (("diag", n), j <= i + n), (bytes_, bytes_)]:
+        for alpha, beta, fill in [(1.0, 0.0, -3.0), (1.0, 0.0, None), (0.5, 2.0, 7.0), (0.5, 2.0, None)]:
+            C = torch.randn(2, n, m, device=dev, generator=g).to(dt).transpose(1, 2) if layout == "c_cols" else \
+                torch.randn(2, m, n + pad, device=dev, generator=g).to(dt)[:, :, pad:]
+            C0 = C.double()
+            yt.gemm_masked(A, B, C, mask, alpha, beta, fill)
+            want = alpha * prod + beta * C0
+            bound = (k + 2) * 2.0 ** -24 * mass + ulp * want.abs() + 4 * 2.0 ** -23 * C0.abs() + 1e-7
+            off = ((C.double() - want).abs() > bound) & vis
+            assert not off.any(), (mask if isinstance(mask, (str, tuple)) else "bytes", alpha, fill)
+            hid = (~vis).expand(2, m, n)
+            assert torch.equal(C.double()[hid], (C0 if fill is None else torch.full_like(C0, fill))[hid])

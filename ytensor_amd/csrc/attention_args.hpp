@@ -32,11 +32,6 @@ struct AttnArgs {
     int any_mask;         // MODE 4: a mask was given, so rows that see no key are zero
 };
 
-// loads at any element address
-typedef uint32_t u32_any __attribute__((aligned(1)));
-typedef f32x4 f32x4_any __attribute__((aligned(4)));
-typedef u32x2 u32x2_any __attribute__((aligned(2)));
-
 // Any layout, type, mask and bias, d and dv up to 256 (attention_any.hip).
 hipError_t attn_any(int dtype, const AttnArgs& a, hipStream_t s);
 

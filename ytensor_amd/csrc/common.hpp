@@ -102,6 +102,58 @@ __device__ __forceinline__ f32x4 mfma_chunk(F32, u32x4 a, u32x4 b, f32x4 c) {
     return c;
 }
 
+// Loads at any element address.
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+typedef u32x2 u32x2_any __attribute__((aligned(2)));
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+
+// The mask of a masked product (YTHIP_MASK_NONE: a plain one). A hidden entry of C
+// keeps its value, or takes `value` when `fill` is set.
+struct MaskDesc {
+    int kind;  // YTHIP_MASK_NONE / CAUSAL / BOOL / DIAG
+    const uint8_t* data;
+    int64_t ld;
+    int64_t off;  // CAUSAL and DIAG: column j visible to row i iff j <= i + off
+    int fill;
+    float value;
+};
+__device__ __forceinline__ bool visible(const MaskDesc& mk, int i, int j) {
+    if (mk.kind == YTHIP_MASK_BOOL) return mk.data[(int64_t)i * mk.ld + j] != 0;
+    if (mk.kind == YTHIP_MASK_CAUSAL || mk.kind == YTHIP_MASK_DIAG) return (int64_t)j <= (int64_t)i + mk.off;
+    return true;
+}
+// bit r: (i, j + r) is visible; columns at or past n are not
+__device__ __forceinline__ uint32_t visible4(const MaskDesc& mk, int i, int j, int n) {
+    uint32_t v = 0;
+    if (mk.kind == YTHIP_MASK_BOOL && j + 3 < n) {
+        const uint32_t w = *reinterpret_cast<const u32_any*>(mk.data + (int64_t)i * mk.ld + j);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v |= (uint32_t)(((w >> (8 * r)) & 0xffu) != 0) << r;
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v |= (uint32_t)(j + r < n && visible(mk, i, j + r)) << r;
+    }
+    return v;
+}
+// rows up to i1 see no column from j0 on
+__device__ __forceinline__ bool hidden_tile(const MaskDesc& mk, int i1, int j0) {
+    return (mk.kind == YTHIP_MASK_CAUSAL || mk.kind == YTHIP_MASK_DIAG) && (int64_t)j0 > (int64_t)i1 + mk.off;
+}
+// Four columns of a masked C row: c at (row, n), element stride cs; v = alpha A.B.
+template <class TO>
+__device__ __forceinline__ void masked_store4(const MaskDesc& mk, typename TO::raw* crow, int64_t cs, int m, int n, int cols,
+                                              f32x4 v, float beta) {
+    const uint32_t vis = visible4(mk, m, n, cols);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (n + r >= cols) continue;
+        const int64_t at = (n + r) * cs;
+        if ((vis >> r) & 1) store_from_f32<TO>(crow, at, beta != 0.0f ? v[r] + beta * load_as_f32<TO>(crow, at) : v[r]);
+        else if (mk.fill) store_from_f32<TO>(crow, at, mk.value);
+    }
+}
+
 // Tile order of the GEMM grids, XCD-aware: the hardware places workgroup w on
 // XCD w % 8, so (when the tile count is a multiple of 8) w is remapped to give
 // each XCD a contiguous range of tiles, taken 4 tile-rows at a time so that an

@@ -26,6 +26,8 @@
 //  * What the DMA cannot take (rows that are not 16-byte aligned, k or n that are
 //    no whole chunks, a transposed A, other strides) runs in gemm_any.hip.
 
+#include <algorithm>
+
 #include "common.hpp"
 #include "launch.hpp"
 
@@ -42,6 +44,7 @@ struct GemmArgs {
     int tiles_m, tiles_n;
     int c_vec_ok;   // C rows allow 4-element vector stores
     int c_line_ok;  // 16-bit C: 16-byte aligned base and rows (the ping-pong kernel's line stores)
+    MaskDesc mask;  // (never on the ping-pong and GEMV kernels)
 };
 
 // Swizzles of the DMA-staged kernel, chosen by measuring gfx950's LDS read rate
@@ -82,7 +85,8 @@ static __device__ const u32x4 dma_zero[1] = {{0u, 0u, 0u, 0u}};
 // per-lane 32-bit byte offset fixed for the whole k loop (dma16_soff), and the
 // LDS destination is the wave's base plus constants -- no VALU address work
 // between the MFMAs of consecutive k steps.
-template <class T, class TO, int BM, int BN, int WM, int WN, bool NN, int STAGES, bool SOFF>
+// MASKED: a masked product (the mask's code costs every other form its length).
+template <class T, class TO, int BM, int BN, int WM, int WN, bool NN, int STAGES, bool SOFF, bool MASKED>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a) {
     using raw = typename T::raw;
     constexpr int THREADS = 64 * WM * WN;
@@ -117,13 +121,15 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
     const raw* __restrict__ Bp = static_cast<const raw*>(a.B) + bz * a.sb_b;
     // A ragged k makes the FIRST step short, [0, first): its missing chunks come
     // from 16 bytes of zeros (dma_zero), and the loop has whole steps only.
-    const int KT = (a.k + BK - 1) / BK;
-    const int first = a.k - (KT - 1) * BK;
+    const int KT_all = (a.k + BK - 1) / BK;
+    const int first = a.k - (KT_all - 1) * BK;
+    // a tile that the mask hides whole: its sums are not used
+    const int KT = MASKED && hidden_tile(a.mask, min(m0 + BM, a.m) - 1, n0) ? 1 : KT_all;
 
     // Step 0 of a ragged k, and every step of operands too large for SOFF.
     auto issue_a = [&](int kt, u32x4* sA) {
         const int k0 = kt == 0 ? 0 : kt * BK - (BK - first);
-#pragma unroll
+#pragma unroll (SOFF ? 1 : A_PT)
         for (int i = 0; i < A_PT; ++i) {
             const int slot = i * THREADS + wave * 64 + lane;
             const int r = slot >> 3;
@@ -136,7 +142,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
     };
     auto issue_b = [&](int kt, u32x4* sB) {
         const int k0 = kt == 0 ? 0 : kt * BK - (BK - first);
-#pragma unroll
+#pragma unroll (SOFF ? 1 : B_PT)
         for (int i = 0; i < B_PT; ++i) {
             const int slot = i * THREADS + wave * 64 + lane;
             const raw* g;
@@ -296,8 +302,23 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
 
     using oraw = typename TO::raw;
     oraw* Cp = static_cast<oraw*>(a.C) + bz * a.sc_b;
+    float alpha = a.alpha;
+    const bool filled = MASKED && a.mask.fill && a.beta == 0.0f;
+    if (MASKED && filled) {  // every entry is written: the value where hidden, then the stores of a plain product
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const int m = min(m0 + wm * WTM + i * 16 + lrow, a.m - 1);
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                const uint32_t vis = visible4(a.mask, m, n0 + wn * WTN + j * 16 + lgrp * 4, a.n);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[i][j][r] = (vis >> r) & 1 ? alpha * acc[i][j][r] : a.mask.value;
+            }
+        }
+        alpha = 1.0f;
+    }
     if constexpr (sizeof(oraw) == 2 && BN >= 64) {
-        if (a.beta == 0.0f && a.c_line_ok && m0 + BM <= a.m && n0 + BN <= a.n) {
+        if (a.beta == 0.0f && (!MASKED || filled) && a.c_line_ok && m0 + BM <= a.m && n0 + BN <= a.n) {
             // A whole 16-bit tile leaves through LDS in rows of BN elements (chunk c of
             // row r at c ^ (r % CPR)): each thread stores 16-byte chunks of whole tile
             // rows, 128-byte lines and up, instead of the fragments' 8-byte pieces of
@@ -315,8 +336,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
                     const int r = wm * WTM + i * 16 + lrow;
                     const int cb = (wn * WTN + j * 16 + lgrp * 4) * 2;
                     *reinterpret_cast<u32x2*>(t + r * (2 * BN) + ((((cb >> 4) ^ (r & (CPR - 1))) << 4) | (cb & 15))) =
-                        u32x2{pack2<TO>(a.alpha * acc[i][j][0], a.alpha * acc[i][j][1]),
-                              pack2<TO>(a.alpha * acc[i][j][2], a.alpha * acc[i][j][3])};
+                        u32x2{pack2<TO>(alpha * acc[i][j][0], alpha * acc[i][j][1]),
+                              pack2<TO>(alpha * acc[i][j][2], alpha * acc[i][j][3])};
                 }
             __syncthreads();
 #pragma unroll
@@ -337,9 +358,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
             const int n = n0 + wn * WTN + j * 16 + lgrp * 4;
             if (n >= a.n) continue;
             oraw* crow = Cp + (int64_t)m * a.rsc;
+            if (MASKED && !filled) {
+                masked_store4<TO>(a.mask, crow, 1, m, n, a.n, acc[i][j] * alpha, a.beta);
+                continue;
+            }
             float v[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = a.alpha * acc[i][j][r];
+            for (int r = 0; r < 4; ++r) v[r] = alpha * acc[i][j][r];
             if (a.beta != 0.0f) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
@@ -638,9 +663,8 @@ __global__ __launch_bounds__(512, 1) void gemm_pingpong_kernel(GemmArgs a) {
 // Skinny GEMM, M <= 16 (the decode GEMVs: x [1..16, K] . W^T). HBM-bound on
 // the weight stream, so the design goal is bytes in flight, not MFMA reuse.
 //   NT (W^T, the `linear` layout): gemv_kernel in gemv.hip.
-//   NN (B [K][N] row-major): VALU; M == 1 in gemv_nn_kernel (16-byte chunks
-//   of 8 k-rows per load), else lane = one output column, coalesced 2-byte
-//   row loads, 8 waves split K, LDS reduction.
+//   NN (B [K][N] row-major): M == 1 in gemv_nn_kernel (16-byte chunks of 8
+//   k-rows per load), else the tile kernels.
 // ---------------------------------------------------------------------------
 constexpr int SKINNY_M = 16;
 // M == 1 with row-major B [K][N] (the configs' weight layout): a workgroup owns
@@ -736,7 +760,7 @@ __global__ __launch_bounds__(1024) void gemv_nn_kernel(GemmArgs a) {
 //     16 kb + 4 g + j, one ds_read_b32 of n = 16 fn + l % 16: the four groups'
 //     rows land in four bank ranges.
 // Rows of A / B past m / n re-read the last row (never stored); k % 4 == 0.
-template <int BM, int BN, int WM, int WN, bool NN, int STAGES>
+template <int BM, int BN, int WM, int WN, bool NN, int STAGES, bool MASKED>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(GemmArgs a) {
     constexpr int THREADS = 64 * WM * WN;
     constexpr int BK = 32;
@@ -790,8 +814,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(GemmArgs a) {
         }
     }
     // A ragged k makes the first step short, as in gemm_mfma_dma_kernel.
-    const int nks = (a.k + BK - 1) / BK;
-    const int first = a.k - (nks - 1) * BK;
+    const int nks_all = (a.k + BK - 1) / BK;
+    const int first = a.k - (nks_all - 1) * BK;
+    const int nks = MASKED && hidden_tile(a.mask, min(m0 + BM, a.m) - 1, n0) ? 1 : nks_all;
     auto issue = [&](int ks) {
         const int k0 = ks == 0 ? 0 : ks * BK - (BK - first);
         u32x4* dA = sA + (ks % STAGES) * STA;
@@ -885,6 +910,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(GemmArgs a) {
         for (int fn = 0; fn < FN; ++fn) {
             const int n = n0 + wn * WTN + fn * 16 + 4 * g;
             f32x4 v = acc[fm][fn] * a.alpha;
+            if constexpr (MASKED) {
+                if (n < a.n) masked_store4<F32>(a.mask, crow, 1, m, n, a.n, v, a.beta);
+                continue;
+            }
             if (a.c_vec_ok && n + 3 < a.n) {
                 if (a.beta != 0.0f) v += a.beta * *reinterpret_cast<const f32x4*>(crow + n);
                 *reinterpret_cast<f32x4*>(crow + n) = v;
@@ -914,28 +943,23 @@ __global__ __launch_bounds__(256) void gemm_scale_kernel(void* C, int m, int n, 
 // ---------------------------------------------------------------------------
 namespace {
 
-template <class T, class TO, int BM, int BN, int WM, int WN, int STAGES>
+template <class T, class TO, int BM, int BN, int WM, int WN, int STAGES, bool SOFF = true, bool MASKED = false>
 hipError_t launch_dma_tile(const GemmArgs& a0, bool nn, int batch, hipStream_t s) {
     GemmArgs a = a0;
     a.tiles_m = (a.m + BM - 1) / BM;
     a.tiles_n = (a.n + BN - 1) / BN;
     dim3 grid(a.tiles_m * a.tiles_n, batch);
     dim3 block(64 * WM * WN);
-    // bytes spanned by one batch entry's A and B (the DMA addresses stay inside)
-    constexpr int64_t es = sizeof(typename T::raw);
-    const int64_t span_a = ((int64_t)(a.m - 1) * a.rsa + a.k) * es;
-    const int64_t span_b = (nn ? (int64_t)(a.k - 1) * a.rsb + a.n : (int64_t)(a.n - 1) * a.csb + a.k) * es;
-    const bool soff = span_a < (int64_t(1) << 31) && span_b < (int64_t(1) << 31);
-    if constexpr (sizeof(typename T::raw) == 2) {
-        if (nn) {
-            if (soff) gemm_mfma_dma_kernel<T, TO, BM, BN, WM, WN, true, STAGES, true><<<grid, block, 0, s>>>(a);
-            else gemm_mfma_dma_kernel<T, TO, BM, BN, WM, WN, true, STAGES, false><<<grid, block, 0, s>>>(a);
-            return hipGetLastError();
-        }
-    }
-    if (soff) gemm_mfma_dma_kernel<T, TO, BM, BN, WM, WN, false, STAGES, true><<<grid, block, 0, s>>>(a);
-    else gemm_mfma_dma_kernel<T, TO, BM, BN, WM, WN, false, STAGES, false><<<grid, block, 0, s>>>(a);
+    if (nn) gemm_mfma_dma_kernel<T, TO, BM, BN, WM, WN, true, STAGES, SOFF, MASKED><<<grid, block, 0, s>>>(a);
+    else gemm_mfma_dma_kernel<T, TO, BM, BN, WM, WN, false, STAGES, SOFF, MASKED><<<grid, block, 0, s>>>(a);
     return hipGetLastError();
+}
+
+// 16-bit operands that span 2^31 bytes or more
+bool dma_far(const GemmArgs& a, bool nn) {
+    const int64_t span_a = ((int64_t)(a.m - 1) * a.rsa + a.k) * 2;
+    const int64_t span_b = (nn ? (int64_t)(a.k - 1) * a.rsb + a.n : (int64_t)(a.n - 1) * a.csb + a.k) * 2;
+    return span_a >= (int64_t(1) << 31) || span_b >= (int64_t(1) << 31);
 }
 
 template <class T, class TO>
@@ -943,21 +967,26 @@ hipError_t launch_dma(const GemmArgs& a, bool nn, int batch, hipStream_t s) {
     auto tiles = [&](int bm, int bn) {
         return (int64_t)((a.m + bm - 1) / bm) * ((a.n + bn - 1) / bn) * batch;
     };
-    // Chosen from a sweep of M x N x K shapes on MI355X (bf16): the 256 x 256 tile
-    // once it has most of the 256 CUs busy, 128 x 128 (two workgroups per CU) for
-    // mid sizes, 64 x 64 below that; the 64 x 64 ring pays off only while its
-    // grid is short of several workgroups per CU.
+    // bytes spanned by one batch entry's A and B: below 2^31 the DMA goes from a
+    // scalar base plus 32-bit lane offsets
+    const bool far = dma_far(a, nn);
+    auto cost = [&](int bm, int bn) { return (tiles(bm, bn) + 255) / 256 * (bm + bn); };
+    if (a.mask.kind != YTHIP_MASK_NONE) {  // (the caller sends far operands elsewhere)
+        if (cost(128, 128) < cost(64, 64)) return launch_dma_tile<T, TO, 128, 128, 2, 4, 4, true, true>(a, nn, batch, s);
+        return launch_dma_tile<T, TO, 64, 64, 2, 2, 4, true, true>(a, nn, batch, s);
+    }
+    if (far) {
+        if (tiles(256, 256) >= 192) return launch_dma_tile<T, TO, 256, 256, 2, 4, 2, false>(a, nn, batch, s);
+        if (tiles(128, 128) >= 256) return launch_dma_tile<T, TO, 128, 128, 2, 2, 2, false>(a, nn, batch, s);
+        return launch_dma_tile<T, TO, 64, 64, 2, 2, 4, false>(a, nn, batch, s);
+    }
     if (tiles(256, 256) >= 192) {
-        if constexpr (sizeof(typename T::raw) == 2) {
-            // whole 256-row tiles: the ping-pong schedule (same bits)
-            constexpr int64_t es = 2;
-            const int64_t span_a = ((int64_t)(a.m - 1) * a.rsa + a.k) * es;
-            const int64_t span_b = (nn ? (int64_t)(a.k - 1) * a.rsb + a.n : (int64_t)(a.n - 1) * a.csb + a.k) * es;
-            // NT with a partial last column of tiles: the whole tiles on the
-            // ping-pong kernel, the last N % 256 columns as a product of their own
-            // (disjoint columns of C; B rows and C columns offset).
-            if (!nn && a.m % 256 == 0 && a.k % 64 == 0 && a.n % 256 != 0 && a.n > 256 && span_a < (int64_t(1) << 31) &&
-                span_b < (int64_t(1) << 31)) {
+        // whole 256-row tiles: the ping-pong schedule (same bits). NT with a partial
+        // last column of tiles: the whole tiles on the ping-pong kernel, the last
+        // N % 256 columns as a product of their own (disjoint columns of C; B rows
+        // and C columns offset).
+        if (a.m % 256 == 0 && a.k % 64 == 0) {
+            if (!nn && a.n % 256 != 0 && a.n > 256) {
                 using oraw = typename TO::raw;
                 GemmArgs g = a;
                 g.n = a.n / 256 * 256;
@@ -972,8 +1001,7 @@ hipError_t launch_dma(const GemmArgs& a, bool nn, int batch, hipStream_t s) {
                 r.C = static_cast<oraw*>(a.C) + g.n;
                 return launch_dma<T, TO>(r, nn, batch, s);
             }
-            if (a.m % 256 == 0 && a.k % 64 == 0 && (nn ? a.n % 16 == 0 : a.n % 256 == 0) && span_a < (int64_t(1) << 31) &&
-                span_b < (int64_t(1) << 31)) {
+            if (nn ? a.n % 16 == 0 : a.n % 256 == 0) {
                 GemmArgs g = a;
                 g.tiles_m = a.m / 256;
                 g.tiles_n = (a.n + 255) / 256;
@@ -985,13 +1013,27 @@ hipError_t launch_dma(const GemmArgs& a, bool nn, int batch, hipStream_t s) {
         }
         return launch_dma_tile<T, TO, 256, 256, 2, 4, 2>(a, nn, batch, s);
     }
-    if (tiles(128, 128) >= 384) return launch_dma_tile<T, TO, 128, 128, 2, 2, 2>(a, nn, batch, s);
-    if (tiles(64, 64) >= 768) return launch_dma_tile<T, TO, 64, 64, 2, 2, 2>(a, nn, batch, s);
-    // Fewer 64 x 64 tiles than CUs: 64 x 32 tiles (two waves) put twice as many
-    // workgroups, hence CUs, on the operand stream (7-10% on the Qwen3 prefill
-    // projections with weights coming from HBM).
-    if (tiles(64, 64) < 256) return launch_dma_tile<T, TO, 64, 32, 2, 1, 4>(a, nn, batch, s);
-    return launch_dma_tile<T, TO, 64, 64, 2, 2, 4>(a, nn, batch, s);
+    // Every tile's k loop runs at about the same bytes a clock into its CU's LDS
+    // (20 to 27, one workgroup or several), so the time is what the busiest CU
+    // stages: passes over the 256 CUs times BM + BN rows a k step. The smallest wins,
+    // the smaller tile when even (its ramp is shorter). Measured on bf16, the rule's
+    // tile against the one of a rule by tile counts that stood here: 2048^3 NN 24.0 /
+    // 31.3 us, 2400^3 40.5 / 62.9, 1536^3 16.2 / 19.1, 512 x 6144 x 1024 NT 12.2 / 12.8
+    // (weights from HBM 13.8 / 16.4), 512 x 4096 x 1024 NT 9.5 / 9.6 (10.3 / 12.0), 2048 x
+    // 1024 x 3072 NT 23.4 / 24.6 (25.1 / 29.5). A ring deeper than 4 steps loses at
+    // every size (512 x 1024 x 3072: 13.6, 8 deep 14.8, 12 deep 17.6 us).
+    const int64_t c0 = cost(64, 32), c1 = cost(64, 64), c2 = cost(128, 64), c3 = cost(128, 128), c4 = cost(256, 128);
+    const int64_t best = std::min(std::min(std::min(c0, c1), std::min(c2, c3)), c4);
+    if (c0 == best) return launch_dma_tile<T, TO, 64, 32, 2, 1, 4>(a, nn, batch, s);
+    if (c1 == best) return launch_dma_tile<T, TO, 64, 64, 2, 2, 4>(a, nn, batch, s);
+    if (c2 == best) return launch_dma_tile<T, TO, 128, 64, 2, 2, 3>(a, nn, batch, s);
+    if (c3 == best) {
+        // one per CU: eight waves and a deep ring; several: two resident per CU
+        // (3072^3: 75.9 us, 80.2 with the deep ring)
+        if (tiles(128, 128) <= 256) return launch_dma_tile<T, TO, 128, 128, 2, 4, 4>(a, nn, batch, s);
+        return launch_dma_tile<T, TO, 128, 128, 2, 2, 2>(a, nn, batch, s);
+    }
+    return launch_dma_tile<T, TO, 256, 128, 2, 4, 3>(a, nn, batch, s);
 }
 
 template <class TO>
@@ -1007,10 +1049,11 @@ bool aligned(const void* p, int bytes) { return (reinterpret_cast<uintptr_t>(p) 
 template <class T, class TO>
 int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int64_t rsa, int64_t csa,
                const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C, int64_t sc_b, int64_t rsc,
-               int64_t csc, float alpha, float beta, hipStream_t s) {
+               int64_t csc, float alpha, float beta, const MaskDesc& mask, hipStream_t s) {
     using raw = typename T::raw;
     using oraw = typename TO::raw;
     constexpr int VEC = 16 / sizeof(raw);
+    const bool plain = mask.kind == YTHIP_MASK_NONE;
     if (k == 0 || alpha == 0.0f) return status_of(launch_scale<TO>(C, m, n, rsc, csc, sc_b, beta, batch, s));
 
     const int es = sizeof(raw);
@@ -1027,7 +1070,8 @@ int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int6
         g.alpha = alpha; g.beta = beta;
         g.c_vec_ok = (rsc % 4 == 0) && (sc_b % 4 == 0) && aligned(C, 4 * sizeof(oraw));
         g.c_line_ok = sizeof(oraw) == 2 && (rsc % 8 == 0) && (sc_b % 8 == 0) && aligned(C, 16);
-        if (m <= SKINNY_M) {
+        g.mask = mask;
+        if (m <= SKINNY_M && plain) {
             if (nt) {
                 GemvArgs v{};
                 v.A = A; v.lda = rsa; v.W = B; v.ldw = csb; v.C = C; v.ldc = rsc;
@@ -1048,11 +1092,10 @@ int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int6
                 return status_of(hipGetLastError());
             }
             // 2..16 rows of a row-major, 16-bit B: the MFMA DMA path (one partial
-            // 64-row tile per column tile) streams B at full width; the column-per-
-            // lane kernel below re-reads A per k and issues 2-byte loads of B
-            // ((16, 3072, 1024): ~100 us there)
-            if (es == 2 && (rsb % VEC) == 0 && (sb_b % VEC) == 0 && (n % VEC) == 0 && aligned(B, 16))
-                return status_of(launch_dma<T, TO>(g, true, batch, s));
+            // 64-row tile per column tile) streams B at full width
+            if constexpr (sizeof(raw) == 2)
+                if ((rsb % VEC) == 0 && (sb_b % VEC) == 0 && (n % VEC) == 0 && aligned(B, 16))
+                    return status_of(launch_dma<T, TO>(g, true, batch, s));
         }
         if constexpr (std::is_same_v<T, F32> && std::is_same_v<TO, F32>) {
             // fp32 on the DMA-staged fp32 MFMA kernel: 16-byte aligned rows of A and
@@ -1068,13 +1111,18 @@ int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int6
                 const dim3 grid(f.tiles_m * f.tiles_n, batch);
                 // 1024^3 (256 tiles of 64 x 64): 8 waves of 32 x 16 and a 4-step ring,
                 // 99 TFLOP/s NN; 4 waves or 3 steps 86-98, 32 x 64 or 64 x 128 tiles <= 92
-                if (big) {
-                    if (f_nn) gemm_f32_kernel<128, 128, 2, 4, true, 3><<<grid, 512, 0, s>>>(f);
-                    else gemm_f32_kernel<128, 128, 2, 4, false, 3><<<grid, 512, 0, s>>>(f);
-                } else {
-                    if (f_nn) gemm_f32_kernel<64, 64, 2, 4, true, 4><<<grid, 512, 0, s>>>(f);
-                    else gemm_f32_kernel<64, 64, 2, 4, false, 4><<<grid, 512, 0, s>>>(f);
-                }
+                auto launch = [&](auto masked) {
+                    constexpr bool M = decltype(masked)::value;
+                    if (big) {
+                        if (f_nn) gemm_f32_kernel<128, 128, 2, 4, true, 3, M><<<grid, 512, 0, s>>>(f);
+                        else gemm_f32_kernel<128, 128, 2, 4, false, 3, M><<<grid, 512, 0, s>>>(f);
+                    } else {
+                        if (f_nn) gemm_f32_kernel<64, 64, 2, 4, true, 4, M><<<grid, 512, 0, s>>>(f);
+                        else gemm_f32_kernel<64, 64, 2, 4, false, 4, M><<<grid, 512, 0, s>>>(f);
+                    }
+                };
+                if (plain) launch(std::false_type{});
+                else launch(std::true_type{});
                 return status_of(hipGetLastError());
             }
         }
@@ -1083,19 +1131,22 @@ int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int6
         // against the register-staged kernel that took those before).
         const bool dma_nn = nn && es == 2 && (rsb % VEC) == 0 && (sb_b % VEC) == 0 && (n % VEC) == 0 &&
                             aligned(B, 16);
-        if (nt || dma_nn) return status_of(launch_dma<T, TO>(g, nn, batch, s));
+        if constexpr (sizeof(raw) == 2)
+            if ((nt || dma_nn) && (plain || !dma_far(g, nn))) return status_of(launch_dma<T, TO>(g, nn, batch, s));
     }
     return gemm_any_dispatch(T::code, TO::code, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b, rsc, csc,
-                             alpha, beta, s);
+                             alpha, beta, mask, s);
 }
 
 }  // namespace
 
-int gemm_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, const void* A, int64_t sa_b,
-                  int64_t rsa, int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C,
-                  int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, hipStream_t s) {
-#define YTHIP_GEMM(TI, TOUT) \
-    return gemm_typed<TI, TOUT>(batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b, rsc, csc, alpha, beta, s)
+int gemm_masked_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, const void* A, int64_t sa_b,
+                         int64_t rsa, int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C,
+                         int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, const MaskDesc& mask,
+                         hipStream_t s) {
+#define YTHIP_GEMM(TI, TOUT)                                                                                        \
+    return gemm_typed<TI, TOUT>(batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b, rsc, csc, alpha, beta, \
+                                mask, s)
     if (dtype_in == YTHIP_F32 && dtype_out == YTHIP_F32) YTHIP_GEMM(F32, F32);
     if (dtype_in == YTHIP_BF16 && dtype_out == YTHIP_BF16) YTHIP_GEMM(BF16, BF16);
     if (dtype_in == YTHIP_BF16 && dtype_out == YTHIP_F32) YTHIP_GEMM(BF16, F32);
@@ -1104,6 +1155,13 @@ int gemm_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, c
 #undef YTHIP_GEMM
     return fail(YTHIP_EUNSUPPORTED, "ythip_gemm: unsupported dtype_in/dtype_out combination %d/%d", dtype_in,
                 dtype_out);
+}
+
+int gemm_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, const void* A, int64_t sa_b,
+                  int64_t rsa, int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C,
+                  int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, hipStream_t s) {
+    return gemm_masked_dispatch(dtype_in, dtype_out, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b, rsc,
+                                csc, alpha, beta, MaskDesc{YTHIP_MASK_NONE, nullptr, 0, 0, 0, 0.f}, s);
 }
 
 }  // namespace ythip

@@ -41,13 +41,11 @@ struct AnyArgs {
     int64_t sa_b, sb_b, sc_b;
     float alpha, beta;
     int tiles_m, tiles_n;
+    MaskDesc mask;
+    int mask_t;  // C is the transpose of the masked matrix
 };
 
 enum { KC = 0, RC = 1, ST = 2 };
-
-typedef u32x4 u32x4_any __attribute__((aligned(2)));
-typedef u32x2 u32x2_any __attribute__((aligned(2)));
-typedef f32x4 f32x4_any __attribute__((aligned(4)));
 
 __device__ __forceinline__ int any_swz(int row, int chunk) { return chunk ^ ((row ^ (row >> 3)) & 7); }
 
@@ -210,7 +208,7 @@ struct Stager {
     }
 };
 
-template <class T, class TO, int BM, int BN, int WM, int WN, int AM, int BMODE>
+template <class T, class TO, int BM, int BN, int WM, int WN, int AM, int BMODE, bool MASKED>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_any_kernel(AnyArgs a) {
     using raw = typename T::raw;
     constexpr int THREADS = 64 * WM * WN;
@@ -238,8 +236,11 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_any_kernel(AnyArgs a) {
     typename SB::Regs rb[PF];
     const bool raga = a.m < m0 + BM && (a.m & 3) != 0, ragb = a.n < n0 + BN && (a.n & 3) != 0;
 
-    const int steps = (a.k + BK - 1) / BK;
-    const int first = a.k - (steps - 1) * BK;  // k in the first step
+    // (a tile that the mask hides whole: one step, its sums are not used)
+    const bool hidden = MASKED && !a.mask_t && hidden_tile(a.mask, min(m0 + BM, a.m) - 1, n0);
+    const int all = (a.k + BK - 1) / BK;
+    const int first = a.k - (all - 1) * BK;  // k in the first step
+    const int steps = hidden ? 1 : all;
     // Past the last step the last one is read again: a load under a condition would
     // make every later wait a wait for all loads.
     auto load = [&](int p, int kt) {
@@ -330,6 +331,22 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_any_kernel(AnyArgs a) {
             const int n = n0 + wn * WTN + j * 16 + g * 4;
             if (n >= a.n) continue;
             f32x4 v = acc[i][j];
+            if constexpr (MASKED) {
+                if (!a.mask_t) {
+                    masked_store4<TO>(a.mask, crow, a.csc, m, n, a.n, v * a.alpha, a.beta);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        if (n + r >= a.n) continue;
+                        const int64_t at = (n + r) * a.csc;
+                        float x = v[r] * a.alpha;
+                        if (a.beta != 0.0f) x += a.beta * load_as_f32<TO>(crow, at);
+                        if (visible(a.mask, n + r, m)) store_from_f32<TO>(crow, at, x);
+                        else if (a.mask.fill) store_from_f32<TO>(crow, at, a.mask.value);
+                    }
+                }
+                continue;
+            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 v[r] *= a.alpha;
@@ -367,14 +384,15 @@ hipError_t launch_any_mode(AnyArgs a, int batch, hipStream_t s) {
         // bf16 97 us on 64 x 64 tiles, 67 us on 128 x 128; fp32 251 us on 64 x 64.
         const bool wide = sizeof(typename T::raw) == 2 ? rounds(128) * 128 < rounds(64) * 64
                                                        : rounds(128) * 128 * 128 <= rounds(64) * 64 * 64;
-        if (wide) {
+        if (wide && a.mask.kind == YTHIP_MASK_NONE) {
             const dim3 gr = grid(128);
-            gemm_any_kernel<T, TO, 128, 128, 2, WN, AM, BMODE><<<gr, 128 * WN, 0, s>>>(a);
+            gemm_any_kernel<T, TO, 128, 128, 2, WN, AM, BMODE, false><<<gr, 128 * WN, 0, s>>>(a);
             return hipGetLastError();
         }
     }
     const dim3 gr = grid(64);
-    gemm_any_kernel<T, TO, 64, 64, 2, WN, AM, BMODE><<<gr, 128 * WN, 0, s>>>(a);
+    if (a.mask.kind == YTHIP_MASK_NONE) gemm_any_kernel<T, TO, 64, 64, 2, WN, AM, BMODE, false><<<gr, 128 * WN, 0, s>>>(a);
+    else gemm_any_kernel<T, TO, 64, 64, 2, WN, AM, BMODE, true><<<gr, 128 * WN, 0, s>>>(a);
     return hipGetLastError();
 }
 
@@ -401,9 +419,10 @@ hipError_t launch_any(const AnyArgs& a, int batch, hipStream_t s) {
 
 int gemm_any_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, const void* A, int64_t sa_b,
                       int64_t rsa, int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C,
-                      int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, hipStream_t s) {
-    AnyArgs a{A, B, C, m, n, k, rsa, csa, rsb, csb, rsc, csc, sa_b, sb_b, sc_b, alpha, beta, 0, 0};
+                      int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, const MaskDesc& mask, hipStream_t s) {
+    AnyArgs a{A, B, C, m, n, k, rsa, csa, rsb, csb, rsc, csc, sa_b, sb_b, sc_b, alpha, beta, 0, 0, mask, 0};
     if (csc != 1 && rsc == 1) {  // a column-major C: C^T = B^T . A^T, so that its stores run along memory
+        a.mask_t = 1;
         std::swap(a.A, a.B);
         std::swap(a.m, a.n);
         std::swap(a.rsa, a.csb);

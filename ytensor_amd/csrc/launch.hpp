@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/ythip.h"
+#include "common.hpp"
 
 namespace ythip {
 
@@ -19,10 +20,17 @@ int gemm_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, c
                   int64_t rsa, int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C,
                   int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, hipStream_t s);
 
+// The same where the mask shows C; k > 0, alpha != 0.
+int gemm_masked_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, const void* A, int64_t sa_b,
+                         int64_t rsa, int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C,
+                         int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, const MaskDesc& mask,
+                         hipStream_t s);
+
 // Any layout, size and alignment (gemm_any.hip); k > 0.
 int gemm_any_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, const void* A, int64_t sa_b,
                       int64_t rsa, int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C,
-                      int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, hipStream_t s);
+                      int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, const MaskDesc& mask,
+                      hipStream_t s);
 
 // The MATH attention backend in one launch (attention.hip); -1 when the layout is
 // not one of the MFMA kernels' (nothing was launched).
