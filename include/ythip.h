@@ -85,6 +85,41 @@ int ythip_gemm(int dtype_in, int dtype_out, int batch, int m, int n, int k,
                float alpha, float beta, void* stream);
 
 /*
+ * ythip_gemm for one matrix with a workspace: a 16-bit product against a weight
+ * ([n][k] rows, rsb == 1) whose grid is too small for the chip is cut along k into fp32
+ * products computed side by side in the workspace and summed by a second launch.
+ * ythip_gemm_workspace_size gives the bytes that takes, 0 where one launch is faster;
+ * then, in another layout or with a smaller workspace this is ythip_gemm.
+ * ythip_gemm_splits: the parts that pay where the caller sums them in a launch it has
+ * anyway (a batch of ythip_gemm over k / parts columns, then ythip_residual_rms_norm).
+ */
+size_t ythip_gemm_workspace_size(int dtype, int m, int n, int k);
+int ythip_gemm_splits(int dtype, int m, int n, int k);
+int ythip_gemm_ws(int dtype_in, int dtype_out, int m, int n, int k, const void* A, int64_t rsa, int64_t csa,
+                  const void* B, int64_t rsb, int64_t csb, void* C, int64_t rsc, int64_t csc, float alpha, float beta,
+                  void* workspace, size_t ws_bytes, void* stream);
+
+/*
+ * The MLP's first half for any number of rows (Qwen3MLP::forward,
+ * example/qwen3/src/qwen3.cpp:193-200): C[m, i] = swish(g) * u with g = A.W[i]^T and
+ * u = A.W[inter + i]^T each rounded to dtype first, W = [gate rows | up rows]
+ * [2*inter][k]: the bits of ythip_gemm into [m][2*inter] followed by ythip_silu_mul.
+ * bf16 / fp16; 16-byte aligned rows of A and W below 2^31 bytes each, 8-byte aligned
+ * rows of C, k % 8 == 0, inter % 4 == 0 (YTHIP_EUNSUPPORTED otherwise).
+ */
+int ythip_gemm_swiglu(int dtype, int m, int inter, int k, const void* A, int64_t lda, const void* W, int64_t ldw,
+                      void* C, int64_t ldc, void* stream);
+
+/*
+ * The residual add and the RMSNorm that follows it (example/qwen3/src/qwen3.cpp:
+ * 271-283) over a projection left in parts: x[r] += sum over s of partials[s][r] (fp32
+ * [splits][rows][n]), then, with w given, y = rmsNorm_(x, w, eps) in dtype_out, with
+ * the arithmetic of ythip_rms_norm. n <= 4096.
+ */
+int ythip_residual_rms_norm(int dtype_out, int rows, int n, int splits, const float* partials, float* x, int64_t ld_x,
+                            const float* w, float eps, void* y, int64_t ld_y, void* stream);
+
+/*
  * Attention forward, prefill (any q_len >= 1):
  *   O[b,h] = softmax(scale * Q[b,h] . K[b,h/G]^T + bias, masked) . V[b,h/G],  G = Hq / Hkv
  * Q: [B,Hq,q_len,d], K: [B,Hkv,kv_len,d], V: [B,Hkv,kv_len,dv], O: [B,Hq,q_len,dv];

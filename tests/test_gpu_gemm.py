@@ -470,3 +470,62 @@ def test_ragged_k_reads_nothing_past_it(yt, layout, dtype):
         Ac, Bc = A[:m, :k].contiguous(), B[:rows, :cols].contiguous()
         want = yt.matmul(Ac, Bc if layout == "NN" else Bc.t())
         assert torch.isfinite(C).all() and torch.equal(C, want)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,n,k", [(17, 1024, 2048), (64, 1024, 3072), (100, 36, 4096), (130, 1000, 2048), (24, 1024, 3072),
+                                   (512, 1024, 3072), (2, 64, 768)])
+def test_split_k_products(yt, m, n, k, dt):
+    """Products cut along k: linear through the workspace call (rows at an odd offset
+    fall back to one launch), gemm_parts with the residual add and norm, at splits of
+    2, 4 and 8, against float64; the norm's bits are those of rms_norm on the same
+    sum. Bound: (k + 10) 2^-24 sum|a||b| plus the rounding of the result."""
+    from ytensor_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=g).to(dt)
+    w = (torch.randn(n, k, device="cuda", generator=g) * 0.05).to(dt)
+    want = x.double() @ w.double().T
+    mass = x.double().abs() @ w.double().abs().T
+    ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -10}[dt]
+    tol = (k + 10) * 2.0 ** -24 * mass
+    assert ((yt.linear(x, w).double() - want).abs() <= tol + ulp * want.abs()).all()
+    assert ((yt.linear(x, w, out_dtype=torch.float32).double() - want).abs() <= tol + 2.0 ** -23 * want.abs()).all()
+    pad = torch.empty(m, k + 1, device="cuda", dtype=dt)
+    pad[:, 1:] = x
+    assert ((yt.linear(pad[:, 1:], w).double() - want).abs() <= tol + ulp * want.abs()).all()
+    for s in {2, 4, 8, ops.gemm_splits(dt, m, n, k)} - {1}:
+        parts = torch.empty(s, m, n, device="cuda")
+        ops.gemm_parts(x, w, parts)
+        r0 = torch.randn(m, n, device="cuda", generator=g)
+        r, nw, out = r0.clone(), torch.randn(n, device="cuda", generator=g), torch.empty(m, n, device="cuda", dtype=dt)
+        ops.residual_rms_norm(r, parts, nw, 1e-6, out)
+        full = r0.double() + want
+        assert ((r.double() - full).abs() <= tol + 2.0 ** -21 * (full.abs() + r0.abs())).all(), s
+        assert torch.equal(out, yt.rms_norm(r, nw, 1e-6, out=torch.empty_like(out)))
+        r2 = r0.clone()
+        ops.residual_rms_norm(r2, parts)
+        assert torch.equal(r2, r)
+    parts = torch.randn(3, m, n, device="cuda", generator=g)  # a count without a form of its own
+    r3 = torch.zeros(m, n, device="cuda")
+    ops.residual_rms_norm(r3, parts)
+    assert torch.equal(r3, parts[0] + parts[1] + parts[2])
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,inter,k", [(1, 4, 8), (17, 100, 72), (64, 32, 64), (130, 516, 200), (300, 3072, 1024), (512, 3072, 1024),
+                                       (700, 3072, 128)])
+def test_gemm_swiglu_equals_gemm_then_silu(yt, m, inter, k, dt):
+    """gate_up + SwiGLU in one product (every tile of its rule, ragged m, inter, k) has
+    the bits of the product into [m, 2 inter] followed by silu_mul."""
+    from ytensor_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(m + inter + k)
+    x = torch.randn(m, k, device="cuda", generator=g).to(dt)
+    w = (torch.randn(2 * inter, k, device="cuda", generator=g) * 0.1).to(dt)
+    out = ops.gemm_swiglu(x, w, torch.empty(m, inter, device="cuda", dtype=dt))
+    gu = torch.empty(m, 2 * inter, device="cuda", dtype=dt)
+    yt.gemm(x, w.t(), gu)
+    want = yt.silu_mul(gu)
+    if m > 16:
+        assert torch.equal(out, want)
+    else:  # gemm takes its GEMV there: sums in another order
+        assert ((out.double() - want.double()).abs() <= 2.0 ** -6 * want.double().abs() + 1e-3).all()

@@ -46,6 +46,11 @@ SIGNATURES = {
     "ythip_abi_version": (_I, []),
     "ythip_last_error": (ctypes.c_char_p, []),
     "ythip_gemm": (_I, [_I, _I, _I, _I, _I, _I, _P, _L, _L, _L, _P, _L, _L, _L, _P, _L, _L, _L, _F, _F, _P]),
+    "ythip_gemm_splits": (_I, [_I, _I, _I, _I]),
+    "ythip_gemm_workspace_size": (ctypes.c_size_t, [_I, _I, _I, _I]),
+    "ythip_gemm_ws": (_I, [_I, _I, _I, _I, _I, _P, _L, _L, _P, _L, _L, _P, _L, _L, _F, _F, _P, ctypes.c_size_t, _P]),
+    "ythip_gemm_swiglu": (_I, [_I, _I, _I, _I, _P, _L, _P, _L, _P, _L, _P]),
+    "ythip_residual_rms_norm": (_I, [_I, _I, _I, _I, _P, _P, _L, _P, _F, _P, _L, _P]),
     "ythip_attn_prefill": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _P, _LP, _P, _LP, _P, _LP, _P, _LP,
                                 _F, _I, _P, _L, _P, _L, _L, _P]),
     "ythip_attn_prefill_workspace_size": (ctypes.c_size_t, [_I, _I]),

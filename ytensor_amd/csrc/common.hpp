@@ -154,6 +154,14 @@ __device__ __forceinline__ void masked_store4(const MaskDesc& mk, typename TO::r
     }
 }
 
+// swish(a) * u with the stable sigmoid of src/ytensor_function.inl:43-52, as
+// ythip_silu_mul computes it.
+__device__ __forceinline__ float swish_mul(float a, float u) {
+    const float z = expf(a >= 0.0f ? -a : a);
+    const float sig = a >= 0.0f ? 1.0f / (1.0f + z) : z / (1.0f + z);
+    return (a * sig) * u;
+}
+
 // Tile order of the GEMM grids, XCD-aware: the hardware places workgroup w on
 // XCD w % 8, so (when the tile count is a multiple of 8) w is remapped to give
 // each XCD a contiguous range of tiles, taken 4 tile-rows at a time so that an

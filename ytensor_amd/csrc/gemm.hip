@@ -85,8 +85,13 @@ static __device__ const u32x4 dma_zero[1] = {{0u, 0u, 0u, 0u}};
 // per-lane 32-bit byte offset fixed for the whole k loop (dma16_soff), and the
 // LDS destination is the wave's base plus constants -- no VALU address work
 // between the MFMAs of consecutive k steps.
-// MASKED: a masked product (the mask's code costs every other form its length).
-template <class T, class TO, int BM, int BN, int WM, int WN, bool NN, int STAGES, bool SOFF, bool MASKED>
+// FORM (templates, since the forms' code would cost the others its length):
+//   PLAIN; MASKED: a masked product;
+//   SWIGLU (NT): B = [gate rows | up rows], a.n columns of C each: a wave's fragments
+//   alternate between 16 gate rows and the same 16 up rows, so a lane holds both
+//   factors of its activations and the [m][2 n] product is never written.
+enum { PLAIN = 0, MASKED = 1, SWIGLU = 2 };
+template <class T, class TO, int BM, int BN, int WM, int WN, bool NN, int STAGES, bool SOFF, int FORM>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a) {
     using raw = typename T::raw;
     constexpr int THREADS = 64 * WM * WN;
@@ -124,7 +129,18 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
     const int KT_all = (a.k + BK - 1) / BK;
     const int first = a.k - (KT_all - 1) * BK;
     // a tile that the mask hides whole: its sums are not used
-    const int KT = MASKED && hidden_tile(a.mask, min(m0 + BM, a.m) - 1, n0) ? 1 : KT_all;
+    const int KT = FORM == MASKED && hidden_tile(a.mask, min(m0 + BM, a.m) - 1, n0) ? 1 : KT_all;
+
+    // the B row behind row r of an NT tile
+    auto b_row = [&](int r) -> int64_t {
+        if constexpr (FORM == SWIGLU) {
+            const int f = (r % WTN) / 16;
+            const int col = n0 / 2 + r / WTN * (WTN / 2) + f / 2 * 16 + r % 16;
+            return (f & 1 ? a.n : 0) + min(col, a.n - 1);
+        } else {
+            return min(n0 + r, a.n - 1);
+        }
+    };
 
     // Step 0 of a ragged k, and every step of operands too large for SOFF.
     auto issue_a = [&](int kt, u32x4* sA) {
@@ -149,8 +165,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
             if constexpr (!NN) {
                 const int r = slot >> 3;
                 const int c = swz_dma(r, slot & 7);
-                const int row = min(n0 + r, a.n - 1);
-                g = Bp + (int64_t)row * a.csb + k0 + c * VEC;
+                g = Bp + b_row(r) * a.csb + k0 + c * VEC;
                 if (kt == 0 && c * VEC >= first) g = reinterpret_cast<const raw*>(dma_zero);
             } else {
                 const int r = slot / (2 * NBLK), ps = slot % (2 * NBLK);
@@ -180,7 +195,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
             if constexpr (!NN) {
                 const int r = slot >> 3;
                 const int c = swz_dma(r, slot & 7);
-                e = (int64_t)min(n0 + r, a.n - 1) * a.csb + c * VEC;
+                e = b_row(r) * a.csb + c * VEC;
             } else {
                 const int r = slot / (2 * NBLK), ps = slot % (2 * NBLK);
                 const int lb = nn_blk(r, ps >> 1, BLK_MASK);
@@ -302,9 +317,32 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
 
     using oraw = typename TO::raw;
     oraw* Cp = static_cast<oraw*>(a.C) + bz * a.sc_b;
+    if constexpr (FORM == SWIGLU) {
+        static_assert(FN % 2 == 0 && !NN && sizeof(oraw) == 2, "gate and up fragments in pairs");
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const int m = m0 + wm * WTM + i * 16 + lrow;
+            if (m >= a.m) continue;
+#pragma unroll
+            for (int j = 0; j < FN; j += 2) {
+                const int n = n0 / 2 + wn * (WTN / 2) + j * 8 + lgrp * 4;
+                uint32_t v[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t gu = pack2<TO>(acc[i][j][r], acc[i][j + 1][r]);  // both rounded first
+                    const float y = swish_mul(lo_as_f32(TO{}, gu), hi_as_f32(TO{}, gu));
+                    // silu_mul's conversion, element by element (fp16 subnormals)
+                    v[r] = std::is_same_v<TO, F16> ? f32_to_f16_bits(y) : f32_to_bf16_bits(y);
+                }
+                if (n < a.n)  // a.n % 4 == 0
+                    *reinterpret_cast<u32x2*>(Cp + (int64_t)m * a.rsc + n) = u32x2{v[0] | v[1] << 16, v[2] | v[3] << 16};
+            }
+        }
+        return;
+    }
     float alpha = a.alpha;
-    const bool filled = MASKED && a.mask.fill && a.beta == 0.0f;
-    if (MASKED && filled) {  // every entry is written: the value where hidden, then the stores of a plain product
+    const bool filled = FORM == MASKED && a.mask.fill && a.beta == 0.0f;
+    if (FORM == MASKED && filled) {  // every entry is written: the value where hidden, then the stores of a plain product
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
             const int m = min(m0 + wm * WTM + i * 16 + lrow, a.m - 1);
@@ -318,7 +356,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
         alpha = 1.0f;
     }
     if constexpr (sizeof(oraw) == 2 && BN >= 64) {
-        if (a.beta == 0.0f && (!MASKED || filled) && a.c_line_ok && m0 + BM <= a.m && n0 + BN <= a.n) {
+        if (a.beta == 0.0f && (FORM != MASKED || filled) && a.c_line_ok && m0 + BM <= a.m && n0 + BN <= a.n) {
             // A whole 16-bit tile leaves through LDS in rows of BN elements (chunk c of
             // row r at c ^ (r % CPR)): each thread stores 16-byte chunks of whole tile
             // rows, 128-byte lines and up, instead of the fragments' 8-byte pieces of
@@ -358,7 +396,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_dma_kernel(GemmArgs a)
             const int n = n0 + wn * WTN + j * 16 + lgrp * 4;
             if (n >= a.n) continue;
             oraw* crow = Cp + (int64_t)m * a.rsc;
-            if (MASKED && !filled) {
+            if (FORM == MASKED && !filled) {
                 masked_store4<TO>(a.mask, crow, 1, m, n, a.n, acc[i][j] * alpha, a.beta);
                 continue;
             }
@@ -760,7 +798,7 @@ __global__ __launch_bounds__(1024) void gemv_nn_kernel(GemmArgs a) {
 //     16 kb + 4 g + j, one ds_read_b32 of n = 16 fn + l % 16: the four groups'
 //     rows land in four bank ranges.
 // Rows of A / B past m / n re-read the last row (never stored); k % 4 == 0.
-template <int BM, int BN, int WM, int WN, bool NN, int STAGES, bool MASKED>
+template <int BM, int BN, int WM, int WN, bool NN, int STAGES, bool MASK>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(GemmArgs a) {
     constexpr int THREADS = 64 * WM * WN;
     constexpr int BK = 32;
@@ -816,7 +854,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(GemmArgs a) {
     // A ragged k makes the first step short, as in gemm_mfma_dma_kernel.
     const int nks_all = (a.k + BK - 1) / BK;
     const int first = a.k - (nks_all - 1) * BK;
-    const int nks = MASKED && hidden_tile(a.mask, min(m0 + BM, a.m) - 1, n0) ? 1 : nks_all;
+    const int nks = MASK && hidden_tile(a.mask, min(m0 + BM, a.m) - 1, n0) ? 1 : nks_all;
     auto issue = [&](int ks) {
         const int k0 = ks == 0 ? 0 : ks * BK - (BK - first);
         u32x4* dA = sA + (ks % STAGES) * STA;
@@ -910,7 +948,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_kernel(GemmArgs a) {
         for (int fn = 0; fn < FN; ++fn) {
             const int n = n0 + wn * WTN + fn * 16 + 4 * g;
             f32x4 v = acc[fm][fn] * a.alpha;
-            if constexpr (MASKED) {
+            if constexpr (MASK) {
                 if (n < a.n) masked_store4<F32>(a.mask, crow, 1, m, n, a.n, v, a.beta);
                 continue;
             }
@@ -943,15 +981,15 @@ __global__ __launch_bounds__(256) void gemm_scale_kernel(void* C, int m, int n, 
 // ---------------------------------------------------------------------------
 namespace {
 
-template <class T, class TO, int BM, int BN, int WM, int WN, int STAGES, bool SOFF = true, bool MASKED = false>
+template <class T, class TO, int BM, int BN, int WM, int WN, int STAGES, bool SOFF = true, int FORM = PLAIN>
 hipError_t launch_dma_tile(const GemmArgs& a0, bool nn, int batch, hipStream_t s) {
     GemmArgs a = a0;
     a.tiles_m = (a.m + BM - 1) / BM;
     a.tiles_n = (a.n + BN - 1) / BN;
     dim3 grid(a.tiles_m * a.tiles_n, batch);
     dim3 block(64 * WM * WN);
-    if (nn) gemm_mfma_dma_kernel<T, TO, BM, BN, WM, WN, true, STAGES, SOFF, MASKED><<<grid, block, 0, s>>>(a);
-    else gemm_mfma_dma_kernel<T, TO, BM, BN, WM, WN, false, STAGES, SOFF, MASKED><<<grid, block, 0, s>>>(a);
+    if (nn) gemm_mfma_dma_kernel<T, TO, BM, BN, WM, WN, true, STAGES, SOFF, FORM><<<grid, block, 0, s>>>(a);
+    else gemm_mfma_dma_kernel<T, TO, BM, BN, WM, WN, false, STAGES, SOFF, FORM><<<grid, block, 0, s>>>(a);
     return hipGetLastError();
 }
 
@@ -972,8 +1010,8 @@ hipError_t launch_dma(const GemmArgs& a, bool nn, int batch, hipStream_t s) {
     const bool far = dma_far(a, nn);
     auto cost = [&](int bm, int bn) { return (tiles(bm, bn) + 255) / 256 * (bm + bn); };
     if (a.mask.kind != YTHIP_MASK_NONE) {  // (the caller sends far operands elsewhere)
-        if (cost(128, 128) < cost(64, 64)) return launch_dma_tile<T, TO, 128, 128, 2, 4, 4, true, true>(a, nn, batch, s);
-        return launch_dma_tile<T, TO, 64, 64, 2, 2, 4, true, true>(a, nn, batch, s);
+        if (cost(128, 128) < cost(64, 64)) return launch_dma_tile<T, TO, 128, 128, 2, 4, 4, true, MASKED>(a, nn, batch, s);
+        return launch_dma_tile<T, TO, 64, 64, 2, 2, 4, true, MASKED>(a, nn, batch, s);
     }
     if (far) {
         if (tiles(256, 256) >= 192) return launch_dma_tile<T, TO, 256, 256, 2, 4, 2, false>(a, nn, batch, s);
@@ -1138,6 +1176,54 @@ int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int6
                              alpha, beta, mask, s);
 }
 
+// C = alpha * sum of the S parts' fp32 products + beta * C, four columns a thread; all
+// parts' loads are in flight at once.
+template <class TO, int S>
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ parts, int64_t mn, int n4,
+                                                            void* C, int64_t rsc, float alpha, float beta) {
+    const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (id * 4 >= mn) return;
+    f32x4 p[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) p[s] = *reinterpret_cast<const f32x4*>(parts + s * mn + id * 4);
+    f32x4 v = p[0];
+#pragma unroll
+    for (int s = 1; s < S; ++s) v += p[s];
+    const int64_t at = id / n4 * rsc + id % n4 * 4;
+    v *= alpha;
+    if (beta != 0.0f)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] += beta * load_as_f32<TO>(C, at + r);
+    auto* c = static_cast<typename TO::raw*>(C) + at;
+    if constexpr (sizeof(*c) == 2) *reinterpret_cast<u32x2_any*>(c) = u32x2{pack2<TO>(v[0], v[1]), pack2<TO>(v[2], v[3])};
+    else *reinterpret_cast<f32x4_any*>(c) = v;
+}
+
+template <class T>
+int swiglu_typed(const GemmArgs& a, hipStream_t s) {
+    auto cost = [&](int bm, int bn) {
+        return ((int64_t)((a.m + bm - 1) / bm) * ((2 * a.n + bn - 1) / bn) + 255) / 256 * (bm + bn);
+    };
+    auto launch = [&](auto bm, auto bn, auto wm, auto wn, auto stages) {
+        GemmArgs g = a;
+        g.tiles_m = (a.m + bm.value - 1) / bm.value;
+        g.tiles_n = (2 * a.n + bn.value - 1) / bn.value;
+        gemm_mfma_dma_kernel<T, T, bm.value, bn.value, wm.value, wn.value, false, stages.value, true, SWIGLU>
+            <<<dim3(g.tiles_m * g.tiles_n), 64 * wm.value * wn.value, 0, s>>>(g);
+        return status_of(hipGetLastError());
+    };
+    using std::integral_constant;
+#define YT_I(x) integral_constant<int, x> {}
+    // the tile rule of launch_dma
+    const int64_t c0 = cost(64, 32), c1 = cost(64, 64), c2 = cost(128, 64), c3 = cost(128, 128);
+    const int64_t best = std::min(std::min(c0, c1), std::min(c2, c3));
+    if (c0 == best) return launch(YT_I(64), YT_I(32), YT_I(2), YT_I(1), YT_I(4));
+    if (c1 == best) return launch(YT_I(64), YT_I(64), YT_I(2), YT_I(2), YT_I(4));
+    if (c2 == best) return launch(YT_I(128), YT_I(64), YT_I(2), YT_I(2), YT_I(3));
+    return launch(YT_I(128), YT_I(128), YT_I(2), YT_I(4), YT_I(4));
+#undef YT_I
+}
+
 }  // namespace
 
 int gemm_masked_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, const void* A, int64_t sa_b,
@@ -1164,4 +1250,97 @@ int gemm_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, c
                                 csc, alpha, beta, MaskDesc{YTHIP_MASK_NONE, nullptr, 0, 0, 0, 0.f}, s);
 }
 
+// How many parts k is cut into for a product too small for the chip (1: none). Such a
+// grid has at most one 64 x 32 tile per CU and each walks the whole k, one step of about
+// 280 ns after the other, whatever the number of rows (64 or 512 x 1024 x 3072: 11.8 and
+// 12.6 us). The parts run side by side as a batch of fp32 products, on larger tiles
+// where there are rows for them, and a second launch sums them.
+int gemm_splits(int m, int n, int k) {
+    const int64_t tiles = (int64_t)((m + 63) / 64) * ((n + 31) / 32);
+    if (m < 2 || n % 4 != 0 || tiles > 256) return 1;
+    for (int s = 8; s > 1; s >>= 1)
+        if (k % (64 * s) == 0 && k / s >= 384 && tiles * s <= 1024) return s;
+    return 1;
+}
+
+// The same where the sum is a launch of its own and not part of one that runs anyway:
+// only a long k over half the CUs or fewer pays for it. bf16, one launch / parts and
+// sum: 128 x 1024 x 3072 11.8 / 8.9 us, 64 x 1024 x 3072 11.8 / 7.2, 24 x 1024 x 2048 9.2 / 6.1,
+// 256 x 512 x 4096 14.9 / 9.9; not taken: 300 x 1024 x 3072 12.1 / 12.2, 512 x 1024 x 2048
+// 9.3 / 12.8, 64 x 4096 x 1024 5.9 / 7.3.
+int gemm_splits_alone(int m, int n, int k) {
+    const int64_t tiles = (int64_t)((m + 63) / 64) * ((n + 31) / 32);
+    return m > 16 && k >= 2048 && tiles <= 128 ? gemm_splits(m, n, k) : 1;
+}
+
 }  // namespace ythip
+
+using namespace ythip;
+
+extern "C" {
+
+__attribute__((visibility("default"))) int ythip_gemm_splits(int dtype, int m, int n, int k) {
+    if ((dtype != YTHIP_BF16 && dtype != YTHIP_F16) || m <= 0 || n <= 0 || k <= 0) return 1;
+    return gemm_splits(m, n, k);
+}
+
+__attribute__((visibility("default"))) size_t ythip_gemm_workspace_size(int dtype, int m, int n, int k) {
+    if ((dtype != YTHIP_BF16 && dtype != YTHIP_F16) || m <= 0 || n <= 0 || k <= 0) return 0;
+    const int s = gemm_splits_alone(m, n, k);
+    return s > 1 ? (size_t)s * m * n * sizeof(float) : 0;
+}
+
+__attribute__((visibility("default"))) int ythip_gemm_ws(int dtype_in, int dtype_out, int m, int n, int k, const void* A,
+                                                         int64_t rsa, int64_t csa, const void* B, int64_t rsb, int64_t csb,
+                                                         void* C, int64_t rsc, int64_t csc, float alpha, float beta,
+                                                         void* workspace, size_t ws_bytes, void* stream) {
+    const size_t need = ythip_gemm_workspace_size(dtype_in, m, n, k);
+    // rows that the DMA kernels take, and a C that the sum can write
+    const bool ok = need > 0 && alpha != 0.0f && A && B && C && workspace && csa == 1 && rsb == 1 && csc == 1 &&
+                    rsa % 8 == 0 && csb % 8 == 0 && aligned(A, 16) && aligned(B, 16) && aligned(workspace, 16) &&
+                    ws_bytes >= need &&
+                    (dtype_out == dtype_in || dtype_out == YTHIP_F32);
+    if (!ok)
+        return ythip_gemm(dtype_in, dtype_out, 1, m, n, k, A, 0, rsa, csa, B, 0, rsb, csb, C, 0, rsc, csc, alpha, beta,
+                          stream);
+    const int s = gemm_splits(m, n, k);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    float* parts = static_cast<float*>(workspace);
+    if (const int e = gemm_dispatch(dtype_in, YTHIP_F32, s, m, n, k / s, A, k / s, rsa, 1, B, k / s, 1, csb, parts,
+                                    (int64_t)m * n, n, 1, 1.0f, 0.0f, st))
+        return e;
+    const int64_t mn = (int64_t)m * n;
+    const dim3 grid((unsigned)((mn / 4 + 255) / 256));
+    auto sum = [&](auto to) {
+        using TO = decltype(to);
+        if (s == 8) splitk_reduce_kernel<TO, 8><<<grid, 256, 0, st>>>(parts, mn, n / 4, C, rsc, alpha, beta);
+        else if (s == 4) splitk_reduce_kernel<TO, 4><<<grid, 256, 0, st>>>(parts, mn, n / 4, C, rsc, alpha, beta);
+        else splitk_reduce_kernel<TO, 2><<<grid, 256, 0, st>>>(parts, mn, n / 4, C, rsc, alpha, beta);
+        return status_of(hipGetLastError());
+    };
+    if (dtype_out == YTHIP_F32) return sum(F32{});
+    return dtype_out == YTHIP_BF16 ? sum(BF16{}) : sum(F16{});
+}
+
+__attribute__((visibility("default"))) int ythip_gemm_swiglu(int dtype, int m, int inter, int k, const void* A, int64_t lda,
+                                                             const void* W, int64_t ldw, void* C, int64_t ldc,
+                                                             void* stream) {
+    const char* who = "ythip_gemm_swiglu";
+    if (m < 0 || inter < 0 || k < 0) return fail(YTHIP_EINVAL, "%s: negative size", who);
+    if (dtype != YTHIP_BF16 && dtype != YTHIP_F16) return fail(YTHIP_EUNSUPPORTED, "%s: 16-bit types only", who);
+    if (m == 0 || inter == 0) return 0;
+    if (!A || !W || !C) return fail(YTHIP_EINVAL, "%s: NULL pointer", who);
+    if (k == 0 || k % 8 || inter % 4 || lda % 8 || ldw % 8 || ldc % 4 || lda < k || ldw < k || ldc < inter ||
+        !aligned(A, 16) || !aligned(W, 16) || !aligned(C, 8) || (int64_t)m * lda * 2 >= (int64_t(1) << 31) ||
+        (int64_t)2 * inter * ldw * 2 >= (int64_t(1) << 31))
+        return fail(YTHIP_EUNSUPPORTED, "%s: 16-byte aligned rows below 2^31 bytes, k %% 8 == 0, inter %% 4 == 0", who);
+    GemmArgs g{};
+    g.A = A; g.B = W; g.C = C;
+    g.m = m; g.n = inter; g.k = k;
+    g.rsa = lda; g.rsb = 1; g.csb = ldw; g.rsc = ldc;
+    g.alpha = 1.0f;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    return dtype == YTHIP_BF16 ? swiglu_typed<BF16>(g, s) : swiglu_typed<F16>(g, s);
+}
+
+}  // extern "C"

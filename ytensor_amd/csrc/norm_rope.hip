@@ -249,7 +249,75 @@ __global__ __launch_bounds__(256) void rms_norm_reg_kernel(const void* x, int64_
     }
 }
 
+// x += the sum of `splits` fp32 products [splits][rows][n] of a projection whose k was
+// cut (ythip_gemm_splits), then (w given) y = the RMSNorm of x as rms_norm_reg_kernel
+// computes it. One launch in place of the sum, the residual add and the norm, and the
+// row is read once; bound by the partials' bytes (rows 512, n 1024, 4 parts: 14.7 MB).
+// SPLITS = 0: any count, summed in a loop; 2, 4, 8: every part's loads in flight at once.
+template <class TO, int J, int SPLITS>
+__global__ __launch_bounds__(256) void residual_rms_kernel(const float* __restrict__ parts, int splits, float* x, int64_t ldx,
+                                                           const float* w, float eps, void* y, int64_t ldy, int n) {
+    const int64_t row = blockIdx.x, rows = gridDim.x;
+    float* xr = x + row * ldx;
+    float v[J], wv[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) v[j] = xr[min((int)threadIdx.x + 256 * j, n - 1)];
+#pragma unroll
+    for (int j = 0; j < J; ++j) wv[j] = w != nullptr ? w[min((int)threadIdx.x + 256 * j, n - 1)] : 0.f;
+    if constexpr (SPLITS > 0) {
+        float p[SPLITS][J];
+#pragma unroll
+        for (int s = 0; s < SPLITS; ++s)
+#pragma unroll
+            for (int j = 0; j < J; ++j) p[s][j] = parts[(s * rows + row) * n + min((int)threadIdx.x + 256 * j, n - 1)];
+#pragma unroll
+        for (int s = 0; s < SPLITS; ++s)
+#pragma unroll
+            for (int j = 0; j < J; ++j) v[j] += p[s][j];
+    } else {
+        for (int s = 0; s < splits; ++s)
+#pragma unroll
+            for (int j = 0; j < J; ++j) v[j] += parts[(s * rows + row) * n + min((int)threadIdx.x + 256 * j, n - 1)];
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+        if ((int)threadIdx.x + 256 * j < n) {
+            xr[threadIdx.x + 256 * j] = v[j];
+            ss = fmaf(v[j], v[j], ss);
+        }
+    if (w == nullptr) return;
+    __shared__ float part[4];
+    ss = wave_sum(ss);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    const float tot = (part[0] + part[1]) + (part[2] + part[3]);
+    const float den = sqrtf(tot / (float)n + eps);
+    auto* yr = static_cast<typename TO::raw*>(y) + row * ldy;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        const int i = threadIdx.x + 256 * j;
+        if (i < n) store_from_f32<TO>(yr, i, (v[j] / den) * wv[j]);
+    }
+}
+
 namespace {
+
+template <class TO>
+hipError_t launch_residual(int rows, int n, int splits, const float* parts, float* x, int64_t ldx, const float* w, float eps,
+                           void* y, int64_t ldy, hipStream_t s) {
+    auto go = [&](auto j) {
+        constexpr int J = decltype(j)::value;
+        if (splits == 8 && J <= 8) residual_rms_kernel<TO, J, J <= 8 ? 8 : 0><<<rows, 256, 0, s>>>(parts, splits, x, ldx, w, eps, y, ldy, n);
+        else if (splits == 4) residual_rms_kernel<TO, J, 4><<<rows, 256, 0, s>>>(parts, splits, x, ldx, w, eps, y, ldy, n);
+        else if (splits == 2) residual_rms_kernel<TO, J, 2><<<rows, 256, 0, s>>>(parts, splits, x, ldx, w, eps, y, ldy, n);
+        else residual_rms_kernel<TO, J, 0><<<rows, 256, 0, s>>>(parts, splits, x, ldx, w, eps, y, ldy, n);
+    };
+    if (n <= 1024) go(std::integral_constant<int, 4>{});
+    else if (n <= 2048) go(std::integral_constant<int, 8>{});
+    else go(std::integral_constant<int, 16>{});
+    return hipGetLastError();
+}
 
 template <class T>
 hipError_t launch_norm_rope(const NormRopeArgs& a, int d, hipStream_t s) {
@@ -362,6 +430,26 @@ __attribute__((visibility("default"))) int ythip_rms_norm(int dtype_in, int dtyp
     if (dtype_in == YTHIP_F16 && dtype_out == YTHIP_F32) YTHIP_RMS(F16, F32);
 #undef YTHIP_RMS
     return fail(YTHIP_EINVAL, "ythip_rms_norm: invalid dtype pair %d/%d", dtype_in, dtype_out);
+}
+
+__attribute__((visibility("default"))) int ythip_residual_rms_norm(int dtype_out, int rows, int n, int splits,
+                                                                   const float* partials, float* x, int64_t ld_x,
+                                                                   const float* w, float eps, void* y, int64_t ld_y,
+                                                                   void* stream) {
+    const char* who = "ythip_residual_rms_norm";
+    if (rows < 0 || n < 0 || splits < 0) return fail(YTHIP_EINVAL, "%s: negative size", who);
+    if (rows == 0 || n == 0) return 0;
+    if (x == nullptr || (splits > 0 && partials == nullptr) || (w != nullptr && y == nullptr))
+        return fail(YTHIP_EINVAL, "%s: NULL pointer", who);
+    if (ld_x < n || (w != nullptr && ld_y < n)) return fail(YTHIP_EINVAL, "%s: leading dimension smaller than n", who);
+    if (n > 4096) return fail(YTHIP_EUNSUPPORTED, "%s: n = %d (at most 4096)", who, n);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    switch (dtype_out) {
+        case YTHIP_F32: return status_of(launch_residual<F32>(rows, n, splits, partials, x, ld_x, w, eps, y, ld_y, s));
+        case YTHIP_BF16: return status_of(launch_residual<BF16>(rows, n, splits, partials, x, ld_x, w, eps, y, ld_y, s));
+        case YTHIP_F16: return status_of(launch_residual<F16>(rows, n, splits, partials, x, ld_x, w, eps, y, ld_y, s));
+        default: return fail(YTHIP_EINVAL, "%s: invalid dtype %d", who, dtype_out);
+    }
 }
 
 __attribute__((visibility("default"))) int ythip_rms_norm_strided(int dtype_in, int dtype_out, int rows, int n,

@@ -19,6 +19,7 @@ done here, mirroring src/function/ops.inl:123-128, 382-387).
 """
 from __future__ import annotations
 
+import functools
 import itertools
 import math
 
@@ -37,8 +38,15 @@ def _code(t: torch.Tensor) -> int:
         raise ValueError(f"unsupported dtype {t.dtype}; the type set is float32/float16/bfloat16") from None
 
 
+# The current stream's handle without building a torch.cuda.Stream around it (that is
+# 1 to 2 us of a call); the public way where this torch has no such function.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def _dev(*ts: torch.Tensor) -> None:
@@ -82,6 +90,40 @@ def gemm(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor, alpha: float = 1.0
     return out
 
 
+def gemm_splits(dtype: torch.dtype, m: int, n: int, k: int) -> int:
+    """Parts that a 16-bit product of a size too small for the chip is cut into along
+    k (1: none), see ythip_gemm_splits."""
+    return _lib.lib().ythip_gemm_splits(_DT[dtype], m, n, k)
+
+
+@functools.lru_cache(maxsize=1024)
+def _gemm_workspace(code: int, m: int, n: int, k: int) -> int:
+    return _lib.lib().ythip_gemm_workspace_size(code, m, n, k)
+
+
+def _gemm2(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
+    """a [m, k] @ b [k, n] of any strides into a new [m, n]; sizes already checked.
+    The whole host path of a small product: straight to the C call."""
+    _dev(a, b)
+    if a.dtype != b.dtype:
+        raise ValueError("a and b must share a dtype")
+    ca = _code(a)
+    (m, k), n = a.shape, b.shape[1]
+    out = torch.empty((m, n), dtype=out_dtype, device=a.device)
+    (rsa, csa), (rsb, csb) = a.stride(), b.stride()
+    need = _gemm_workspace(ca, m, n, k) if rsb == 1 and m > 16 else 0
+    if need:
+        ws = torch.empty(need, dtype=torch.uint8, device=a.device)
+        check(_lib.lib().ythip_gemm_ws(ca, _code(out), m, n, k, a.data_ptr(), rsa, csa, b.data_ptr(), rsb, csb,
+                                       out.data_ptr(), n, 1, 1.0, 0.0, ws.data_ptr(), need, _stream()), "ythip_gemm_ws")
+        return out
+    st = _lib.lib().ythip_gemm(ca, _code(out), 1, m, n, k, a.data_ptr(), 0, rsa, csa, b.data_ptr(), 0, rsb, csb,
+                               out.data_ptr(), 0, n, 1, 1.0, 0.0, _stream())
+    if st:
+        check(st, "ythip_gemm")
+    return out
+
+
 def matmul(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """YTensor::matmul (src/ytensor_math.inl:284-316, 954-1051): a [..., M, K] @
     b [..., K, N] over the last two dims, the leading dims broadcast against each
@@ -94,6 +136,8 @@ def matmul(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype | None = Non
     kb, n = b.shape[-2], b.shape[-1]
     if kb != k:
         raise ValueError(f"matmul: inner dimensions differ ({k} vs {kb})")
+    if a.dim() == 2 and b.dim() == 2:
+        return _gemm2(a, b, out_dtype)
     try:
         lead = tuple(torch.broadcast_shapes(a.shape[:-2], b.shape[:-2]))
     except RuntimeError:
@@ -105,10 +149,7 @@ def matmul(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype | None = Non
         # Batch-flatten fast path (src/ytensor_math.inl:960-1017): a's rows are
         # uniform, so [..., M, K] is one [prod(lead) * M, K] product.
         if a.dim() > 2 and a.is_contiguous() and tuple(a.shape[:-2]) == lead:
-            a2 = a.reshape(-1, k)
-            out = torch.empty((a2.shape[0], n), dtype=out_dtype, device=a.device)
-            gemm(a2, b2, out)
-            return out.reshape(*lead, m, n)
+            return _gemm2(a.reshape(-1, k), b2, out_dtype).reshape(*lead, m, n)
     out = torch.empty((*lead, m, n), dtype=out_dtype, device=a.device)
     if not lead:
         gemm(a, b, out)
@@ -136,16 +177,15 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
         if bias.dtype != out_dtype:
             raise ValueError(f"linear: bias has dtype {bias.dtype}, the output {out_dtype}")
         _dev(bias)
-    x2 = x.reshape(-1, k)
-    out = torch.empty((x2.shape[0], weight.shape[0]), dtype=out_dtype, device=x.device)
-    gemm(x2, weight.t(), out)
+    flat = x.dim() == 2
+    out = _gemm2(x if flat else x.reshape(-1, k), weight.t(), out_dtype)
     if bias is not None:
         # ops.inl:93-104: the product is rounded to the output type first, then
         # the bias is added in that type
         b = bias.contiguous()
         check(_lib.lib().ythip_add_bias(_code(out), out.shape[0], out.shape[1], out.data_ptr(), out.stride(0),
                                         b.data_ptr(), _stream()), "ythip_add_bias")
-    return out.reshape(*x.shape[:-1], weight.shape[0])
+    return out if flat else out.reshape(*x.shape[:-1], weight.shape[0])
 
 
 # ---------------------------------------------------------------------------
@@ -716,6 +756,53 @@ def gemv_swiglu(a: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, prolo
                                        gate_up.data_ptr(), gate_up.stride(0), o2.data_ptr(), o2.stride(0),
                                        _stream()), "ythip_gemv_swiglu")
     return out
+
+
+def gemm_swiglu(a: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+    """gemv_swiglu's prologue-free form for any number of rows: out [m, I] =
+    silu(a @ gate.T) * (a @ up.T), gate_up = [gate | up] ([2I, K]), both products rounded
+    to the type first; the bits of gemm into [m, 2I] followed by silu_mul."""
+    _dev(a, gate_up, out)
+    (m, k), n2 = a.shape, gate_up.shape[0]
+    if n2 % 2 or gate_up.shape[1] != k or tuple(out.shape) != (m, n2 // 2):
+        raise ValueError(f"gemm_swiglu: a {tuple(a.shape)}, gate_up {tuple(gate_up.shape)}, out {tuple(out.shape)}")
+    if not (a.dtype == gate_up.dtype == out.dtype) or not (a.stride(1) == gate_up.stride(1) == out.stride(1) == 1):
+        raise ValueError("gemm_swiglu needs one dtype and unit column strides")
+    check(_lib.lib().ythip_gemm_swiglu(_code(a), m, n2 // 2, k, a.data_ptr(), a.stride(0), gate_up.data_ptr(),
+                                       gate_up.stride(0), out.data_ptr(), out.stride(0), _stream()), "ythip_gemm_swiglu")
+    return out
+
+
+def gemm_parts(a: torch.Tensor, weight: torch.Tensor, parts: torch.Tensor) -> torch.Tensor:
+    """a [m, k] @ weight[n, k].T with k cut into parts.shape[0] pieces: parts [s, m, n]
+    (fp32) takes the product of each, for residual_rms_norm to sum."""
+    s, (m, k), n = parts.shape[0], a.shape, weight.shape[0]
+    if k % s:
+        raise ValueError(f"gemm_parts: k = {k} is not a multiple of {s} parts")
+    gemm(a.unflatten(1, (s, k // s)).transpose(0, 1), weight.unflatten(1, (s, k // s)).permute(1, 2, 0), parts)
+    return parts
+
+
+def residual_rms_norm(x: torch.Tensor, parts: torch.Tensor, weight: torch.Tensor | None = None, eps: float = 1e-6,
+                      out: torch.Tensor | None = None) -> torch.Tensor:
+    """x [m, n] (fp32, in place) += parts.sum(0) (fp32 [s, m, n]); with weight (fp32 [n]),
+    out = rms_norm(x, weight, eps) in out's dtype. n <= 4096."""
+    _dev(x, parts, weight, out)
+    m, n = x.shape
+    if x.dtype != torch.float32 or parts.dtype != torch.float32 or x.stride(1) != 1:
+        raise ValueError("residual_rms_norm: x and parts are float32, x with unit column stride")
+    if tuple(parts.shape[1:]) != (m, n) or not parts.is_contiguous():
+        raise ValueError(f"residual_rms_norm: parts must be contiguous [s, {m}, {n}]")
+    if (weight is None) != (out is None):
+        raise ValueError("residual_rms_norm: weight and out go together")
+    if weight is not None and (weight.dtype != torch.float32 or not weight.is_contiguous() or weight.numel() != n
+                               or tuple(out.shape) != (m, n) or out.stride(1) != 1):
+        raise ValueError("residual_rms_norm: weight is float32 [n], out [m, n] with unit column stride")
+    check(_lib.lib().ythip_residual_rms_norm(
+        _lib.F32 if out is None else _code(out), m, n, parts.shape[0], parts.data_ptr(), x.data_ptr(), x.stride(0),
+        None if weight is None else weight.data_ptr(), float(eps), None if out is None else out.data_ptr(),
+        0 if out is None else out.stride(0), _stream()), "ythip_residual_rms_norm")
+    return x
 
 
 def argmax_finish(parts: torch.Tensor, n_parts: int, token: torch.Tensor, history: torch.Tensor | None = None,
