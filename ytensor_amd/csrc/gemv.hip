@@ -73,6 +73,7 @@ struct GemvPrologue {
     static constexpr bool EW = PRO == 1 || PRO == 2;  // elementwise prologues
     static constexpr int PJ = PRO == 2 ? 8 : 4;        // elements per thread held in registers
     static constexpr int MS = 8;                       // merge: splits held in registers
+    static constexpr int SPEC = 2;                     // ... and loaded before it is known how many hold keys
     float p0[EW ? PJ : 1], p1[EW ? PJ : 1];
     float xr[PRO == 1 ? 4 : 1];                        // RMSNorm: first reduction group of row 0
     float opre[PRO == 3 ? 2 : 1][PRO == 3 ? MS : 1];   // merge: o of this thread's 2 elements
@@ -117,21 +118,28 @@ struct GemvPrologue {
         }
         if constexpr (PRO == 3) {
             const int S = a.splits, stride = a.hd + 2;
-            // the split kernel's partition (decode_used); the loads below do not wait for it
+            // The split kernel's partition (decode_used). The first SPEC splits are loaded
+            // without waiting for it, the others only where they hold keys: a short
+            // context in a large ring reads a quarter of the bytes (each of the 64
+            // workgroups reads all of them). Qwen3-0.6B decode, 4096-row ring: up to 256 keys
+            // 740 -> 720 us a token, 512 keys 753 -> 749, 1000 keys (all 8 in use) 764 -> 767.
             used = a.dstate != nullptr ? decode_used(max(0, min(a.dstate[YTHIP_ST_KV_LEN], a.max_ctx)), S) : S;
+            const float* src[2];
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int e = tid + j * NT;
-                const float* src = merge_src(a, bz, e < total ? e : 0);
-#pragma unroll
-                for (int q = 0; q < MS; ++q) opre[j][q] = (e < total && q < S) ? src[q * stride] : 0.f;
-            }
+            for (int j = 0; j < 2; ++j) src[j] = merge_src(a, bz, tid + j * NT < total ? tid + j * NT : 0);
             const bool owner = tid < a.m * a.hq;
             const float* msrc = merge_msrc(a, bz, owner ? tid : 0);
+            auto take = [&](int q, bool on) {
 #pragma unroll
-            for (int q = 0; q < MS; ++q) {
-                mreg[q] = (owner && q < S) ? msrc[q * stride] : -INFINITY;
-                lreg[q] = (owner && q < S) ? msrc[q * stride + 1] : 0.f;
+                for (int j = 0; j < 2; ++j) opre[j][q] = (on && tid + j * NT < total) ? src[j][q * stride] : 0.f;
+                mreg[q] = (on && owner) ? msrc[q * stride] : -INFINITY;
+                lreg[q] = (on && owner) ? msrc[q * stride + 1] : 0.f;
+            };
+#pragma unroll
+            for (int q = 0; q < SPEC; ++q) take(q, q < S);
+            if (used > SPEC) {
+#pragma unroll
+                for (int q = SPEC; q < MS; ++q) take(q, q < used);
             }
         }
     }
@@ -576,12 +584,28 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_row_kernel(GemvArgs a) {
 // state update as argmax_step_kernel.
 __global__ __launch_bounds__(1024) void argmax_finish_kernel(const float* parts, int n_parts, int32_t* token,
                                                              int32_t* history, int32_t* state) {
+    // One workgroup, so all of its time is latency: every pair of a thread and the
+    // decode-state record are in flight at once (the 151936-token head's 9496 pairs
+    // and then the record's fields one after the other: 6.3 us).
+    int32_t st[YTHIP_ST_WORDS];
+    if (threadIdx.x == 0 && state != nullptr)
+#pragma unroll
+        for (int f = 0; f < YTHIP_ST_WORDS; ++f) st[f] = state[f];
     float best = -INFINITY;
     int idx = 0x7fffffff;
-    for (int i = threadIdx.x; i < n_parts; i += 1024) {
-        const float v = parts[2 * i];
-        const int id = __float_as_int(parts[2 * i + 1]);
-        if (v > best || (v == best && id < idx)) { best = v; idx = id; }
+    constexpr int UNR = 10;
+    for (int i0 = threadIdx.x; i0 < n_parts; i0 += 1024 * UNR) {
+        float v[UNR];
+        int id[UNR];
+#pragma unroll
+        for (int u = 0; u < UNR; ++u) {
+            const int i = min(i0 + 1024 * u, n_parts - 1);  // past the end: the last pair again
+            v[u] = parts[2 * (int64_t)i];
+            id[u] = __float_as_int(parts[2 * (int64_t)i + 1]);
+        }
+#pragma unroll
+        for (int u = 0; u < UNR; ++u)
+            if (v[u] > best || (v[u] == best && id[u] < idx)) { best = v[u]; idx = id[u]; }
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
@@ -601,7 +625,11 @@ __global__ __launch_bounds__(1024) void argmax_finish_kernel(const float* parts,
             if (sb[w] > b || (sb[w] == b && si[w] < id)) { b = sb[w]; id = si[w]; }
         if (id == 0x7fffffff) id = 0;  // all NaN / empty: token 0
         token[0] = id;
-        if (state != nullptr) decode_state_advance(state, history, id);
+        if (state != nullptr) {
+            decode_state_advance(st, history, id);
+            for (int f : {YTHIP_ST_GENERATED, YTHIP_ST_ROPE_POS, YTHIP_ST_KV_LEN, YTHIP_ST_SLOT, YTHIP_ST_TOTAL, YTHIP_ST_ERROR})
+                state[f] = st[f];
+        }
     }
 }
 
