@@ -1,5 +1,5 @@
 // attention.hip — attention forward for gfx950: MFMA flash-attention prefill,
-// split-context decode, and an any-layout row-wise kernel.
+// split-context decode (other layouts: attention_any.hip).
 //
 // Reference semantics (src/kernel/avx2/flash_attention.inl):
 //   prefill 274-443: blockwise online softmax over key tiles, masked entries
@@ -313,15 +313,15 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
                 dma16_soff(vbase, vbo[i], lv + (uint32_t)(i * THREADS) * 16u);
             }
         } else {
-            // a tail stage's K rows past the end re-read the last key (never used),
-            // its V rows read zeros
+            // a tail stage's rows past the end re-read the last key (never used; MODE 4,
+            // where 0 . V counts: its V rows read zeros)
 #pragma unroll
             for (int i = 0; i < PT; ++i) {
                 const int row = slot_row(i);
                 const int sh = k0 + SBKV <= a.Skv ? 0 : min(k0 + row, a.Skv - 1) - k0 - row;
                 dma16_async(kbase + koff(i) + sh * (int)a.ks2, &dK[i * THREADS + wave * 64]);
                 const raw* vp = vbase + voff(i) + sh * (int)a.vs2;
-                if (k0 + row >= a.Skv) vp = reinterpret_cast<const raw*>(dma_zero);
+                if (MODE == 4 && k0 + row >= a.Skv) vp = reinterpret_cast<const raw*>(dma_zero);
                 dma16_async(vp, &dV[i * THREADS + wave * 64]);
             }
         }
@@ -1427,12 +1427,12 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_f32(AttnArgs a) {
         }
 #pragma unroll
         for (int i = 0; i < PT; ++i) {
-            // K rows past the end re-read the last key (masked, never used), V rows zeros
+            // rows past the end re-read the last key (masked, never used; MODE 4: V rows zeros)
             const int row = slot_row(i);
             const int sh = min(k0 + row, a.Skv - 1) - k0 - row;
             dma16_async(kbase + koff(i) + sh * (int)a.ks2, &dK[i * 64 * NW + wave * 64]);
             const float* vp = vbase + voff(i) + sh * (int)a.vs2;
-            if (k0 + row >= a.Skv) vp = reinterpret_cast<const float*>(dma_zero);
+            if (MODE == 4 && k0 + row >= a.Skv) vp = reinterpret_cast<const float*>(dma_zero);
             dma16_async(vp, &dV[i * 64 * NW + wave * 64]);
         }
     };
