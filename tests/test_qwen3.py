@@ -314,3 +314,25 @@ def test_qwen3_fused_decode_equals_unfused(orc):
     b._decode_step()
     torch.cuda.synchronize()
     assert torch.equal(a.token, b.token)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kw,fused", [(dict(hidden=260), False), (dict(hidden=260), True), (dict(inter=514), False)],
+                         ids=["hidden-260-unfused", "hidden-260-prompt", "inter-514"])
+def test_qwen3_prompt_of_sizes_without_fused_kernels(orc, kw, fused):
+    """Rows of hidden or inter values that are no whole 16-byte (8-byte) chunks: neither the
+    SwiGLU product nor the fused head takes them, the prompt runs launch by launch."""
+    import torch
+
+    from ytensor_amd.qwen3 import Qwen3, Qwen3Config
+    kw = dict(SMALL, **kw)
+    cfg_o = oracle.Qwen3Config(**kw)
+    W = _small_weights(orc, cfg_o)
+    pr = oracle.qwen3_prompt(cfg_o, 37, seed=4)
+    _, _, lo = orc.qwen3_generate(cfg_o, W, pr, 1)
+    m = Qwen3(Qwen3Config(**kw), W, max_ctx=64, max_prompt=64, fused=fused)
+    m.prefill(pr)
+    torch.cuda.synchronize()
+    lg = m.logits.float().cpu().numpy()[0]
+    # bf16 activations through SMALL's layers, as in test_qwen3_small_gpu_tokens_and_logits
+    assert np.abs(lg - lo).max() / np.abs(lo).max() <= 2e-2

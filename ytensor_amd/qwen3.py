@@ -329,7 +329,7 @@ class Qwen3:
             ops.gemm(self.act[:S], L["down"].t(), x, beta=1.0)        # x += act . Wdown^T
             return
         self._add_norm(x, self.attn[:S], L["o"], L["n2"], h)          # x += attn . Wo^T; h = norm(x)
-        if S > 16:  # 512 rows: 13.9 us, 15.3 + 5.1 as two launches (fewer rows take the GEMV)
+        if S > 16 and self._swiglu_fits(S):  # 512 rows: 13.9 us, 15.3 + 5.1 as two launches (fewer rows take the GEMV)
             ops.gemm_swiglu(h, L["gu"], self.act[:S])
         else:
             ops.gemm(h, L["gu"].t(), self.gu[:S])
@@ -371,8 +371,16 @@ class Qwen3:
         ops.gemv_swiglu(x, L["gu"], self.act[:1], "rmsnorm", L["n2"], cfg.eps)    # act = swiglu(norm(x) . Wgu^T)
         ops.gemv_fused(self.act[:1], L["down"], x, beta=1.0)                      # x += act . Wdown^T
 
+    def _swiglu_fits(self, S: int) -> bool:
+        """Sizes that gemm_swiglu takes: rows of whole 16-byte chunks, operands below 2^31 bytes."""
+        H, I = self.cfg.hidden, self.cfg.inter
+        return H % 8 == 0 and I % 4 == 0 and 2 * H * max(S, 2 * I) < 1 << 31
+
     def _head(self, S: int) -> None:
-        if self.fused:
+        H = self.cfg.hidden
+        # a prompt's last row takes the fused head where the GEMV takes its sizes (whole
+        # 16-byte chunks, the normed row in 64 KiB); a decode step has no other
+        if self.fused and (S == 1 or (H % 8 == 0 and 2 * H <= 1 << 16)):
             # final norm + tied LM head + per-tile argmax in one launch, then the pick
             # (also a prompt's last row: 54 us, against 104 with the argmax on its own)
             ops.gemv_fused(self.x[S - 1:S], self.lm_head, self.logits, "rmsnorm", self.fnorm, self.cfg.eps,
