@@ -177,14 +177,15 @@ int ythip_attn_prefill_ws(int dtype, int B, int Hq, int Hkv, int q_len, int kv_l
 
 /*
  * Attention forward with the MATH backend (scaledDotProductAttention with
- * sdpaBackend::MATH, src/function/ops.inl:388-418, 474-490): the score matrix is
- * materialised,
+ * sdpaBackend::MATH, src/function/ops.inl:388-418, 474-490):
  *   S = masked_matmul(Q, K^T, mask, -1e9) * scale + bias,  P = softmax_(S, -1),
  *   O = P . V,  rows with no visible key -> 0 (ops.inl:18-40),
  * with S in fp32 and P in the input type (the reference's score tensor has the
- * input type). Same tensor and mask arguments as ythip_attn_prefill, except that
+ * input type); in one launch without S and P in memory where the layout is one of the
+ * flash kernels' (d == dv 64 or 128, 16-byte aligned rows). Same tensor and mask arguments as ythip_attn_prefill, except that
  * every stride may be any value (transposed K / V included). workspace: device
- * scratch of ythip_attn_math_workspace_size(dtype, B, Hq, q_len, kv_len) bytes.
+ * scratch of ythip_attn_math_workspace_size(dtype, B, Hq, q_len, kv_len) bytes,
+ * required for every layout.
  */
 size_t ythip_attn_math_workspace_size(int dtype, int B, int Hq, int q_len, int kv_len);
 int ythip_attn_math(int dtype, int B, int Hq, int Hkv, int q_len, int kv_len, int d, int dv,
@@ -203,8 +204,8 @@ int ythip_attn_math(int dtype, int B, int Hq, int Hkv, int q_len, int kv_len, in
  *   C = alpha * A.B + beta * C   (k == 0 or alpha == 0: C *= beta, 0 for beta == 0)
  * and elsewhere C is left unchanged, or set to masked_value when fill_masked != 0
  * (masked_matmul's fill). mask_kind / mask / mask_ld as for attention, with the
- * causal offset n - m. workspace: ythip_gemm_masked_workspace_size(batch, m, n)
- * bytes of device scratch (the fp32 product).
+ * causal offset n - m. One launch; workspace of ythip_gemm_masked_workspace_size(batch,
+ * m, n) bytes is still required where a product is computed, and not written.
  */
 size_t ythip_gemm_masked_workspace_size(int batch, int m, int n);
 int ythip_gemm_masked(int dtype_in, int dtype_out, int batch, int m, int n, int k,
