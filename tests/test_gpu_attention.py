@@ -912,3 +912,24 @@ def test_prefill_any_layout_non_finite_values(yt):
         assert torch.equal(torch.isfinite(out[h]), finite)
         assert out[h, 1, 5] == float("inf") and out[h, 2, 6] == float("inf") and out[h, 3, 6].isnan() and out[h, 4, 7].isnan()
         assert torch.equal(out[h, 0], v[0, h, 10])
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("Skv", [1, 2, 3, 4])
+def test_prefill_any_layout_smallest_operands(yt, Skv, masked, dtype):
+    """One kv head, one dimension, fewer keys than a mask word: K is as small as 2
+    bytes and ends its allocation, and nothing but K, V and the mask is read. With
+    d = 1 and V = key index + 1 the softmax is checked against float64 (bound: the
+    rounding of the result and 1e-6 of the sums)."""
+    td = TORCH_DT[dtype]
+    q = torch.arange(1, 4, device="cuda", dtype=torch.float32).view(1, 1, 3, 1).to(td)
+    k = (0.5 * torch.arange(Skv, device="cuda")).view(1, 1, Skv, 1).to(td)
+    v = (torch.arange(Skv, device="cuda") + 1.0).view(1, 1, Skv, 1).to(td)
+    vis = torch.ones(3, Skv, dtype=torch.bool, device="cuda")
+    if masked:
+        vis[0, 0] = vis[2, Skv - 1] = False
+    out = yt.scaled_dot_product_attention(q, k, v, 0.0, mask=vis if masked else None)
+    want = _sdpa64(q[0], k[0], v[0], 1.0, vis, None)
+    ulp = {"f32": 2.0 ** -22, "bf16": 2.0 ** -8, "f16": 2.0 ** -11}[dtype]
+    assert ((out[0].double() - want).abs() <= (1e-6 + ulp) * Skv).all()

@@ -28,6 +28,10 @@
 
 namespace ythip {
 
+// What a lane reads where no mask word is (no mask, or fewer keys than four): K may
+// be smaller than the word.
+static __device__ const uint32_t no_mask_word = 0x01010101u;
+
 // Four elements as they were loaded: consecutive ones in one load (PIECE), or one
 // by one at a stride. Converted only where they are used, so that a load in flight
 // is not waited for.
@@ -109,9 +113,10 @@ __global__ __launch_bounds__(64 * W) void attn_any_kernel(AttnArgs a) {
     const int per = (nblk + W - 1) / W, b0 = wave * per, n = min(max(nblk - b0, 0), per);
     const int turn = n > 0 ? (int)(blockIdx.x % (unsigned)n) : 0;
     // the mask word of four keys is read where it fits; without a mask, or with
-    // fewer keys than four, anything readable stands in for it
+    // fewer keys than four, a constant stands in for it
     const bool words = a.mask != nullptr && a.Skv >= 4;
-    const uint8_t* mrow = words ? a.mask + (int64_t)qr * a.mask_ld : static_cast<const uint8_t*>(a.K);
+    const uint8_t* mrow =
+        words ? a.mask + (int64_t)qr * a.mask_ld : reinterpret_cast<const uint8_t*>(&no_mask_word);
 
     // One block's operands. The next block's K is loaded as soon as the scores have
     // used this one's, its V after the output product: each load has the other
