@@ -933,3 +933,31 @@ def test_prefill_any_layout_smallest_operands(yt, Skv, masked, dtype):
     want = _sdpa64(q[0], k[0], v[0], 1.0, vis, None)
     ulp = {"f32": 2.0 ** -22, "bf16": 2.0 ** -8, "f16": 2.0 ** -11}[dtype]
     assert ((out[0].double() - want).abs() <= (1e-6 + ulp) * Skv).all()
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("layout", ["k_t", "odd", "aligned_f32"])
+def test_prefill_non_finite_scores(yt, layout, bad):
+    """A row with a NaN or +inf among its visible scores is zero, in the any-layout
+    kernel as in the aligned fp32 one; the other rows are those of finite inputs (the
+    score's key weighs nothing in them: bound 1e-5 of the values' size)."""
+    g = torch.Generator(device="cuda").manual_seed(9)
+    Sq, Skv, D = 40, 300, 64
+    q = torch.rand(1, 2, Sq, D, device="cuda", generator=g) + 0.5  # positive, so that inf . q = inf
+    if layout == "k_t":
+        k = torch.randn(1, 2, D, Skv, device="cuda", generator=g).transpose(-1, -2)
+    else:
+        pad = 1 if layout == "odd" else 0
+        k = torch.randn(1, 2, Skv, D + pad, device="cuda", generator=g)[..., pad:]
+    v = torch.randn(1, 2, Skv, D, device="cuda", generator=g)
+    vis = torch.rand(Sq, Skv, device="cuda", generator=g) < 0.5
+    key = 130
+    vis[:, key] = torch.arange(Sq, device="cuda") % 3 == 0
+    clean = vis.clone()
+    clean[:, key] = False
+    want = _sdpa64(q[0], k[0], v[0], 1.0 / math.sqrt(D), clean, None)
+    want[:, vis[:, key]] = 0.0
+    k[0, :, key, 5] = bad
+    out = yt.scaled_dot_product_attention(q, k, v, 0.0, mask=vis)[0].double()
+    assert torch.equal(out[:, vis[:, key]], want[:, vis[:, key]])
+    assert ((out - want).abs() <= 1e-5 * float(v.abs().max())).all()

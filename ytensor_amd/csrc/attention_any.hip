@@ -342,6 +342,7 @@ __global__ __launch_bounds__(64 * W) void attn_any_kernel(AttnArgs a) {
         L = fmaf(sl[w][r], wt[w], L);
     }
     if (qrow >= a.Sq) return;
+    // a row that sees no key, or whose scores hold a NaN or +inf (L is NaN), is zero
     const float inv = L > 0.f ? 1.0f / L : 0.f;
     const int64_t oo = b * a.os0 + h * a.os1 + (int64_t)qrow * a.os2;
     for (int t = wave; t < NB; t += W) {
@@ -351,7 +352,7 @@ __global__ __launch_bounds__(64 * W) void attn_any_kernel(AttnArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int d = 16 * t + 4 * g + i;
-            if (d < a.Dv) store_from_f32<T>(a.O, oo + d * a.os3, L != 0.f ? acc[i] * inv : 0.f);
+            if (d < a.Dv) store_from_f32<T>(a.O, oo + d * a.os3, L > 0.f ? acc[i] * inv : 0.f);
         }
     }
 }
