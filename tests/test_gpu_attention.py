@@ -961,3 +961,23 @@ def test_prefill_non_finite_scores(yt, layout, bad):
     out = yt.scaled_dot_product_attention(q, k, v, 0.0, mask=vis)[0].double()
     assert torch.equal(out[:, vis[:, key]], want[:, vis[:, key]])
     assert ((out - want).abs() <= 1e-5 * float(v.abs().max())).all()
+
+
+@pytest.mark.parametrize("layout", ["aligned_bias", "k_t", "d80"])
+@pytest.mark.parametrize("Skv", [16385, 20011])
+def test_prefill_any_layout_long_keys(yt, Skv, layout):
+    """The any-layout kernel streams its keys, so their number has no limit: fp32 with a
+    diagonal mask and a bias in the aligned layout, a transposed K, a head dim of 80.
+    Bound: 32-bit sums (1e-5 of the values' size)."""
+    g = torch.Generator(device="cuda").manual_seed(Skv)
+    Sq, D = 5, 80 if layout == "d80" else 64
+    q = torch.randn(1, 2, Sq, D, device="cuda", generator=g)
+    k = torch.randn(1, 1, Skv, D, device="cuda", generator=g)
+    v = torch.randn(1, 1, Skv, D, device="cuda", generator=g)
+    bias = torch.randn(Sq, Skv, device="cuda", generator=g) if layout == "aligned_bias" else None
+    off = Skv - 40
+    kk = k.transpose(-1, -2).contiguous().transpose(-1, -2) if layout == "k_t" else k
+    out = yt.scaled_dot_product_attention(q, kk, v, 0.0, mask=("diag", off), bias=bias)
+    vis = torch.arange(Skv, device="cuda")[None, :] <= torch.arange(Sq, device="cuda")[:, None] + off
+    want = _sdpa64(q[0], k[0], v[0], 1.0 / math.sqrt(D), vis, bias)
+    assert ((out[0].double() - want).abs() <= 1e-5 * float(v.abs().max())).all()

@@ -1300,10 +1300,6 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pingpong(AttnArgs a) {
     }
 }
 
-// Layouts the MFMA kernels do not take (attention_any.hip) are limited to this
-// many keys.
-constexpr int ANY_MAX = 16384;
-
 // ---------------------------------------------------------------------------
 // fp32 prefill on the matrix cores. The reference's flash backend is fp32-only
 // (src/function/ops.inl:119-121; _flashAttentionImpl, src/kernel/avx2/
@@ -2357,8 +2353,6 @@ int prefill_typed(AttnArgs a, hipStream_t s) {
             return status_of(launch_prefill_f32<64>(a, fmode, s));
         }
     }
-    if (a.Skv > ANY_MAX)
-        return fail(YTHIP_EUNSUPPORTED, "ythip_attn_prefill: this layout is limited to kv_len <= %d", ANY_MAX);
     return status_of(attn_any(T::code, a, s));
 }
 
