@@ -349,3 +349,22 @@ def test_gemm_masked_layouts(yt, dev, m, n, k, layout, dt):
             assert not off.any(), (mask if isinstance(mask, (str, tuple)) else "bytes", alpha, fill)
             hid = (~vis).expand(2, m, n)
             assert torch.equal(C.double()[hid], (C0 if fill is None else torch.full_like(C0, fill))[hid])
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("where", ["q", "k", "k_shifted", "apart_in_one_buffer"])
+def test_sdpa_math_output_over_an_input(yt, dev, where, dt):
+    """O over Q or K (whole, or shifted by some rows) gives the result of an O apart from
+    them: one launch would write O while other workgroups read K. Bound: the rounding
+    of weights and result (the overlapped call runs in separate launches)."""
+    g = torch.Generator(device=dev).manual_seed(5)
+    H, S, D = 16, 1024, 64
+    buf = torch.randn(4 * H * S * D, device=dev, generator=g).to(dt)
+    n = H * S * D
+    q, k, v = (buf[i * n:(i + 1) * n].view(1, H, S, D) for i in range(3))
+    want = yt.scaled_dot_product_attention(q, k, v, mask="causal", backend="math").double()
+    at = {"q": 0, "k": n, "k_shifted": n // 2 + 8 * D, "apart_in_one_buffer": 3 * n}[where]
+    out = buf[at:at + n].view(1, H, S, D)
+    yt.scaled_dot_product_attention(q, k, v, mask="causal", out=out, backend="math")
+    ulp = {torch.float32: 2e-6, torch.bfloat16: 2.0 ** -7}[dt]
+    assert ((out.double() - want).abs() <= ulp * float(v.double().abs().max())).all()

@@ -2358,7 +2358,6 @@ int prefill_typed(AttnArgs a, hipStream_t s) {
 
 template <class T>
 int math_typed(const AttnArgs& a, hipStream_t s) {
-    if (!mfma_layout<T>(a)) return -1;
     if constexpr (std::is_same_v<T, F32>)
         return status_of(a.D == 128 ? launch_math_f32<128>(a, s) : launch_math_f32<64>(a, s));
     else
@@ -2476,7 +2475,7 @@ int decode_route(int dtype, const AttnArgs& p, int mask_kind, const uint8_t* mas
 
 }  // namespace
 
-int attn_math_fused(const AttnCall& c, hipStream_t s) {
+static AttnArgs math_args(const AttnCall& c) {
     AttnArgs a{};
     a.Q = c.Q; a.K = c.K; a.V = c.V; a.O = c.O;
     a.qs0 = c.q_str[0]; a.qs1 = c.q_str[1]; a.qs2 = c.q_str[2]; a.qs3 = c.q_str[3];
@@ -2494,6 +2493,24 @@ int attn_math_fused(const AttnCall& c, hipStream_t s) {
     a.mask = c.mask_kind == YTHIP_MASK_BOOL ? c.mask : nullptr;
     a.mask_ld = c.mask_ld;
     a.bias = c.bias; a.brs = c.brs; a.bcs = c.bcs;
+    return a;
+}
+
+bool attn_math_one_launch(const AttnCall& c) {
+    const AttnArgs a = math_args(c);
+    if (!(c.dtype == YTHIP_F32 ? mfma_layout<F32>(a) : mfma_layout<F16>(a))) return false;
+    // One launch writes O while other workgroups still read Q, K, the mask and the
+    // bias; the separate launches are done with those before O is written.
+    const int es = c.dtype == YTHIP_F32 ? 4 : 2;
+    const Span o = span_of(c.O, es, {{c.B, a.os0}, {c.Hq, a.os1}, {c.Sq, a.os2}, {c.Dv, a.os3}});
+    return !overlap(o, span_of(c.Q, es, {{c.B, a.qs0}, {c.Hq, a.qs1}, {c.Sq, a.qs2}, {c.D, a.qs3}})) &&
+           !overlap(o, span_of(c.K, es, {{c.B, a.ks0}, {c.Hkv, a.ks1}, {c.Skv, a.ks2}, {c.D, a.ks3}})) &&
+           !(a.mask != nullptr && overlap(o, span_of(a.mask, 1, {{c.Sq, a.mask_ld}, {c.Skv, 1}}))) &&
+           !(a.bias != nullptr && overlap(o, span_of(a.bias, 4, {{c.Sq, a.brs}, {c.Skv, a.bcs}})));
+}
+
+int attn_math_fused(const AttnCall& c, hipStream_t s) {
+    const AttnArgs a = math_args(c);
     switch (c.dtype) {
         case YTHIP_F32: return math_typed<F32>(a, s);
         case YTHIP_F16: return math_typed<F16>(a, s);

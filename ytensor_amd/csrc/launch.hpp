@@ -3,6 +3,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <initializer_list>
+#include <utility>
+
 #include "../../include/ythip.h"
 #include "common.hpp"
 
@@ -32,8 +35,21 @@ int gemm_any_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int 
                       int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, const MaskDesc& mask,
                       hipStream_t s);
 
-// The MATH attention backend in one launch (attention.hip); -1 when the layout is
-// not one of the MFMA kernels' (nothing was launched).
+// The bytes from the first to the last element of a strided operand (element sizes and
+// strides; base may be any address, nothing is read).
+struct Span {
+    const char *lo, *hi;
+};
+inline Span span_of(const void* base, int es, std::initializer_list<std::pair<int64_t, int64_t>> size_stride) {
+    int64_t lo = 0, hi = 0;
+    for (const auto& [n, st] : size_stride) (st < 0 ? lo : hi) += (n - 1) * st;
+    const char* p = static_cast<const char*>(base);
+    return {p + lo * es, p + (hi + 1) * es};
+}
+inline bool overlap(const Span& a, const Span& b) { return a.lo < b.hi && b.lo < a.hi; }
+
+// The MATH attention backend in one launch (attention.hip): whether a call takes it,
+// and the launch of one that does.
 struct AttnCall {
     int dtype, B, Hq, Hkv, Sq, Skv, D, Dv;
     const void *Q, *K, *V;
@@ -46,6 +62,7 @@ struct AttnCall {
     const float* bias;
     int64_t brs, bcs;
 };
+bool attn_math_one_launch(const AttnCall& c);
 int attn_math_fused(const AttnCall& c, hipStream_t s);
 
 // Skinny GEMM / fused decode GEMV (gemv.hip): C[m, n] = alpha * A' . W^T + beta * C

@@ -267,10 +267,9 @@ __attribute__((visibility("default"))) int ythip_attn_math(
     const size_t need = ythip_attn_math_workspace_size(dtype, B, Hq, q_len, kv_len);
     if (!workspace || ws_bytes < need)
         return fail(YTHIP_EINVAL, "%s: workspace of %zu bytes needed (%zu given)", who, need, ws_bytes);
-    // one launch for the layouts of the MFMA attention kernels
     const AttnCall call{dtype, B, Hq, Hkv, q_len, kv_len, d, dv, Q, K, V, O, q_str, k_str, v_str, o_str,
                         scale, mask_kind, mask, mask_ld, bias, rs_bias, cs_bias};
-    if (const int st = attn_math_fused(call, s); st != -1) return st;
+    if (attn_math_one_launch(call)) return attn_math_fused(call, s);
     const int G = Hq / Hkv;
     const size_t cells = (size_t)B * Hq * q_len * kv_len;
     float* S = static_cast<float*>(workspace);
