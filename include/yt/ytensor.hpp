@@ -991,10 +991,12 @@ YTensor<T, dim> _sdpa_hip(YTensor<T, dim>& query, YTensor<T, dim>& key, YTensor<
         const int64_t qstr[4] = {f.bq, f.hq, qs2, qs3}, kstr[4] = {f.bk, f.hk, ks2, ks3},
                       vstr[4] = {f.bv, f.hv, vs2, vs3}, ostr[4] = {f.bo, f.ho, os2, 1};
         if (backend == sdpaBackend::MATH) {
-            const size_t need = ythip_attn_math_workspace_size(code, f.batch, f.heads_q, Lq, Lkv);
+            const size_t need = ythip_attn_math_workspace_needed(code, f.batch, f.heads_q, f.heads_kv, Lq, Lkv, D, Dv, q,
+                                                                 qstr, k, kstr, v, vstr, o, ostr, mask_kind, mp, mask_ld,
+                                                                 bp, brs, bcs);
             hip::check(ythip_attn_math(code, f.batch, f.heads_q, f.heads_kv, Lq, Lkv, D, Dv, q, qstr, k, kstr, v,
-                                       vstr, o, ostr, sc, mask_kind, mp, mask_ld, bp, brs, bcs, hip::workspace(need),
-                                       need, hip::stream()),
+                                       vstr, o, ostr, sc, mask_kind, mp, mask_ld, bp, brs, bcs,
+                                       need ? hip::workspace(need) : nullptr, need, hip::stream()),
                        "yt::function::scaledDotProductAttention(MATH)");
             return;
         }

@@ -181,13 +181,20 @@ int ythip_attn_prefill_ws(int dtype, int B, int Hq, int Hkv, int q_len, int kv_l
  *   S = masked_matmul(Q, K^T, mask, -1e9) * scale + bias,  P = softmax_(S, -1),
  *   O = P . V,  rows with no visible key -> 0 (ops.inl:18-40),
  * with S in fp32 and P in the input type (the reference's score tensor has the
- * input type); in one launch without S and P in memory where the layout is one of the
- * flash kernels' (d == dv 64 or 128, 16-byte aligned rows). Same tensor and mask arguments as ythip_attn_prefill, except that
- * every stride may be any value (transposed K / V included). workspace: device
- * scratch of ythip_attn_math_workspace_size(dtype, B, Hq, q_len, kv_len) bytes,
- * required for every layout.
+ * input type). One launch without S and P in memory where the layout is one of the
+ * flash kernels' (d == dv 64 or 128, 16-byte aligned rows) and O lies apart from Q, K, the
+ * mask and the bias; separate launches with both in the workspace elsewhere. Same
+ * tensor and mask arguments as ythip_attn_prefill, except that every stride may be any
+ * value (transposed K / V included). workspace: device scratch of at least the bytes that
+ * ythip_attn_math_workspace_needed gives for the call (0: none, NULL is accepted);
+ * ythip_attn_math_workspace_size gives enough for any layout.
  */
 size_t ythip_attn_math_workspace_size(int dtype, int B, int Hq, int q_len, int kv_len);
+size_t ythip_attn_math_workspace_needed(int dtype, int B, int Hq, int Hkv, int q_len, int kv_len, int d, int dv,
+                                        const void* Q, const int64_t q_str[4], const void* K, const int64_t k_str[4],
+                                        const void* V, const int64_t v_str[4], const void* O,
+                                        const int64_t o_str[4], int mask_kind, const uint8_t* mask, int64_t mask_ld,
+                                        const float* bias, int64_t rs_bias, int64_t cs_bias);
 int ythip_attn_math(int dtype, int B, int Hq, int Hkv, int q_len, int kv_len, int d, int dv,
                     const void* Q, const int64_t q_str[4],
                     const void* K, const int64_t k_str[4],

@@ -113,6 +113,39 @@ def test_prefill_workspace_size_and_short_workspace():
     assert b"workspace of 256 bytes" in lib.ythip_last_error()
 
 
+def _math_call(lib, dtype, H, Hkv, Sq, Skv, D, at, strides=None, B=1, mask=0):
+    """ythip_attn_math_workspace_needed for [B, H, S, D] operands at byte addresses `at`
+    (Q, K, V, O; nothing is read)."""
+    from ytensor_amd import _lib
+    q4 = _lib.i64array([H * Sq * D, Sq * D, D, 1])
+    k4 = _lib.i64array(strides or [Hkv * Skv * D, Skv * D, D, 1])
+    q, k, v, o = (ctypes.c_void_p(x) for x in at)
+    args = (dtype, B, H, Hkv, Sq, Skv, D, D, q, q4, k, k4, v, k4, o, q4)
+    return args, int(lib.ythip_attn_math_workspace_needed(*args, mask, ctypes.c_void_p(1 << 40), Skv, None, 0, 0))
+
+
+def test_math_workspace_only_where_it_is_written():
+    """A MATH call that runs in one launch needs no workspace; one whose layout or whose
+    output (over Q or K) sends it through the separate launches needs all of it, and
+    is refused without (before any launch: the pointers are never dereferenced)."""
+    import ytensor_amd
+    from ytensor_amd import _lib
+    lib = ytensor_amd.load()
+    step = 1 << 30
+    at = [step, 2 * step, 3 * step, 4 * step]
+    for dtype in (_lib.F32, _lib.BF16, _lib.F16):
+        full = int(lib.ythip_attn_math_workspace_size(dtype, 1, 16, 2048, 2048))
+        assert _math_call(lib, dtype, 16, 8, 2048, 2048, 128, at)[1] == 0
+        assert _math_call(lib, dtype, 16, 8, 2048, 2048, 128, [step + 2] + at[1:])[1] == full     # unaligned rows
+        assert _math_call(lib, dtype, 16, 8, 2048, 2048, 128, at, [8 * 2048 * 128, 2048 * 128, 1, 2048])[1] == full
+        assert _math_call(lib, dtype, 16, 8, 2048, 2048, 128, at[:3] + at[:1])[1] == full         # O over Q
+        args, need = _math_call(lib, dtype, 16, 8, 2048, 2048, 128, at[:3] + [2 * step + 256])    # O into K
+        assert need == full
+        assert lib.ythip_attn_math(*args, 0.0, 0, None, 0, None, 0, 0, None, 0, None) == _lib.YTHIP_EINVAL
+        assert b"workspace of" in lib.ythip_last_error()
+    assert _math_call(lib, _lib.BF16, 16, 8, 2048, 0, 128, at)[1] == 0
+
+
 def test_probe_library_loads_and_rejects_bad_shapes():
     """The roofline probe library (libythip_probe.so, measurement support for
     bench.py) loads and refuses shapes it does not take before any launch

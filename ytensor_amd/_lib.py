@@ -58,6 +58,8 @@ SIGNATURES = {
     "ythip_attn_prefill_ws": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _P, _LP, _P, _LP, _P, _LP, _P, _LP,
                                    _F, _I, _P, _L, _P, _L, _L, _P, ctypes.c_size_t, _P]),
     "ythip_attn_math_workspace_size": (ctypes.c_size_t, [_I, _I, _I, _I, _I]),
+    "ythip_attn_math_workspace_needed": (ctypes.c_size_t, [_I, _I, _I, _I, _I, _I, _I, _I, _P, _LP, _P, _LP, _P, _LP,
+                                                            _P, _LP, _I, _P, _L, _P, _L, _L]),
     "ythip_attn_math": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _P, _LP, _P, _LP, _P, _LP, _P, _LP,
                              _F, _I, _P, _L, _P, _L, _L, _P, ctypes.c_size_t, _P]),
     "ythip_gemm_masked_workspace_size": (ctypes.c_size_t, [_I, _I, _I]),

@@ -2477,15 +2477,13 @@ int decode_route(int dtype, const AttnArgs& p, int mask_kind, const uint8_t* mas
 
 static AttnArgs math_args(const AttnCall& c) {
     AttnArgs a{};
-    a.Q = c.Q; a.K = c.K; a.V = c.V; a.O = c.O;
+    a.Q = c.Q; a.K = c.K; a.V = c.V; a.O = const_cast<void*>(c.O);
     a.qs0 = c.q_str[0]; a.qs1 = c.q_str[1]; a.qs2 = c.q_str[2]; a.qs3 = c.q_str[3];
     a.ks0 = c.k_str[0]; a.ks1 = c.k_str[1]; a.ks2 = c.k_str[2]; a.ks3 = c.k_str[3];
     a.vs0 = c.v_str[0]; a.vs1 = c.v_str[1]; a.vs2 = c.v_str[2]; a.vs3 = c.v_str[3];
     a.os0 = c.o_str[0]; a.os1 = c.o_str[1]; a.os2 = c.o_str[2]; a.os3 = c.o_str[3];
     a.o_line = a.os3 == 1 && a.os0 % 8 == 0 && a.os1 % 8 == 0 && a.os2 % 8 == 0 && al(a.O, 16);
     a.B = c.B; a.Hq = c.Hq; a.Hkv = c.Hkv; a.Sq = c.Sq; a.Skv = c.Skv; a.D = c.D; a.Dv = c.Dv;
-    a.scale = c.scale;
-    a.scale_log2 = c.scale * LOG2E;
     a.causal = c.mask_kind == YTHIP_MASK_CAUSAL || c.mask_kind == YTHIP_MASK_DIAG;
     const int64_t off = c.mask_kind == YTHIP_MASK_DIAG ? c.mask_ld : (int64_t)c.Skv - c.Sq;
     a.diag_off = (int)std::max<int64_t>(-(int64_t)c.Sq - 1, std::min<int64_t>(off, c.Skv));
@@ -2509,8 +2507,11 @@ bool attn_math_one_launch(const AttnCall& c) {
            !(a.bias != nullptr && overlap(o, span_of(a.bias, 4, {{c.Sq, a.brs}, {c.Skv, a.bcs}})));
 }
 
-int attn_math_fused(const AttnCall& c, hipStream_t s) {
-    const AttnArgs a = math_args(c);
+int attn_math_fused(const AttnCall& c, void* O, float scale, hipStream_t s) {
+    AttnArgs a = math_args(c);
+    a.O = O;
+    a.scale = scale;
+    a.scale_log2 = scale * LOG2E;
     switch (c.dtype) {
         case YTHIP_F32: return math_typed<F32>(a, s);
         case YTHIP_F16: return math_typed<F16>(a, s);

@@ -53,9 +53,8 @@ inline bool overlap(const Span& a, const Span& b) { return a.lo < b.hi && b.lo <
 struct AttnCall {
     int dtype, B, Hq, Hkv, Sq, Skv, D, Dv;
     const void *Q, *K, *V;
-    void* O;
+    const void* O;
     const int64_t *q_str, *k_str, *v_str, *o_str;
-    float scale;
     int mask_kind;
     const uint8_t* mask;
     int64_t mask_ld;
@@ -63,7 +62,7 @@ struct AttnCall {
     int64_t brs, bcs;
 };
 bool attn_math_one_launch(const AttnCall& c);
-int attn_math_fused(const AttnCall& c, hipStream_t s);
+int attn_math_fused(const AttnCall& c, void* O, float scale, hipStream_t s);
 
 // Skinny GEMM / fused decode GEMV (gemv.hip): C[m, n] = alpha * A' . W^T + beta * C
 // with A' built by the prologue (0: A as is, 1: RMSNorm of fp32 rows, 2: SwiGLU

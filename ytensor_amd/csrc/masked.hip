@@ -237,6 +237,18 @@ __attribute__((visibility("default"))) size_t ythip_attn_math_workspace_size(int
     return dtype == YTHIP_F32 ? cells * 4 : align256(cells * 4) + cells * 2;
 }
 
+__attribute__((visibility("default"))) size_t ythip_attn_math_workspace_needed(
+    int dtype, int B, int Hq, int Hkv, int q_len, int kv_len, int d, int dv, const void* Q, const int64_t q_str[4],
+    const void* K, const int64_t k_str[4], const void* V, const int64_t v_str[4], const void* O,
+    const int64_t o_str[4], int mask_kind, const uint8_t* mask, int64_t mask_ld, const float* bias, int64_t rs_bias,
+    int64_t cs_bias) {
+    const size_t need = dv > 0 ? ythip_attn_math_workspace_size(dtype, B, Hq, q_len, kv_len) : 0;
+    if (need == 0 || !q_str || !k_str || !v_str || !o_str) return need;
+    const AttnCall call{dtype, B, Hq, Hkv, q_len, kv_len, d, dv, Q, K, V, O, q_str, k_str, v_str, o_str,
+                        mask_kind, mask, mask_ld, bias, rs_bias, cs_bias};
+    return attn_math_one_launch(call) ? 0 : need;
+}
+
 __attribute__((visibility("default"))) int ythip_attn_math(
     int dtype, int B, int Hq, int Hkv, int q_len, int kv_len, int d, int dv, const void* Q, const int64_t q_str[4],
     const void* K, const int64_t k_str[4], const void* V, const int64_t v_str[4], void* O, const int64_t o_str[4],
@@ -264,12 +276,12 @@ __attribute__((visibility("default"))) int ythip_attn_math(
                 return st;
         return 0;
     }
+    const AttnCall call{dtype, B, Hq, Hkv, q_len, kv_len, d, dv, Q, K, V, O, q_str, k_str, v_str, o_str,
+                        mask_kind, mask, mask_ld, bias, rs_bias, cs_bias};
+    if (attn_math_one_launch(call)) return attn_math_fused(call, O, scale, s);
     const size_t need = ythip_attn_math_workspace_size(dtype, B, Hq, q_len, kv_len);
     if (!workspace || ws_bytes < need)
         return fail(YTHIP_EINVAL, "%s: workspace of %zu bytes needed (%zu given)", who, need, ws_bytes);
-    const AttnCall call{dtype, B, Hq, Hkv, q_len, kv_len, d, dv, Q, K, V, O, q_str, k_str, v_str, o_str,
-                        scale, mask_kind, mask, mask_ld, bias, rs_bias, cs_bias};
-    if (attn_math_one_launch(call)) return attn_math_fused(call, s);
     const int G = Hq / Hkv;
     const size_t cells = (size_t)B * Hq * q_len * kv_len;
     float* S = static_cast<float*>(workspace);

@@ -267,8 +267,9 @@ def scaled_dot_product_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tens
     mask kind, as flash_attention's q_len == 1 branch does; with a bool mask or
     Sq == 1, a workspace of ythip_attn_sdpa_workspace_size bytes for the mask's
     tile classes or the decode partials) or
-    "math" (MATH: materialised scores in a workspace of
-    ythip_attn_math_workspace_size bytes). A workspace not given or too small
+    "math" (MATH: softmax over every key, hidden scores at -1e9; layouts that do not
+    run in one launch hold the scores in a workspace of
+    ythip_attn_math_workspace_needed bytes). A workspace not given or too small
     is allocated.
     """
     _dev(q, k, v)
@@ -307,14 +308,15 @@ def scaled_dot_product_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tens
 
     def call(qt, kt, vt, ot, B, Hq, Hkv, qs, ks, vs, os_):
         if backend == "math":
-            need = int(_lib.lib().ythip_attn_math_workspace_size(_code(q), B, Hq, Sq, Skv))
+            tensors = (_code(q), B, Hq, Hkv, Sq, Skv, D, dv, qt.data_ptr(), i64array(qs), kt.data_ptr(), i64array(ks),
+                       vt.data_ptr(), i64array(vs), ot.data_ptr(), i64array(os_))
+            need = int(_lib.lib().ythip_attn_math_workspace_needed(*tensors, kind, mptr, mld, bptr, brs, bcs))
             ws = workspace
-            if ws is None or ws.numel() * ws.element_size() < need:
-                ws = torch.empty(max(need, 1), dtype=torch.uint8, device=q.device)
+            if need and (ws is None or ws.numel() * ws.element_size() < need):
+                ws = torch.empty(need, dtype=torch.uint8, device=q.device)
             st = _lib.lib().ythip_attn_math(
-                _code(q), B, Hq, Hkv, Sq, Skv, D, dv, qt.data_ptr(), i64array(qs), kt.data_ptr(), i64array(ks),
-                vt.data_ptr(), i64array(vs), ot.data_ptr(), i64array(os_), float(scale), kind, mptr, mld,
-                bptr, brs, bcs, ws.data_ptr(), ws.numel() * ws.element_size(), _stream())
+                *tensors, float(scale), kind, mptr, mld, bptr, brs, bcs,
+                ws.data_ptr() if need else None, need, _stream())
             check(st, "ythip_attn_math")
         elif kind == _lib.MASK_BOOL or Sq == 1:
             # room for the mask's tile classes (the long-sequence path lists the
