@@ -529,3 +529,24 @@ def test_gemm_swiglu_equals_gemm_then_silu(yt, m, inter, k, dt):
         assert torch.equal(out, want)
     else:  # gemm takes its GEMV there: sums in another order
         assert ((out.double() - want.double()).abs() <= 2.0 ** -6 * want.double().abs() + 1e-3).all()
+
+
+@pytest.mark.parametrize("layout", ["NN", "padded", "batch"])
+@pytest.mark.parametrize("m,n,k", [(2, 4, 4), (2, 64, 8192), (3, 68, 12), (4, 1000, 1020), (8, 512, 516), (9, 64, 2048), (10, 64, 2048),
+                                   (5, 8192, 128), (5, 8192, 132), (10, 20000, 64), (16, 40000, 36)])
+def test_fp32_few_rows_row_major(yt, m, n, k, layout):
+    """2 to 16 fp32 rows against a row-major B on both sides of the rule between the skinny
+    and the tile kernel, k no multiple of its 8 waves, with alpha / beta, padded rows and a
+    batch, against float64. Bound: (k + 2) 2^-24 sum|a||b| plus the rounding of the result."""
+    bt = 3 if layout == "batch" else 1
+    pad = 4 if layout == "padded" else 0
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    A = torch.randn(bt, m, k + pad, device="cuda", generator=g)[:, :, :k]
+    B = torch.randn(bt, k, n + pad, device="cuda", generator=g)[:, :, :n]
+    C = torch.randn(bt, m, n + pad, device="cuda", generator=g)[:, :, :n]
+    C0 = C.clone()
+    yt.gemm(A, B, C, 0.5, 2.0)
+    want = 0.5 * (A.double() @ B.double()) + 2.0 * C0.double()
+    mass = A.double().abs() @ B.double().abs()
+    bound = (k + 2) * 2.0 ** -24 * mass + 2.0 ** -22 * (want.abs() + 2.0 * C0.double().abs()) + 1e-7
+    assert ((C.double() - want).abs() <= bound).all()

@@ -702,9 +702,63 @@ __global__ __launch_bounds__(512, 1) void gemm_pingpong_kernel(GemmArgs a) {
 // the weight stream, so the design goal is bytes in flight, not MFMA reuse.
 //   NT (W^T, the `linear` layout): gemv_kernel in gemv.hip.
 //   NN (B [K][N] row-major): M == 1 in gemv_nn_kernel (16-byte chunks of 8
-//   k-rows per load), else the tile kernels.
+//   k-rows per load), few fp32 rows in gemm_skinny_nn_kernel, else the tile kernels.
 // ---------------------------------------------------------------------------
 constexpr int SKINNY_M = 16;
+constexpr int SKINNY_WAVES = 8;
+
+// A few fp32 rows (m <= 16) with row-major B: lane = one output column, coalesced row
+// loads, 8 waves split k, fp32 sums reduced through LDS. Bound by the weight stream
+// at 2 to 4 rows, by the row loads of A above.
+__global__ __launch_bounds__(64 * SKINNY_WAVES) void gemm_skinny_nn_kernel(GemmArgs a) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = blockIdx.x * 64 + lane;
+    const int bz = blockIdx.y;
+    const float* __restrict__ Ap = static_cast<const float*>(a.A) + bz * a.sa_b;
+    const float* __restrict__ Bp = static_cast<const float*>(a.B) + bz * a.sb_b;
+    const int per_wave = (a.k + SKINNY_WAVES - 1) / SKINNY_WAVES;
+    const int k_begin = wave * per_wave, k_end = min(a.k, k_begin + per_wave);
+    float acc[SKINNY_M];
+#pragma unroll
+    for (int i = 0; i < SKINNY_M; ++i) acc[i] = 0.f;
+    const bool col = n < a.n;
+    const float* bp = Bp + (col ? n : 0);
+    constexpr int UNR = 8;
+    int k = k_begin;
+    for (; k + UNR <= k_end; k += UNR) {
+        float b[UNR];
+#pragma unroll
+        for (int u = 0; u < UNR; ++u) b[u] = col ? bp[(int64_t)(k + u) * a.rsb] : 0.f;
+#pragma unroll
+        for (int i = 0; i < SKINNY_M; ++i) {
+            if (i < a.m) {
+#pragma unroll
+                for (int u = 0; u < UNR; ++u) acc[i] = fmaf(Ap[(int64_t)i * a.rsa + k + u], b[u], acc[i]);
+            }
+        }
+    }
+    for (; k < k_end; ++k) {
+        const float b = col ? bp[(int64_t)k * a.rsb] : 0.f;
+#pragma unroll
+        for (int i = 0; i < SKINNY_M; ++i)
+            if (i < a.m) acc[i] = fmaf(Ap[(int64_t)i * a.rsa + k], b, acc[i]);
+    }
+    __shared__ float red[SKINNY_WAVES][SKINNY_M][64];
+#pragma unroll
+    for (int i = 0; i < SKINNY_M; ++i) red[wave][i][lane] = acc[i];
+    __syncthreads();
+    if (wave != 0 || !col) return;
+    for (int i = 0; i < a.m; ++i) {
+        float t = 0.f;
+#pragma unroll
+        for (int w = 0; w < SKINNY_WAVES; ++w) t += red[w][i][lane];
+        float* crow = static_cast<float*>(a.C) + bz * a.sc_b + (int64_t)i * a.rsc;
+        float v = a.alpha * t;
+        if (a.beta != 0.0f) v += a.beta * crow[n];
+        crow[n] = v;
+    }
+}
+
 // M == 1 with row-major B [K][N] (the configs' weight layout): a workgroup owns
 // CPR * VEC consecutive columns (CPR 16-byte chunks of a k-row); its 16 waves
 // split K, and within a wave lane (r, c) = (lane / CPR, lane % CPR) reads chunk c
@@ -1082,6 +1136,22 @@ hipError_t launch_scale(void* C, int m, int n, int64_t rsc, int64_t csc, int64_t
     return hipGetLastError();
 }
 
+// Few fp32 rows against a row-major B: the tile kernel walks the whole k in one chain of
+// 32-wide steps whatever the rows, 18.5 ns per k and pass over the CUs; the skinny kernel
+// cuts k over 8 waves and pays per row, more once A no longer stays in the caches that the
+// workgroups of an XCD share. Fitted to 770 products (k 256 to 8192, n 36 to 40000, 2 to 16
+// rows, batches of 8 and 64). Skinny / tiles, us, k = 8192: n = 64, 2 rows 82 / 153, 8 rows 135 / 153;
+// n = 8192, 4 rows 150 / 155, 8 rows 223 / 155; n = 40000, 8 rows 283 / 436.
+bool skinny_nn_pays(int m, int n, int k, int batch) {
+    const int64_t tiles = (int64_t)((n + 63) / 64) * batch, passes = (tiles + 255) / 256;
+    double row = 1.15;  // ns per k and row
+    if (tiles * k > 65536 && (int64_t)m * k > 3072) {
+        row = batch == 1 && passes > 1 && k <= 2048 ? 1.8 : 2.2;
+        if (batch > 1) row *= std::min(1.6, std::max(1.0, tiles / 330.0));
+    }
+    return 8.0 + 7.0 * (passes - 1) + row * m <= (passes < 4 ? 18.5 : 20.5) * passes;
+}
+
 bool aligned(const void* p, int bytes) { return (reinterpret_cast<uintptr_t>(p) % bytes) == 0; }
 
 template <class T, class TO>
@@ -1129,6 +1199,12 @@ int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int6
                     gemv_nn_kernel<T, TO, 2><<<dim3((n + 2 * VEC - 1) / (2 * VEC), batch), 1024, 0, s>>>(g);
                 return status_of(hipGetLastError());
             }
+            // 2..16 rows of a row-major fp32 B: see skinny_nn_pays
+            if constexpr (std::is_same_v<T, F32>)
+                if (nn && skinny_nn_pays(m, n, k, batch)) {
+                    gemm_skinny_nn_kernel<<<dim3((n + 63) / 64, batch), 64 * SKINNY_WAVES, 0, s>>>(g);
+                    return status_of(hipGetLastError());
+                }
             // 2..16 rows of a row-major, 16-bit B: the MFMA DMA path (one partial
             // 64-row tile per column tile) streams B at full width
             if constexpr (sizeof(raw) == 2)
