@@ -146,6 +146,28 @@ def test_math_workspace_only_where_it_is_written():
     assert _math_call(lib, _lib.BF16, 16, 8, 2048, 0, 128, at)[1] == 0
 
 
+def test_math_one_launch_rule():
+    """Few workgroups over many keys take the separate launches (one launch measured 1.5 to 5 times
+    their time there), a filled chip, few keys and large batches one launch."""
+    import ytensor_amd
+    from ytensor_amd import _lib
+    lib = ytensor_amd.load()
+    at = [i << 40 for i in range(1, 5)]
+    one = lambda dt, *a, **k: _math_call(lib, dt, *a, at, **k)[1] == 0  # noqa: E731
+    for dt in (_lib.BF16, _lib.F16):
+        for Sq in (1, 16, 64):
+            assert not one(dt, 16, 8, Sq, 4096, 128)
+            assert not one(dt, 1, 1, Sq, 16384, 64)
+            assert not one(dt, 1, 1, Sq, 8192, 128, mask=_lib.MASK_BOOL)
+        assert not one(dt, 16, 8, 128, 4096, 128, mask=_lib.MASK_BOOL)
+        assert one(dt, 16, 8, 512, 512, 128) and one(dt, 16, 8, 1024, 1024, 128, mask=_lib.MASK_BOOL)
+        assert one(dt, 16, 8, 256, 4096, 128) and one(dt, 16, 8, 4096, 4096, 64)
+        assert one(dt, 16, 8, 1, 256, 128) and one(dt, 16, 8, 1, 4096, 128, B=16)
+    assert not one(_lib.F32, 16, 8, 1, 4096, 128) and not one(_lib.F32, 16, 8, 256, 4096, 128)
+    assert not one(_lib.F32, 1, 1, 2048, 2048, 64)
+    assert one(_lib.F32, 16, 8, 2048, 2048, 128) and one(_lib.F32, 16, 16, 4096, 4096, 64)
+
+
 def test_probe_library_loads_and_rejects_bad_shapes():
     """The roofline probe library (libythip_probe.so, measurement support for
     bench.py) loads and refuses shapes it does not take before any launch

@@ -368,3 +368,25 @@ def test_sdpa_math_output_over_an_input(yt, dev, where, dt):
     yt.scaled_dot_product_attention(q, k, v, mask="causal", out=out, backend="math")
     ulp = {torch.float32: 2e-6, torch.bfloat16: 2.0 ** -7}[dt]
     assert ((out.double() - want).abs() <= ulp * float(v.double().abs().max())).all()
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Sq,Skv", [(1, 4100), (3, 5000), (65, 4099)])
+def test_sdpa_math_few_queries_many_keys(yt, dev, Sq, Skv, dt):
+    """The aligned layouts that take the separate launches (few workgroups, many keys),
+    GQA 2:1, against float64. Bound as in test_sdpa_math_one_launch."""
+    g = torch.Generator(device=dev).manual_seed(Sq + Skv)
+    D = 64
+    q = torch.randn(1, 4, Sq, D, device=dev, generator=g).to(dt)
+    k = torch.randn(1, 2, Skv, D, device=dev, generator=g).to(dt)
+    v = torch.randn(1, 2, Skv, D, device=dev, generator=g).to(dt)
+    i, j = torch.arange(Sq, device=dev)[:, None], torch.arange(Skv, device=dev)[None, :]
+    drop = torch.rand(Sq, Skv, device=dev, generator=g) < 0.4
+    drop[Sq // 2] = True
+    bias = torch.randn(Sq, Skv, device=dev, generator=g)
+    ulp = {torch.float32: 2e-7, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dt]
+    for mask, vis, bs in [(None, None, None), ("causal", j <= i + Skv - Sq, None), (~drop, ~drop, bias)]:
+        out = yt.scaled_dot_product_attention(q, k, v, 0.0, mask=mask, bias=bs, backend="math")[0]
+        want = _math64(q[0], k[0], v[0], 1.0 / D ** 0.5, vis, bs)
+        bound = (1e-5 + ulp) * float(v.double().abs().max()) + 2 * ulp * want.abs()
+        assert ((out.double() - want).abs() <= bound).all()

@@ -2494,6 +2494,32 @@ static AttnArgs math_args(const AttnCall& c) {
     return a;
 }
 
+// One launch walks all keys in one workgroup per 64 queries and head, so its time is
+// passes over the 256 CUs times keys times what a key costs a workgroup; the separate
+// launches spread the keys over the chip but move every score through memory. Both
+// estimates are in us. Their constants are the ones that choose best over 1356 measured calls
+// (d 64 and 128; 16-bit and fp32; B 1 to 16, 1 to 16 heads, 1 to 4096 queries, 256 to 16384 keys;
+// no mask, bytes, bias): the choice is 0.3% off the faster form on average. Separate / one
+// launch, us: bf16, d 128, 16 heads, 1 query over 4096 keys 33.8 / 49.8 and with bytes 35.6 /
+// 102, 256 queries 70.6 / 51.2 and 79.1 / 108.5, 512 x 4096 105.8 / 51.9; fp32, 1 query 71.7 /
+// 295.6, 2048 x 2048 474 / 309.
+static bool math_one_launch_pays(const AttnCall& c) {
+    const bool f32 = c.dtype == YTHIP_F32, general = c.mask_kind == YTHIP_MASK_BOOL || c.bias != nullptr;
+    const double keys = c.Skv, cells = (double)c.B * c.Hq * c.Sq * keys;
+    const int64_t passes = ((int64_t)((c.Sq + 63) / 64) * c.B * c.Hq + 255) / 256;
+    double ns;  // per key, of a workgroup (general: every score through math_scores4)
+    if (f32) ns = c.D == 128 ? (general ? 71.9 : 74.4) : (general ? 56.1 : 38.3);
+    else ns = c.D == 128 ? (general ? 28.0 : 12.1) : (general ? 24.1 : 8.25);
+    const double one = (f32 ? 1.1 : 2.5) + passes * keys * ns * 1e-3;
+    // the query heads of one kv head are one matrix only where they lie row after row
+    const bool rows = c.q_str[1] == (int64_t)c.Sq * c.q_str[2] && c.o_str[1] == (int64_t)c.Sq * c.o_str[2];
+    const double products = (double)c.B * (rows ? 1 : c.Hq / c.Hkv);
+    const double past_cache = std::max(0.0, cells - 34e6);  // scores that the memory-side cache does not hold
+    const double separate = f32 ? std::max(15.5, products * (9.4 + 0.0134 * keys) + 4.72e-6 * cells + 6.4e-6 * past_cache)
+                                : std::max(20.6, products * (5.0 + 0.00586 * keys) + 2.74e-6 * cells + 10.7e-6 * past_cache);
+    return one <= separate;
+}
+
 bool attn_math_one_launch(const AttnCall& c) {
     const AttnArgs a = math_args(c);
     if (!(c.dtype == YTHIP_F32 ? mfma_layout<F32>(a) : mfma_layout<F16>(a))) return false;
@@ -2501,7 +2527,7 @@ bool attn_math_one_launch(const AttnCall& c) {
     // bias; the separate launches are done with those before O is written.
     const int es = c.dtype == YTHIP_F32 ? 4 : 2;
     const Span o = span_of(c.O, es, {{c.B, a.os0}, {c.Hq, a.os1}, {c.Sq, a.os2}, {c.Dv, a.os3}});
-    return !overlap(o, span_of(c.Q, es, {{c.B, a.qs0}, {c.Hq, a.qs1}, {c.Sq, a.qs2}, {c.D, a.qs3}})) &&
+    return math_one_launch_pays(c) && !overlap(o, span_of(c.Q, es, {{c.B, a.qs0}, {c.Hq, a.qs1}, {c.Sq, a.qs2}, {c.D, a.qs3}})) &&
            !overlap(o, span_of(c.K, es, {{c.B, a.ks0}, {c.Hkv, a.ks1}, {c.Skv, a.ks2}, {c.D, a.ks3}})) &&
            !(a.mask != nullptr && overlap(o, span_of(a.mask, 1, {{c.Sq, a.mask_ld}, {c.Skv, 1}}))) &&
            !(a.bias != nullptr && overlap(o, span_of(a.bias, 4, {{c.Sq, a.brs}, {c.Skv, a.bcs}})));
