@@ -390,3 +390,26 @@ def test_sdpa_math_few_queries_many_keys(yt, dev, Sq, Skv, dt):
         want = _math64(q[0], k[0], v[0], 1.0 / D ** 0.5, vis, bs)
         bound = (1e-5 + ulp) * float(v.double().abs().max()) + 2 * ulp * want.abs()
         assert ((out.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("din,dout", [(torch.float32, torch.bfloat16), (torch.float32, torch.float16),
+                                      (torch.bfloat16, torch.float16), (torch.float16, torch.bfloat16),
+                                      (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("m,n,k", [(5, 7, 3), (130, 200, 72)])
+def test_gemm_masked_output_types(yt, dev, m, n, k, din, dout):
+    """A C of any type, kept or filled, with alpha / beta, against float64: (k + 2) 2^-24
+    sum|a||b| plus the rounding of the result."""
+    g = torch.Generator(device=dev).manual_seed(m)
+    A = torch.randn(m, k, device=dev, generator=g).to(din)
+    B = torch.randn(k, n, device=dev, generator=g).to(din)
+    vis = torch.rand(m, n, device=dev, generator=g) < 0.5
+    prod, mass = A.double() @ B.double(), A.double().abs() @ B.double().abs()
+    ulp = {torch.float32: 2.0 ** -23, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -10}[dout]
+    for alpha, beta, fill in [(1.0, 0.0, -3.0), (1.0, 0.0, None), (0.5, 2.0, 7.0), (0.5, 0.0, None)]:
+        C = torch.randn(m, n, device=dev, generator=g).to(dout)
+        C0 = C.double()
+        yt.gemm_masked(A, B, C, vis, alpha, beta, fill)
+        want = alpha * prod + beta * C0
+        bound = (k + 2) * 2.0 ** -24 * mass + ulp * want.abs() + 4 * 2.0 ** -23 * C0.abs() + 1e-7
+        assert ((C.double() - want).abs() <= bound)[vis].all()
+        assert torch.equal(C.double()[~vis], (C0 if fill is None else torch.full_like(C0, fill))[~vis])

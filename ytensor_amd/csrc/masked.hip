@@ -30,18 +30,29 @@
 
 namespace ythip {
 
-// The k == 0 / alpha == 0 case of sgemm_masked: visible entries scaled by beta (zero
-// for beta = 0), hidden ones kept or filled.
+// C[b] (m x n) from the product W[b] = A.B (fp32, row stride n): where visible,
+// C = alpha * W + beta * C; elsewhere C keeps its value, or takes the mask's when it
+// fills. W == nullptr is the k == 0 / alpha == 0 case of sgemm_masked (visible entries scaled
+// by beta, zero for beta = 0). Bound by the bytes of W, C and the mask.
 template <class TO>
-__global__ __launch_bounds__(256) void masked_scale_kernel(void* C, int64_t sc_b, int64_t rsc, int64_t csc, int m, int n,
-                                                           MaskDesc mk, float beta) {
+__global__ __launch_bounds__(256) void masked_blend_kernel(const float* __restrict__ W, void* C, int64_t sc_b,
+                                                           int64_t rsc, int64_t csc, int m, int n, MaskDesc mk,
+                                                           float alpha, float beta) {
     const int cb = (gridDim.x + m - 1) / m;  // column blocks per row
     const int i = blockIdx.x / cb;
     const int b = blockIdx.z;
+    const float* wr = W != nullptr ? W + ((int64_t)b * m + i) * n : nullptr;
     for (int j = (blockIdx.x - i * cb) * 256 + threadIdx.x; j < n; j += cb * 256) {
         const int64_t co = (int64_t)b * sc_b + (int64_t)i * rsc + (int64_t)j * csc;
         if (visible(mk, i, j)) {
-            if (beta != 1.0f) store_from_f32<TO>(C, co, beta == 0.0f ? 0.0f : beta * load_as_f32<TO>(C, co));
+            float v;
+            if (wr == nullptr) {
+                if (beta == 1.0f) continue;
+                v = beta == 0.0f ? 0.0f : beta * load_as_f32<TO>(C, co);
+            } else {
+                v = beta == 0.0f ? alpha * wr[j] : alpha * wr[j] + beta * load_as_f32<TO>(C, co);
+            }
+            store_from_f32<TO>(C, co, v);
         } else if (mk.fill) {
             store_from_f32<TO>(C, co, mk.value);
         }
@@ -178,15 +189,20 @@ int check_mask(const char* who, int kind, const uint8_t* data, int64_t ld, int n
     return 0;
 }
 
-hipError_t masked_scale(int dtype_out, void* C, int64_t sc_b, int64_t rsc, int64_t csc, int batch, int m, int n,
-                        const MaskDesc& mk, float beta, hipStream_t s) {
+hipError_t masked_blend(int dtype_out, const float* W, void* C, int64_t sc_b, int64_t rsc, int64_t csc, int batch, int m,
+                        int n, const MaskDesc& mk, float alpha, float beta, hipStream_t s) {
     const int cb = (n + 255) / 256 < 8 ? (n + 255) / 256 : 8;
     const dim3 grid((unsigned)((int64_t)m * cb), 1, batch);
-    if (dtype_out == YTHIP_F32) masked_scale_kernel<F32><<<grid, 256, 0, s>>>(C, sc_b, rsc, csc, m, n, mk, beta);
-    else if (dtype_out == YTHIP_BF16) masked_scale_kernel<BF16><<<grid, 256, 0, s>>>(C, sc_b, rsc, csc, m, n, mk, beta);
-    else masked_scale_kernel<F16><<<grid, 256, 0, s>>>(C, sc_b, rsc, csc, m, n, mk, beta);
+    if (dtype_out == YTHIP_F32) masked_blend_kernel<F32><<<grid, 256, 0, s>>>(W, C, sc_b, rsc, csc, m, n, mk, alpha, beta);
+    else if (dtype_out == YTHIP_BF16)
+        masked_blend_kernel<BF16><<<grid, 256, 0, s>>>(W, C, sc_b, rsc, csc, m, n, mk, alpha, beta);
+    else masked_blend_kernel<F16><<<grid, 256, 0, s>>>(W, C, sc_b, rsc, csc, m, n, mk, alpha, beta);
     return hipGetLastError();
 }
+
+// Whether the product's store applies the mask. A type of C that no product kernel
+// stores goes through the fp32 product in the workspace.
+bool masked_in_store(int dtype_in, int dtype_out) { return dtype_out == dtype_in || dtype_out == YTHIP_F32; }
 
 int esize(int dtype) { return dtype == YTHIP_F32 ? 4 : 2; }
 
@@ -221,13 +237,19 @@ __attribute__((visibility("default"))) int ythip_gemm_masked(
     mk.value = masked_value;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (k == 0 || alpha == 0.0f)  // sgemm.inl:352-363 (fill still applies to the masked entries)
-        return status_of(masked_scale(dtype_out, C, sc_b, rsc, csc, batch, m, n, mk, beta, s));
+        return status_of(masked_blend(dtype_out, nullptr, C, sc_b, rsc, csc, batch, m, n, mk, 0.0f, beta, s));
     if (!A || !B) return fail(YTHIP_EINVAL, "%s: A or B is NULL", who);
     const size_t need = ythip_gemm_masked_workspace_size(batch, m, n);
     if (!workspace || ws_bytes < need)
         return fail(YTHIP_EINVAL, "%s: workspace of %zu bytes needed (%zu given)", who, need, ws_bytes);
-    return gemm_masked_dispatch(dtype_in, dtype_out, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b, rsc,
-                                csc, alpha, beta, mk, s);
+    if (masked_in_store(dtype_in, dtype_out))
+        return gemm_masked_dispatch(dtype_in, dtype_out, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b,
+                                    rsc, csc, alpha, beta, mk, s);
+    float* W = static_cast<float*>(workspace);
+    if (int st = gemm_dispatch(dtype_in, YTHIP_F32, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, W,
+                               (int64_t)m * n, n, 1, 1.0f, 0.0f, s))
+        return st;
+    return status_of(masked_blend(dtype_out, W, C, sc_b, rsc, csc, batch, m, n, mk, alpha, beta, s));
 }
 
 __attribute__((visibility("default"))) size_t ythip_attn_math_workspace_size(int dtype, int B, int Hq, int q_len,
