@@ -413,3 +413,24 @@ def test_gemm_masked_output_types(yt, dev, m, n, k, din, dout):
         bound = (k + 2) * 2.0 ** -24 * mass + ulp * want.abs() + 4 * 2.0 ** -23 * C0.abs() + 1e-7
         assert ((C.double() - want).abs() <= bound)[vis].all()
         assert torch.equal(C.double()[~vis], (C0 if fill is None else torch.full_like(C0, fill))[~vis])
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("where", ["a", "b", "a_shifted", "apart_in_one_buffer"])
+def test_gemm_masked_output_over_an_input(yt, dev, where, dt):
+    """C over A or B (whole, or shifted by some rows) gives the result of a C apart from them:
+    with the mask in the product's store, tiles of C would be written while others
+    still read A and B. Against float64 as in test_gemm_masked_layouts; kept entries are
+    the input's."""
+    g = torch.Generator(device=dev).manual_seed(6)
+    n = 1024
+    buf = (torch.randn(3 * n * n, device=dev, generator=g) * 0.25).to(dt)
+    a, b = buf[:n * n].view(n, n), buf[n * n:2 * n * n].view(n, n)
+    vis = torch.rand(n, n, device=dev, generator=g) < 0.5
+    at = {"a": 0, "b": n * n, "a_shifted": 72 * n, "apart_in_one_buffer": 2 * n * n}[where]
+    c = buf[at:at + n * n].view(n, n)
+    c0, prod, mass = c.clone(), a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    ulp = {torch.float32: 2.0 ** -23, torch.bfloat16: 2.0 ** -8}[dt]
+    yt.gemm_masked(a, b, c, vis)
+    assert ((c.double() - prod).abs() <= (n + 2) * 2.0 ** -24 * mass + ulp * prod.abs())[vis].all()
+    assert torch.equal(c[~vis], c0[~vis])

@@ -200,11 +200,27 @@ hipError_t masked_blend(int dtype_out, const float* W, void* C, int64_t sc_b, in
     return hipGetLastError();
 }
 
-// Whether the product's store applies the mask. A type of C that no product kernel
-// stores goes through the fp32 product in the workspace.
-bool masked_in_store(int dtype_in, int dtype_out) { return dtype_out == dtype_in || dtype_out == YTHIP_F32; }
-
 int esize(int dtype) { return dtype == YTHIP_F32 ? 4 : 2; }
+
+struct MaskedCall {
+    int dtype_in, dtype_out, batch, m, n, k;
+    const void* A;
+    int64_t sa_b, rsa, csa;
+    const void* B;
+    int64_t sb_b, rsb, csb;
+    const void* C;
+    int64_t sc_b, rsc, csc;
+};
+
+// Whether the product's store applies the mask. Otherwise the fp32 product goes to the
+// workspace and a second launch blends it into C: a type of C that no product kernel
+// stores; a C over A or B, which other workgroups still read when tiles of C are stored.
+bool masked_in_store(const MaskedCall& c) {
+    if (c.dtype_out != c.dtype_in && c.dtype_out != YTHIP_F32) return false;
+    const Span o = span_of(c.C, esize(c.dtype_out), {{c.batch, c.sc_b}, {c.m, c.rsc}, {c.n, c.csc}});
+    return !overlap(o, span_of(c.A, esize(c.dtype_in), {{c.batch, c.sa_b}, {c.m, c.rsa}, {c.k, c.csa}})) &&
+           !overlap(o, span_of(c.B, esize(c.dtype_in), {{c.batch, c.sb_b}, {c.k, c.rsb}, {c.n, c.csb}}));
+}
 
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
@@ -242,7 +258,7 @@ __attribute__((visibility("default"))) int ythip_gemm_masked(
     const size_t need = ythip_gemm_masked_workspace_size(batch, m, n);
     if (!workspace || ws_bytes < need)
         return fail(YTHIP_EINVAL, "%s: workspace of %zu bytes needed (%zu given)", who, need, ws_bytes);
-    if (masked_in_store(dtype_in, dtype_out))
+    if (masked_in_store({dtype_in, dtype_out, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b, rsc, csc}))
         return gemm_masked_dispatch(dtype_in, dtype_out, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b,
                                     rsc, csc, alpha, beta, mk, s);
     float* W = static_cast<float*>(workspace);
