@@ -211,10 +211,17 @@ int ythip_attn_math(int dtype, int B, int Hq, int Hkv, int q_len, int kv_len, in
  *   C = alpha * A.B + beta * C   (k == 0 or alpha == 0: C *= beta, 0 for beta == 0)
  * and elsewhere C is left unchanged, or set to masked_value when fill_masked != 0
  * (masked_matmul's fill). mask_kind / mask / mask_ld as for attention, with the
- * causal offset n - m. One launch; workspace of ythip_gemm_masked_workspace_size(batch,
- * m, n) bytes is still required where a product is computed, and not written.
+ * causal offset n - m. One launch, or the fp32 product in the workspace and a pass over
+ * it: for a C whose type differs from the inputs' and is not fp32, and a C that lies over
+ * A or B. workspace: at least the bytes that ythip_gemm_masked_workspace_needed gives for the
+ * call (0: none, NULL is accepted); ythip_gemm_masked_workspace_size gives enough for any.
  */
 size_t ythip_gemm_masked_workspace_size(int batch, int m, int n);
+size_t ythip_gemm_masked_workspace_needed(int dtype_in, int dtype_out, int batch, int m, int n, int k,
+                                          const void* A, int64_t sa_b, int64_t rsa, int64_t csa,
+                                          const void* B, int64_t sb_b, int64_t rsb, int64_t csb,
+                                          const void* C, int64_t sc_b, int64_t rsc, int64_t csc, float alpha,
+                                          int mask_kind, int64_t mask_ld, int fill_masked);
 int ythip_gemm_masked(int dtype_in, int dtype_out, int batch, int m, int n, int k,
                       const void* A, int64_t sa_b, int64_t rsa, int64_t csa,
                       const void* B, int64_t sb_b, int64_t rsb, int64_t csb,

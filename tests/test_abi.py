@@ -168,6 +168,36 @@ def test_math_one_launch_rule():
     assert one(_lib.F32, 16, 8, 2048, 2048, 128) and one(_lib.F32, 16, 16, 4096, 4096, 64)
 
 
+def _masked_call(din, dout, m, n, k, at=(1 << 40, 2 << 40, 3 << 40), nt=False, alpha=1.0, kind=2, mask_ld=0, fill=1, batch=1):
+    """(needed bytes, operand arguments) of a masked product at byte addresses `at`; nothing is read."""
+    import ytensor_amd
+    a, b, c = (ctypes.c_void_p(x) for x in at)
+    bs = (1, k) if nt else (n, 1)
+    args = (din, dout, batch, m, n, k, a, m * k, k, 1, b, n * k, *bs, c, m * n, n, 1, alpha)
+    return int(ytensor_amd.load().ythip_gemm_masked_workspace_needed(*args, kind, mask_ld or n, fill)), args
+
+
+def test_masked_workspace_only_where_it_is_written():
+    """A masked product in one launch needs no workspace; a C of another type or over an
+    input needs m n floats, and is refused without (before any launch)."""
+    import ytensor_amd
+    from ytensor_amd import _lib
+    lib = ytensor_amd.load()
+    m, n, k = 200, 300, 128
+    for dt in (_lib.F32, _lib.BF16, _lib.F16):
+        assert _masked_call(dt, dt, m, n, k)[0] == 0
+        assert _masked_call(dt, _lib.F32, m, n, k)[0] == 0
+        for at in ((1 << 40, 2 << 40, 1 << 40), (1 << 40, 2 << 40, (2 << 40) + 64), (1 << 40, 2 << 40, (1 << 40) - 64)):
+            need, args = _masked_call(dt, dt, m, n, k, at)
+            assert need == m * n * 4 == lib.ythip_gemm_masked_workspace_size(1, m, n)
+            st = lib.ythip_gemm_masked(*args, 0.0, 2, ctypes.c_void_p(1 << 44), n, 1, 0.0, None, 0, None)
+            assert st == _lib.YTHIP_EINVAL and b"workspace of" in lib.ythip_last_error()
+        assert _masked_call(dt, dt, m, n, k, (1 << 40, 2 << 40, 1 << 40), alpha=0.0)[0] == 0
+        assert _masked_call(dt, dt, m, n, 0)[0] == 0
+    assert _masked_call(_lib.F32, _lib.BF16, m, n, k)[0] == m * n * 4
+    assert _masked_call(_lib.BF16, _lib.F16, m, n, k)[0] == m * n * 4
+
+
 def test_probe_library_loads_and_rejects_bad_shapes():
     """The roofline probe library (libythip_probe.so, measurement support for
     bench.py) loads and refuses shapes it does not take before any launch

@@ -63,6 +63,8 @@ SIGNATURES = {
     "ythip_attn_math": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _P, _LP, _P, _LP, _P, _LP, _P, _LP,
                              _F, _I, _P, _L, _P, _L, _L, _P, ctypes.c_size_t, _P]),
     "ythip_gemm_masked_workspace_size": (ctypes.c_size_t, [_I, _I, _I]),
+    "ythip_gemm_masked_workspace_needed": (ctypes.c_size_t, [_I, _I, _I, _I, _I, _I, _P, _L, _L, _L, _P, _L, _L, _L,
+                                                             _P, _L, _L, _L, _F, _I, _L, _I]),
     "ythip_gemm_masked": (_I, [_I, _I, _I, _I, _I, _I, _P, _L, _L, _L, _P, _L, _L, _L, _P, _L, _L, _L, _F, _F,
                                _I, _P, _L, _I, _F, _P, ctypes.c_size_t, _P]),
     "ythip_attn_decode_workspace_size": (ctypes.c_size_t, [_I, _I, _I, _I]),

@@ -210,6 +210,7 @@ struct MaskedCall {
     int64_t sb_b, rsb, csb;
     const void* C;
     int64_t sc_b, rsc, csc;
+    MaskDesc mask;
 };
 
 // Whether the product's store applies the mask. Otherwise the fp32 product goes to the
@@ -236,6 +237,18 @@ __attribute__((visibility("default"))) size_t ythip_gemm_masked_workspace_size(i
     return (size_t)batch * m * n * sizeof(float);
 }
 
+__attribute__((visibility("default"))) size_t ythip_gemm_masked_workspace_needed(
+    int dtype_in, int dtype_out, int batch, int m, int n, int k, const void* A, int64_t sa_b, int64_t rsa,
+    int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, const void* C, int64_t sc_b, int64_t rsc,
+    int64_t csc, float alpha, int mask_kind, int64_t mask_ld, int fill_masked) {
+    const size_t need = ythip_gemm_masked_workspace_size(batch, m, n);
+    if (need == 0 || k <= 0 || alpha == 0.0f) return 0;
+    MaskDesc mk = make_mask(mask_kind, nullptr, mask_ld, m, n);
+    mk.fill = fill_masked;
+    return masked_in_store({dtype_in, dtype_out, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b, rsc, csc,
+                            mk}) ? 0 : need;
+}
+
 __attribute__((visibility("default"))) int ythip_gemm_masked(
     int dtype_in, int dtype_out, int batch, int m, int n, int k, const void* A, int64_t sa_b, int64_t rsa,
     int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C, int64_t sc_b, int64_t rsc,
@@ -255,12 +268,12 @@ __attribute__((visibility("default"))) int ythip_gemm_masked(
     if (k == 0 || alpha == 0.0f)  // sgemm.inl:352-363 (fill still applies to the masked entries)
         return status_of(masked_blend(dtype_out, nullptr, C, sc_b, rsc, csc, batch, m, n, mk, 0.0f, beta, s));
     if (!A || !B) return fail(YTHIP_EINVAL, "%s: A or B is NULL", who);
+    if (masked_in_store({dtype_in, dtype_out, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b, rsc, csc, mk}))
+        return gemm_masked_dispatch(dtype_in, dtype_out, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b,
+                                    rsc, csc, alpha, beta, mk, s);
     const size_t need = ythip_gemm_masked_workspace_size(batch, m, n);
     if (!workspace || ws_bytes < need)
         return fail(YTHIP_EINVAL, "%s: workspace of %zu bytes needed (%zu given)", who, need, ws_bytes);
-    if (masked_in_store({dtype_in, dtype_out, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b, rsc, csc}))
-        return gemm_masked_dispatch(dtype_in, dtype_out, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b,
-                                    rsc, csc, alpha, beta, mk, s);
     float* W = static_cast<float*>(workspace);
     if (int st = gemm_dispatch(dtype_in, YTHIP_F32, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, W,
                                (int64_t)m * n, n, 1, 1.0f, 0.0f, s))

@@ -378,7 +378,9 @@ def gemm_masked(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor, mask, alpha
     """sgemm_masked (src/kernel/avx2/sgemm.inl:342-584) on 2-D or batched 3-D
     operands: where `mask` ([m, n], shared by the batch; forms as for attention)
     is set, out = alpha * a @ b + beta * out; elsewhere out is kept, or set to
-    `fill` when given (masked_matmul's maskedValue)."""
+    `fill` when given (masked_matmul's maskedValue). out may lie over a or b. A workspace
+    that the call needs (ythip_gemm_masked_workspace_needed) and that is not given or too
+    small is allocated."""
     _dev(a, b, out)
     if a.dtype != b.dtype:
         raise ValueError("a and b must share a dtype")
@@ -392,17 +394,16 @@ def gemm_masked(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor, mask, alpha
     if tuple(C.shape) != (bt, m, n) or Bm.shape[0] not in (1, bt):
         raise ValueError("masked_matmul: shapes do not match")
     kind, mptr, mld, keep = _mask_args(mask, m, n, a.device)
-    need = masked_gemm_workspace_bytes(bt, m, n)
+    operands = (_code(a), _code(out), bt, m, n, k, A.data_ptr(), A.stride(0), A.stride(1), A.stride(2),
+                Bm.data_ptr(), 0 if Bm.shape[0] == 1 else Bm.stride(0), Bm.stride(1), Bm.stride(2),
+                C.data_ptr(), C.stride(0), C.stride(1), C.stride(2), float(alpha))
+    filled = int(fill is not None)
+    need = int(_lib.lib().ythip_gemm_masked_workspace_needed(*operands, kind, mld, filled))
     ws = workspace
-    if ws is None or ws.numel() * ws.element_size() < need:
-        ws = torch.empty(max(need, 1), dtype=torch.uint8, device=a.device)
-    st = _lib.lib().ythip_gemm_masked(
-        _code(a), _code(out), bt, m, n, k,
-        A.data_ptr(), A.stride(0), A.stride(1), A.stride(2),
-        Bm.data_ptr(), 0 if Bm.shape[0] == 1 else Bm.stride(0), Bm.stride(1), Bm.stride(2),
-        C.data_ptr(), C.stride(0), C.stride(1), C.stride(2), float(alpha), float(beta),
-        kind, mptr, mld, int(fill is not None), float(fill or 0.0), ws.data_ptr(), ws.numel() * ws.element_size(),
-        _stream())
+    if need and (ws is None or ws.numel() * ws.element_size() < need):
+        ws = torch.empty(need, dtype=torch.uint8, device=a.device)
+    st = _lib.lib().ythip_gemm_masked(*operands, float(beta), kind, mptr, mld, filled, float(fill or 0.0),
+                                      ws.data_ptr() if need else None, need, _stream())
     check(st, "ythip_gemm_masked")
     return out
 
