@@ -182,8 +182,9 @@ int ythip_attn_prefill_ws(int dtype, int B, int Hq, int Hkv, int q_len, int kv_l
  *   O = P . V,  rows with no visible key -> 0 (ops.inl:18-40),
  * with S in fp32 and P in the input type (the reference's score tensor has the
  * input type). One launch without S and P in memory where the layout is one of the
- * flash kernels' (d == dv 64 or 128, 16-byte aligned rows) and O lies apart from Q, K, the
- * mask and the bias; separate launches with both in the workspace elsewhere. Same
+ * flash kernels' (d == dv 64 or 128, 16-byte aligned rows), O lies apart from Q, K, the
+ * mask and the bias, and there are queries enough to fill the chip while each workgroup
+ * walks all keys; separate launches with both in the workspace elsewhere. Same
  * tensor and mask arguments as ythip_attn_prefill, except that every stride may be any
  * value (transposed K / V included). workspace: device scratch of at least the bytes that
  * ythip_attn_math_workspace_needed gives for the call (0: none, NULL is accepted);
@@ -212,8 +213,8 @@ int ythip_attn_math(int dtype, int B, int Hq, int Hkv, int q_len, int kv_len, in
  * and elsewhere C is left unchanged, or set to masked_value when fill_masked != 0
  * (masked_matmul's fill). mask_kind / mask / mask_ld as for attention, with the
  * causal offset n - m. One launch, or the fp32 product in the workspace and a pass over
- * it: for a C whose type differs from the inputs' and is not fp32, and a C that lies over
- * A or B. workspace: at least the bytes that ythip_gemm_masked_workspace_needed gives for the
+ * it: for a C whose type differs from the inputs' and is not fp32, a C that lies over A or
+ * B, and sizes that are faster so. workspace: at least the bytes that ythip_gemm_masked_workspace_needed gives for the
  * call (0: none, NULL is accepted); ythip_gemm_masked_workspace_size gives enough for any.
  */
 size_t ythip_gemm_masked_workspace_size(int batch, int m, int n);

@@ -198,6 +198,30 @@ def test_masked_workspace_only_where_it_is_written():
     assert _masked_call(_lib.BF16, _lib.F16, m, n, k)[0] == m * n * 4
 
 
+def test_masked_store_rule():
+    """Masked products that are faster as a product in the workspace and a blend: few rows with
+    a long k, 256-wide tiles with a long k, operands of 2 GiB; the others keep the one launch."""
+    from ytensor_amd import _lib
+    need = lambda *a, **k: _masked_call(*a, **k)[0] > 0  # noqa: E731
+    causal, bytes_, diag = _lib.MASK_CAUSAL, _lib.MASK_BOOL, _lib.MASK_DIAG
+    H, F = _lib.BF16, _lib.F32
+    for m in (1, 16):
+        assert need(H, H, m, 1024, 8192, nt=True) and not need(H, H, m, 1024, 1024, nt=True)
+        assert need(F, F, m, 1024, 1024, nt=True) and not need(F, F, m, 1024, 256, nt=True)
+    assert need(H, H, 1, 1024, 8192) and need(F, F, 2, 1024, 1024) and not need(H, H, 2, 1024, 8192)
+    assert not need(H, H, 17, 1024, 8192, nt=True)
+    for n in (512, 2048, 3072):
+        for kind in (causal, bytes_):
+            assert not need(H, H, n, n, n, kind=kind) and not need(H, H, n, n, n, kind=kind, fill=0)
+    assert need(H, H, 4096, 4096, 4096) and need(H, H, 4096, 4096, 4096, fill=0) and need(H, H, 8192, 8192, 8192, kind=causal)
+    assert not need(H, H, 4096, 4096, 1024) and not need(H, H, 4096, 4096, 512, fill=0)
+    assert not need(H, H, 4096, 4096, 4096, kind=diag, mask_ld=-4000)
+    assert not need(F, F, 4096, 4096, 4096) and not need(F, F, 8192, 8192, 8192, kind=causal)
+    assert need(H, H, 131200, 256, 8192) and not need(H, H, 131200, 64, 8192)
+    assert not need(H, H, 131200, 256, 8192, kind=causal) and need(H, H, 256, 131200, 8192, nt=True, kind=causal)
+    assert not need(H, H, 4096, 4096, 4096, kind=_lib.MASK_NONE)
+
+
 def test_probe_library_loads_and_rejects_bad_shapes():
     """The roofline probe library (libythip_probe.so, measurement support for
     bench.py) loads and refuses shapes it does not take before any launch

@@ -145,6 +145,13 @@ template <class TO>
 __device__ __forceinline__ void masked_store4(const MaskDesc& mk, typename TO::raw* crow, int64_t cs, int m, int n, int cols,
                                               f32x4 v, float beta) {
     const uint32_t vis = visible4(mk, m, n, cols);
+    if (vis == 0xf && cs == 1 && beta == 0.0f) {  // the common case in one store
+        if constexpr (sizeof(typename TO::raw) == 2)
+            *reinterpret_cast<u32x2_any*>(crow + n) = u32x2{pack2<TO>(v[0], v[1]), pack2<TO>(v[2], v[3])};
+        else
+            *reinterpret_cast<f32x4_any*>(crow + n) = v;
+        return;
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         if (n + r >= cols) continue;

@@ -1048,11 +1048,12 @@ hipError_t launch_dma_tile(const GemmArgs& a0, bool nn, int batch, hipStream_t s
 }
 
 // 16-bit operands that span 2^31 bytes or more
-bool dma_far(const GemmArgs& a, bool nn) {
-    const int64_t span_a = ((int64_t)(a.m - 1) * a.rsa + a.k) * 2;
-    const int64_t span_b = (nn ? (int64_t)(a.k - 1) * a.rsb + a.n : (int64_t)(a.n - 1) * a.csb + a.k) * 2;
+bool dma_far(int m, int n, int k, int64_t rsa, int64_t rsb, int64_t csb, bool nn) {
+    const int64_t span_a = ((int64_t)(m - 1) * rsa + k) * 2;
+    const int64_t span_b = (nn ? (int64_t)(k - 1) * rsb + n : (int64_t)(n - 1) * csb + k) * 2;
     return span_a >= (int64_t(1) << 31) || span_b >= (int64_t(1) << 31);
 }
+bool dma_far(const GemmArgs& a, bool nn) { return dma_far(a.m, a.n, a.k, a.rsa, a.rsb, a.csb, nn); }
 
 template <class T, class TO>
 hipError_t launch_dma(const GemmArgs& a, bool nn, int batch, hipStream_t s) {
@@ -1154,6 +1155,22 @@ bool skinny_nn_pays(int m, int n, int k, int batch) {
 
 bool aligned(const void* p, int bytes) { return (reinterpret_cast<uintptr_t>(p) % bytes) == 0; }
 
+// The operand forms that the aligned kernels take: A's rows in 16-byte chunks, B as [n][k]
+// rows (nt), as [k][n] rows in pieces of 4 (nn) or in 16-byte chunks (nn16).
+struct Forms {
+    bool a, nt, nn, nn16;
+};
+Forms forms_of(int es, int n, int k, const void* A, int64_t sa_b, int64_t rsa, int64_t csa, const void* B, int64_t sb_b,
+               int64_t rsb, int64_t csb) {
+    const int vec = 16 / es;
+    Forms f;
+    f.a = csa == 1 && rsa % vec == 0 && sa_b % vec == 0 && aligned(A, 16) && k % vec == 0;
+    f.nt = rsb == 1 && csb % vec == 0 && sb_b % vec == 0 && aligned(B, 16);
+    f.nn = !f.nt && csb == 1 && rsb % 4 == 0 && sb_b % 4 == 0 && n % 4 == 0 && aligned(B, 4 * es);
+    f.nn16 = f.nn && rsb % vec == 0 && sb_b % vec == 0 && n % vec == 0 && aligned(B, 16);
+    return f;
+}
+
 template <class T, class TO>
 int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int64_t rsa, int64_t csa,
                const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C, int64_t sc_b, int64_t rsc,
@@ -1164,12 +1181,9 @@ int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int6
     const bool plain = mask.kind == YTHIP_MASK_NONE;
     if (k == 0 || alpha == 0.0f) return status_of(launch_scale<TO>(C, m, n, rsc, csc, sc_b, beta, batch, s));
 
-    const int es = sizeof(raw);
-    const bool a_ok = csa == 1 && (rsa % VEC) == 0 && (sa_b % VEC) == 0 && aligned(A, 16) && (k % VEC) == 0;
-    const bool nt = rsb == 1 && (csb % VEC) == 0 && (sb_b % VEC) == 0 && aligned(B, 16);
-    const bool nn = !nt && csb == 1 && (rsb % 4) == 0 && (sb_b % 4) == 0 && (n % 4) == 0 && aligned(B, 4 * es);
-    const bool c_ok = csc == 1;
-    if (a_ok && (nt || nn) && c_ok) {
+    const Forms fo = forms_of(sizeof(raw), n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb);
+    const bool nt = fo.nt, nn = fo.nn;
+    if (fo.a && (nt || nn) && csc == 1) {
         GemmArgs g{};
         g.A = A; g.B = B; g.C = C;
         g.m = m; g.n = n; g.k = k;
@@ -1187,7 +1201,7 @@ int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int6
                 v.m = m; v.n = n; v.k = k; v.alpha = alpha; v.beta = beta;
                 return gemv_dispatch(0, T::code, TO::code, v, batch, s);
             }
-            if (m == 1 && (n % VEC) == 0 && (rsb % VEC) == 0 && (sb_b % VEC) == 0 && aligned(B, 16)) {
+            if (m == 1 && fo.nn16) {
                 auto tiles = [&](int cpr) { return (int64_t)((n + cpr * VEC - 1) / (cpr * VEC)) * batch; };
                 // >= 192 workgroups: (1, 3072, 1024) 8.0 us with 96 workgroups of 32
                 // columns, 7.1 us with 192 of 16 (XCD-remapped, lines shared in L2)
@@ -1208,14 +1222,13 @@ int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int6
             // 2..16 rows of a row-major, 16-bit B: the MFMA DMA path (one partial
             // 64-row tile per column tile) streams B at full width
             if constexpr (sizeof(raw) == 2)
-                if ((rsb % VEC) == 0 && (sb_b % VEC) == 0 && (n % VEC) == 0 && aligned(B, 16))
-                    return status_of(launch_dma<T, TO>(g, true, batch, s));
+                if (fo.nn16) return status_of(launch_dma<T, TO>(g, true, batch, s));
         }
         if constexpr (std::is_same_v<T, F32> && std::is_same_v<TO, F32>) {
             // fp32 on the DMA-staged fp32 MFMA kernel: 16-byte aligned rows of A and
             // of B (NT) or B's k-rows (NN). 1000^3: 37.8 us on the register-staged
             // kernel that took k % 32 != 0 before, 24.6 us here
-            const bool f_nn = nn && (rsb % 4) == 0 && (sb_b % 4) == 0 && aligned(B, 16) && n >= 4;
+            const bool f_nn = fo.nn16;
             if (nt || f_nn) {
                 auto ntiles = [&](int bm, int bn) { return (int64_t)((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batch; };
                 const bool big = ntiles(128, 128) >= 512;
@@ -1243,10 +1256,8 @@ int gemm_typed(int batch, int m, int n, int k, const void* A, int64_t sa_b, int6
         // DMA-staged fast path: 16-byte aligned rows everywhere, k in whole chunks
         // (k % 64 != 0, 4096 x 4096 x 4072 NN: 228 -> 119 us, 1000^3 17.3 -> 7.8 us
         // against the register-staged kernel that took those before).
-        const bool dma_nn = nn && es == 2 && (rsb % VEC) == 0 && (sb_b % VEC) == 0 && (n % VEC) == 0 &&
-                            aligned(B, 16);
         if constexpr (sizeof(raw) == 2)
-            if ((nt || dma_nn) && (plain || !dma_far(g, nn))) return status_of(launch_dma<T, TO>(g, nn, batch, s));
+            if ((nt || fo.nn16) && (plain || !dma_far(g, nn))) return status_of(launch_dma<T, TO>(g, nn, batch, s));
     }
     return gemm_any_dispatch(T::code, TO::code, batch, m, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb, C, sc_b, rsc, csc,
                              alpha, beta, mask, s);
@@ -1317,6 +1328,53 @@ int gemm_masked_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, i
 #undef YTHIP_GEMM
     return fail(YTHIP_EUNSUPPORTED, "ythip_gemm: unsupported dtype_in/dtype_out combination %d/%d", dtype_in,
                 dtype_out);
+}
+
+// Whether a masked product is faster with the mask in its store than as an fp32 product in
+// a workspace and a blend. What the store costs: it exists on 64- and 128-wide tiles only.
+//  * m <= 16 rows that the plain product gives to a GEMV kernel: the tile kernel walks k in one
+//    chain. 1 x 1024 x 8192 NT, store / workspace: bf16 30 / 16 us, fp32 154 / 16; at k = 1024
+//    bf16 10 / 15, fp32 22 / 16. Many columns fill the chip with tiles: bf16 16 x 8192 x 8192 NT 30 / 40.
+//  * 16-bit products of 192 and more 256 x 256 tiles: the plain one is the ping-pong kernel (1.54 us
+//    a 64-wide step and pass over the CUs, 128 x 128 tiles 0.656), against the blend's own
+//    bytes and blocks. bf16 4096^3 NN byte mask kept 152 / 137 us, filled 145 / 137; 8192^3 causal 1031 /
+//    898, bytes 1133 / 924; 4096 x 4096 x 1024 bytes 54 / 101. The constants are fitted to 940 products
+//    (k 256 to 8192, five mask shapes, kept and filled): none is slower than the workspace form.
+//    A diagonal's hidden tiles only help where the busiest XCD, which holds the last eighth of the
+//    rows (tile_coords), has some.
+//  * operands of 2^31 bytes and more have no masked DMA form; register-staged 64 x 64 tiles
+//    re-read both operands per tile (131200 x 256 x 8192 bytes 1092 / 818 us, one row or column
+//    of tiles 466 / 637).
+//  * aligned operands and a strided C: only the register-staged kernel stores it.
+bool gemm_masked_store_pays(int dtype_in, int batch, int m, int n, int k, const void* A, int64_t sa_b, int64_t rsa,
+                            int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, int64_t csc,
+                            const MaskDesc& mask) {
+    if (mask.kind == YTHIP_MASK_NONE) return true;
+    const bool f32 = dtype_in == YTHIP_F32;
+    const Forms f = forms_of(f32 ? 4 : 2, n, k, A, sa_b, rsa, csa, B, sb_b, rsb, csb);
+    if (!f.a || !(f.nt || f.nn16 || (f32 && f.nn))) return true;
+    if (m <= SKINNY_M && (f.nt || (m == 1 && f.nn16) || (f32 && skinny_nn_pays(m, n, k, batch))))
+        return f32 ? k <= 512 : k <= 2048 || (n > 4096 && !(m == 1 && f.nt));
+    if (csc != 1) return false;
+    if (f32) return true;
+    double share = 1.0;  // visible, of the last eighth of the rows
+    if (mask.kind == YTHIP_MASK_CAUSAL || mask.kind == YTHIP_MASK_DIAG) {
+        share = 0.0;
+        for (int t = 0; t < 16; ++t) {
+            const int64_t row = m - 1 - (int64_t)(m / 8) * t / 16;
+            share += std::max<int64_t>(0, std::min<int64_t>(n, row + mask.off + 1)) / (16.0 * n);
+        }
+    }
+    if (dma_far(m, n, k, rsa, rsb, csb, f.nn16)) return m <= 64 || n <= 64 || share < 0.7;
+    auto tiles = [&](int b) { return (int64_t)((m + b - 1) / b) * ((n + b - 1) / b) * batch; };
+    if (tiles(256) < 192) return true;
+    const double steps = (k + 63) / 64, cells = (double)batch * m * n;
+    const double blocks = (double)batch * m * std::min(8, (n + 255) / 256);
+    const double bytes = mask.kind == YTHIP_MASK_BOOL && mask.fill ? 0.6e-6 * cells : 0.0;
+    const double blend = 1.83e-6 * cells + 0.848e-3 * blocks + bytes;
+    const double store = mask.fill ? 3.3 : mask.kind == YTHIP_MASK_BOOL ? 8.24 : 3.7;  // kept bytes: entry by entry
+    return (tiles(128) + 255) / 256 * (0.656 * share * steps + store) <=
+           (tiles(256) + 255) / 256 * 1.54 * steps + blend;
 }
 
 int gemm_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, const void* A, int64_t sa_b,

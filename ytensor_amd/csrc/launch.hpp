@@ -23,7 +23,11 @@ int gemm_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, c
                   int64_t rsa, int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C,
                   int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, hipStream_t s);
 
-// The same where the mask shows C; k > 0, alpha != 0.
+// The same where the mask shows C; k > 0, alpha != 0. gemm_masked_store_pays: this is faster
+// than gemm_dispatch into fp32 and a blend.
+bool gemm_masked_store_pays(int dtype_in, int batch, int m, int n, int k, const void* A, int64_t sa_b, int64_t rsa,
+                            int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, int64_t csc,
+                            const MaskDesc& mask);
 int gemm_masked_dispatch(int dtype_in, int dtype_out, int batch, int m, int n, int k, const void* A, int64_t sa_b,
                          int64_t rsa, int64_t csa, const void* B, int64_t sb_b, int64_t rsb, int64_t csb, void* C,
                          int64_t sc_b, int64_t rsc, int64_t csc, float alpha, float beta, const MaskDesc& mask,

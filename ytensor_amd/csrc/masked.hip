@@ -18,7 +18,8 @@
 //
 // MI355X design: the masked product is the plain one with the mask in its store, and
 // without the tiles that a diagonal mask hides whole (2048^3 bf16 causal: 50.5 us with
-// the product in an fp32 workspace and a pass over it, 23.8 us here). MATH attention in
+// the product in an fp32 workspace and a pass over it, 23.8 us here); that pass stays for
+// what the store cannot take (masked_in_store). MATH attention in
 // the layouts of the MFMA attention kernels is one launch (attention.hip, MODE 4); the
 // passes here (scores in fp32, a softmax workgroup per row, weights in the input
 // type, a second product) serve the rest.
@@ -215,12 +216,15 @@ struct MaskedCall {
 
 // Whether the product's store applies the mask. Otherwise the fp32 product goes to the
 // workspace and a second launch blends it into C: a type of C that no product kernel
-// stores; a C over A or B, which other workgroups still read when tiles of C are stored.
+// stores; a C over A or B, which other workgroups still read when tiles of C are stored;
+// sizes that are faster so (gemm_masked_store_pays).
 bool masked_in_store(const MaskedCall& c) {
     if (c.dtype_out != c.dtype_in && c.dtype_out != YTHIP_F32) return false;
     const Span o = span_of(c.C, esize(c.dtype_out), {{c.batch, c.sc_b}, {c.m, c.rsc}, {c.n, c.csc}});
     return !overlap(o, span_of(c.A, esize(c.dtype_in), {{c.batch, c.sa_b}, {c.m, c.rsa}, {c.k, c.csa}})) &&
-           !overlap(o, span_of(c.B, esize(c.dtype_in), {{c.batch, c.sb_b}, {c.k, c.rsb}, {c.n, c.csb}}));
+           !overlap(o, span_of(c.B, esize(c.dtype_in), {{c.batch, c.sb_b}, {c.k, c.rsb}, {c.n, c.csb}})) &&
+           gemm_masked_store_pays(c.dtype_in, c.batch, c.m, c.n, c.k, c.A, c.sa_b, c.rsa, c.csa, c.B, c.sb_b, c.rsb,
+                                  c.csb, c.csc, c.mask);
 }
 
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
