@@ -310,13 +310,15 @@ def scaled_dot_product_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tens
         if backend == "math":
             tensors = (_code(q), B, Hq, Hkv, Sq, Skv, D, dv, qt.data_ptr(), i64array(qs), kt.data_ptr(), i64array(ks),
                        vt.data_ptr(), i64array(vs), ot.data_ptr(), i64array(os_))
-            need = int(_lib.lib().ythip_attn_math_workspace_needed(*tensors, kind, mptr, mld, bptr, brs, bcs))
-            ws = workspace
-            if need and (ws is None or ws.numel() * ws.element_size() < need):
-                ws = torch.empty(need, dtype=torch.uint8, device=q.device)
+            ws, need = workspace, 0
+            if ws is not None:  # enough for any call?
+                need = int(_lib.lib().ythip_attn_math_workspace_size(_code(q), B, Hq, Sq, Skv))
+            if ws is None or ws.numel() * ws.element_size() < need:
+                need = int(_lib.lib().ythip_attn_math_workspace_needed(*tensors, kind, mptr, mld, bptr, brs, bcs))
+                ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
             st = _lib.lib().ythip_attn_math(
                 *tensors, float(scale), kind, mptr, mld, bptr, brs, bcs,
-                ws.data_ptr() if need else None, need, _stream())
+                None if ws is None else ws.data_ptr(), need, _stream())
             check(st, "ythip_attn_math")
         elif kind == _lib.MASK_BOOL or Sq == 1:
             # room for the mask's tile classes (the long-sequence path lists the
@@ -398,12 +400,12 @@ def gemm_masked(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor, mask, alpha
                 Bm.data_ptr(), 0 if Bm.shape[0] == 1 else Bm.stride(0), Bm.stride(1), Bm.stride(2),
                 C.data_ptr(), C.stride(0), C.stride(1), C.stride(2), float(alpha))
     filled = int(fill is not None)
-    need = int(_lib.lib().ythip_gemm_masked_workspace_needed(*operands, kind, mld, filled))
-    ws = workspace
-    if need and (ws is None or ws.numel() * ws.element_size() < need):
-        ws = torch.empty(need, dtype=torch.uint8, device=a.device)
+    ws, need = workspace, 4 * bt * m * n  # what any call takes
+    if ws is None or ws.numel() * ws.element_size() < need:
+        need = int(_lib.lib().ythip_gemm_masked_workspace_needed(*operands, kind, mld, filled))
+        ws = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
     st = _lib.lib().ythip_gemm_masked(*operands, float(beta), kind, mptr, mld, filled, float(fill or 0.0),
-                                      ws.data_ptr() if need else None, need, _stream())
+                                      None if ws is None else ws.data_ptr(), need, _stream())
     check(st, "ythip_gemm_masked")
     return out
 
