@@ -1129,7 +1129,12 @@ hipError_t launch_dma(const GemmArgs& a, bool nn, int batch, hipStream_t s) {
     // (weights from HBM 13.8 / 16.4), 512 x 4096 x 1024 NT 9.5 / 9.6 (10.3 / 12.0), 2048 x
     // 1024 x 3072 NT 23.4 / 24.6 (25.1 / 29.5). A ring deeper than 4 steps loses at
     // every size (512 x 1024 x 3072: 13.6, 8 deep 14.8, 12 deep 17.6 us).
-    const int64_t c0 = cost(64, 32), c1 = cost(64, 64), c2 = cost(128, 64), c3 = cost(128, 128), c4 = cost(256, 128);
+    const int64_t c0 = cost(64, 32), c1 = cost(64, 64), c2 = cost(128, 64), c3 = cost(128, 128);
+    // The 256-wide tiles of a small matrix in a batch share little of the XCDs' L2s, and lose
+    // more by it than the smaller ones do: 256 x 128 / 128 x 128 NT at 32 tiles a matrix (8 x 1024 x 1024 x
+    // 1024) 26.3 / 20.5 us, at 60 (4 x 1280 x 1536 x 640) 15.4 / 14.4, at 72 (3 x 1500 x 1500 x 1504)
+    // 26.6 / 28.4, at 100 (2 x 2560 x 1280 x 1280) 20.8 / 22.2.
+    const int64_t c4 = batch == 1 || tiles(256, 128) >= 72 * (int64_t)batch ? cost(256, 128) : INT64_MAX;
     const int64_t best = std::min(std::min(std::min(c0, c1), std::min(c2, c3)), c4);
     if (c0 == best) return launch_dma_tile<T, TO, 64, 32, 2, 1, 4>(a, nn, batch, s);
     if (c1 == best) return launch_dma_tile<T, TO, 64, 64, 2, 2, 4>(a, nn, batch, s);
