@@ -117,31 +117,40 @@ struct GemvPrologue {
             for (int j = 0; j < 4; ++j) xr[j] = (tid < 256 && tid + 256 * j < a.k) ? X[tid + 256 * j] : 0.f;
         }
         if constexpr (PRO == 3) {
-            const int S = a.splits, stride = a.hd + 2;
             // The split kernel's partition (decode_used). The first SPEC splits are loaded
-            // without waiting for it, the others only where they hold keys: a short
-            // context in a large ring reads a quarter of the bytes (each of the 64
-            // workgroups reads all of them). Qwen3-0.6B decode, 4096-row ring: up to 256 keys
-            // 740 -> 720 us a token, 512 keys 753 -> 749, 1000 keys (all 8 in use) 764 -> 767.
-            used = a.dstate != nullptr ? decode_used(max(0, min(a.dstate[YTHIP_ST_KV_LEN], a.max_ctx)), S) : S;
-            const float* src[2];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) src[j] = merge_src(a, bz, tid + j * NT < total ? tid + j * NT : 0);
-            const bool owner = tid < a.m * a.hq;
-            const float* msrc = merge_msrc(a, bz, owner ? tid : 0);
-            auto take = [&](int q, bool on) {
-#pragma unroll
-                for (int j = 0; j < 2; ++j) opre[j][q] = (on && tid + j * NT < total) ? src[j][q * stride] : 0.f;
-                mreg[q] = (on && owner) ? msrc[q * stride] : -INFINITY;
-                lreg[q] = (on && owner) ? msrc[q * stride + 1] : 0.f;
-            };
-#pragma unroll
-            for (int q = 0; q < SPEC; ++q) take(q, q < S);
-            if (used > SPEC) {
-#pragma unroll
-                for (int q = SPEC; q < MS; ++q) take(q, q < used);
-            }
+            // without waiting for it, the others only where they hold keys, and after the first
+            // weights (load_rest): a short context in a large ring reads a quarter of the bytes (each
+            // of the 64 workgroups reads all of them), and a long one does not hold the weights
+            // up while it waits for the count. Qwen3-0.6B decode, 4096-row ring, us a token with
+            // all 8 loaded here / as it is / with the others here behind the count: 16 keys 739 /
+            // 718 / 718, 250 keys 743 / 726 / 730, 500 keys 748 / 738 / 741, 900 keys 754 / 753 / 757,
+            // 1000 keys 769 / 772 / 773, 3900 keys 1444 / 1446 / 1448.
+            used = a.dstate != nullptr ? decode_used(max(0, min(a.dstate[YTHIP_ST_KV_LEN], a.max_ctx)), a.splits) : a.splits;
+            take<0, SPEC>(a, bz, a.splits);
         }
+    }
+    // merge: this thread's part of splits Q0 .. Q1 - 1, those below `upto`
+    template <int Q0, int Q1>
+    __device__ __forceinline__ void take(const GemvArgs& a, int bz, int upto) {
+        const int tid = threadIdx.x, total = a.m * a.k, stride = a.hd + 2;
+        const float* src[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) src[j] = merge_src(a, bz, tid + j * NT < total ? tid + j * NT : 0);
+        const bool owner = tid < a.m * a.hq;
+        const float* msrc = merge_msrc(a, bz, owner ? tid : 0);
+#pragma unroll
+        for (int q = Q0; q < Q1; ++q) {
+            const bool on = q < upto;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) opre[j][q] = (on && tid + j * NT < total) ? src[j][q * stride] : 0.f;
+            mreg[q] = (on && owner) ? msrc[q * stride] : -INFINITY;
+            lreg[q] = (on && owner) ? msrc[q * stride + 1] : 0.f;
+        }
+    }
+    // After the first weight loads.
+    __device__ __forceinline__ void load_rest(const GemvArgs& a, int bz) {
+        if constexpr (PRO == 3)
+            if (used > SPEC) take<SPEC, MS>(a, bz, used);
     }
 
     __device__ __forceinline__ void build(const GemvArgs& a, int bz, raw* sAp) {
@@ -314,13 +323,14 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvArgs a) {
             return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wrp + (int64_t)s * KSTEP));
         return u32x4{0u, 0u, 0u, 0u};
     };
-    // Latency plan: the prologue's loads, then the first round of weight loads,
-    // then the epilogue's, all before anything waits on memory.
+    // Latency plan: the prologue's loads, then the first round of weight loads (and the
+    // merge's other splits), then the epilogue's, all before anything waits on memory.
     GemvPrologue<T, 64 * WAVES, PRO> pro;
     if constexpr (PRO != 0) pro.load(a, bz);
     u32x4 fb[UNR];
 #pragma unroll
     for (int u = 0; u < UNR; ++u) fb[u] = load_w(s_begin + u);
+    pro.load_rest(a, bz);
 
     using oraw = typename TO::raw;
     oraw* crow = static_cast<oraw*>(a.C) + bz * a.sc_b + (int64_t)r * a.ldc;
@@ -493,6 +503,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_row_kernel(GemvArgs a) {
     if constexpr (PRO != 0) pro.load(a, 0);
     u32x4 w[RPW][CPL];
     load_round(0, w);
+    pro.load_rest(a, 0);
 
     using oraw = typename TO::raw;
     oraw* Cp = static_cast<oraw*>(a.C);
