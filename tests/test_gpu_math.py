@@ -285,8 +285,9 @@ def test_sdpa_math_one_launch(yt, dev, Sq, Skv, D, dt):
     """The one-launch MATH kernels against float64 at the edges of their 64-query and
     64- / 128-key blocks, every mask kind, GQA 2:1. Beside ordinary scales: a
     negative one and one of 1e-8 (hidden keys keep weight), a bias that lifts
-    hidden keys back up. Bound: 32-bit arithmetic on scores up to 8 (1e-5 of the
-    values' size) and in 16 bits the rounding of the weights and the result."""
+    hidden keys back up (at a scale of 2^-20, where -1e9 scale is exact in fp32 and cancels
+    exactly against a bias of 1e9 scale plus eighths). Bound: 32-bit arithmetic on scores up
+    to 8 (1e-5 of the values' size) and in 16 bits the rounding of the weights and the result."""
     g = torch.Generator(device=dev).manual_seed(Sq + Skv + D)
     q = torch.randn(2, 4, Sq, D, device=dev, generator=g).to(dt)
     k = torch.randn(2, 2, Skv, D, device=dev, generator=g).to(dt)
@@ -295,10 +296,12 @@ def test_sdpa_math_one_launch(yt, dev, Sq, Skv, D, dt):
     drop = torch.rand(Sq, Skv, device=dev, generator=g) < 0.4
     drop[Sq // 2] = True
     bias = torch.randn(Sq, Skv, device=dev, generator=g)
-    lift = torch.where(drop, torch.full_like(bias, 1e9 / D ** 0.5), bias)
+    eighths = torch.randint(-16, 17, (Sq, Skv), device=dev, generator=g).float() / 8
+    lift = torch.where(drop, 1e9 * 2.0 ** -20 + eighths, bias)
+    assert torch.equal(lift.double()[drop], (1e9 * 2.0 ** -20 + eighths.double())[drop])
     cases = [(None, None, 0.0, None), ("causal", j <= i + Skv - Sq, 0.0, None), (("diag", -3), j <= i - 3, 0.0, None),
              (~drop, ~drop, 0.0, None), (~drop, ~drop, 0.0, bias), ("causal", j <= i + Skv - Sq, 1e-8, None),
-             (~drop, ~drop, -1e-9, None), (~drop, ~drop, 0.0, lift)]
+             (~drop, ~drop, -1e-9, None), (~drop, ~drop, 2.0 ** -20, lift)]
     ulp = {torch.float32: 2e-7, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dt]
     for mask, vis, scale, bs in cases:
         out = yt.scaled_dot_product_attention(q, k, v, scale, mask=mask, bias=bs, backend="math")
@@ -306,8 +309,6 @@ def test_sdpa_math_one_launch(yt, dev, Sq, Skv, D, dt):
             want = _math64(q[b], k[b], v[b], scale or 1.0 / D ** 0.5, vis, bs)
             top = float(v.double().abs().max())
             bound = (1e-5 + ulp) * top + 2 * ulp * want.abs()
-            if bs is lift:  # -1e9 scale + 1e9 / sqrt(d) cancels to the size of a float's ulp at 1e8
-                continue
             assert ((out[b].double() - want).abs() <= bound).all(), (scale, bs is not None)
         assert torch.isfinite(out).all()
     if Skv >= 63 and Sq > 1:
@@ -345,8 +346,8 @@ def test_gemm_masked_layouts(yt, dev, m, n, k, layout, dt):
             yt.gemm_masked(A, B, C, mask, alpha, beta, fill)
             want = alpha * prod + beta * C0
             bound = (k + 2) * 2.0 ** -24 * mass + ulp * want.abs() + 4 * 2.0 ** -23 * C0.abs() + 1e-7
-            off = ((C.double() - want).abs() > bound) & vis
-            assert not off.any(), (mask if isinstance(mask, (str, tuple)) else "bytes", alpha, fill)
+            ok = (C.double() - want).abs() <= bound  # (false for a NaN)
+            assert ok[vis.expand(2, m, n)].all(), (mask if isinstance(mask, (str, tuple)) else "bytes", alpha, fill)
             hid = (~vis).expand(2, m, n)
             assert torch.equal(C.double()[hid], (C0 if fill is None else torch.full_like(C0, fill))[hid])
 
