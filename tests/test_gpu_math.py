@@ -435,3 +435,32 @@ def test_gemm_masked_output_over_an_input(yt, dev, where, dt):
     yt.gemm_masked(a, b, c, vis)
     assert ((c.double() - prod).abs() <= (n + 2) * 2.0 ** -24 * mass + ulp * prod.abs())[vis].all()
     assert torch.equal(c[~vis], c0[~vis])
+
+
+@pytest.mark.parametrize("dt,nt,m,n,k", [(torch.bfloat16, False, 3584, 3592, 3072), (torch.float16, True, 3600, 3584, 4104),
+                                         (torch.bfloat16, True, 1, 1000, 4096), (torch.bfloat16, True, 16, 1024, 8192),
+                                         (torch.bfloat16, False, 1, 1024, 8192), (torch.float32, True, 7, 1000, 1024),
+                                         (torch.float32, False, 1, 1024, 1000), (torch.float32, False, 3, 1004, 2048)])
+def test_gemm_masked_through_the_workspace(yt, dev, dt, nt, m, n, k):
+    """Sizes that run as an fp32 product in the workspace and a blend (256-wide tiles with a
+    long k, few rows), with a contiguous and a strided C, each mask kind, kept and filled,
+    against float64 as in test_gemm_masked_layouts."""
+    g = torch.Generator(device=dev).manual_seed(m + n + k)
+    A = torch.randn(m, k, device=dev, generator=g).to(dt)
+    B = torch.randn(n, k, device=dev, generator=g).to(dt).t() if nt else torch.randn(k, n, device=dev, generator=g).to(dt)
+    prod = A.double() @ B.double().contiguous()
+    mass = A.double().abs() @ B.double().abs().contiguous()
+    i, j = torch.arange(m, device=dev)[:, None], torch.arange(n, device=dev)[None, :]
+    bytes_ = torch.rand(m, n, device=dev, generator=g) < 0.5
+    ulp = {torch.float32: 2.0 ** -23, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -10}[dt]
+    for mask, vis in [("causal", j <= i + n - m), (("diag", 5), j <= i + 5), (bytes_, bytes_)]:
+        for alpha, beta, fill, step in [(1.0, 0.0, -3.0, 1), (0.5, 2.0, None, 1), (1.0, 0.0, None, 2)]:
+            C = torch.randn(m, step * n, device=dev, generator=g).to(dt)[:, ::step]
+            C0 = C.double()
+            yt.gemm_masked(A, B, C, mask, alpha, beta, fill)
+            want = alpha * prod + beta * C0
+            bound = (k + 2) * 2.0 ** -24 * mass + ulp * want.abs() + 4 * 2.0 ** -23 * C0.abs() + 1e-7
+            ok = (C.double() - want).abs() <= bound
+            assert ok[vis.expand(m, n)].all(), (mask if isinstance(mask, (str, tuple)) else "bytes", alpha, fill)
+            hid = (~vis).expand(m, n)
+            assert torch.equal(C.double()[hid], (C0 if fill is None else torch.full_like(C0, fill))[hid])
