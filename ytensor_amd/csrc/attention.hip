@@ -407,113 +407,113 @@ __global__ __launch_bounds__(256 * GH * KSPLIT, 2 / (GH * KSPLIT)) void attn_fwd
 #pragma unroll
                 for (int kk = 0; kk < NKT / 2; ++kk) pk[qt][kk] = u32x4{0u, 0u, 0u, 0u};
         } else {
-        float lmax[QT];
-        bool trig = false;
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-            const int qa = q0 + qt * 16 + l16;
-            if constexpr (MODE == 4) {
-                if (!need_mask) {
-#pragma unroll
-                    for (int kt = 0; kt < NKT; ++kt) s[qt][kt] *= c;
-                } else {
-                    const bool diag = a.mask == nullptr && a.bias == nullptr && k0 + BKV <= a.Skv;
-#pragma unroll
-                    for (int kt = 0; kt < NKT; ++kt) {
-                        const int key = k0 + kt * 16 + g * 4;
-                        if (diag) math_scores4_diag(a, s[qt][kt], qa, key);
-                        else math_scores4(a, s[qt][kt], min(qa, a.Sq - 1), qa, key, seen[qt]);
-                    }
-                }
-            } else if (need_mask) {
-#pragma unroll
-                for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        float x = s[qt][kt][r];
-                        const int key = k0 + kt * 16 + g * 4 + r;
-                        bool vis = key < a.Skv;
-                        if (MODE == 1) vis = vis && (key <= qa + off);
-                        if (MODE == 3) {
-                            if (staged) {
-                                const uint32_t w = reinterpret_cast<const uint32_t*>(sM + mslot(kb) * MSTG)
-                                    [((qa - qb * BQ) * BKV + kt * 16 + g * 4) >> 2];
-                                vis = ((w >> (8 * r)) & 0xffu) != 0u;
-                            } else if (vis && qa < a.Sq) {
-                                vis = a.mask[(int64_t)qa * a.mask_ld + key] != 0;
-                            }
-                        }
-                        if (MODE == 2 && vis && qa < a.Sq) {
-                            if (a.mask != nullptr) vis = a.mask[(int64_t)qa * a.mask_ld + key] != 0;
-                            // bias is added after scaling: log2 units, like the scores
-                            if (vis && a.bias != nullptr)
-                                x += a.bias[(int64_t)qa * a.brs + (int64_t)key * a.bcs] * LOG2E;
-                        }
-                        s[qt][kt][r] = vis ? x : -INFINITY;
-                    }
-            }
-            // IEEE maximum (NaN-propagating) instead of fmaxf: gfx950's v_maximum3_f32
-            // takes the MFMA results as they are, where fmaxf first canonicalises
-            // every input (one extra VALU op per score); same value for any non-NaN row
-            float mx = -INFINITY;
-#pragma unroll
-            for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) mx = __builtin_elementwise_maximum(mx, s[qt][kt][r]);
-            lmax[qt] = mx;
-            // the reference point of a row moves (set on its first visible block,
-            // afterwards only for a block max far above it) iff one of its lanes sees this
-            if constexpr (MODE == 4) trig = trig || mx - m[qt] > thr[qt];
-            else trig = trig || mx > thr[qt];
-        }
-        auto exps = [&]() {
-#pragma unroll
-            for (int qt = 0; qt < QT; ++qt)
-#pragma unroll
-                for (int kk = 0; kk < NKT / 2; ++kk) {
-                    float e[8];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        // MODE 4 keeps the scores themselves: next to a hidden key's
-                        // -1e9, s - m would lose a visible score's digits
-                        const float z = MODE == 4 ? m[qt] : 0.f;
-                        e[r] = __builtin_amdgcn_exp2f(s[qt][2 * kk][r] - z);
-                        e[4 + r] = __builtin_amdgcn_exp2f(s[qt][2 * kk + 1][r] - z);
-                    }
-                    pk[qt][kk] = u32x4{pack2<T>(e[0], e[1]), pack2<T>(e[2], e[3]), pack2<T>(e[4], e[5]),
-                                       pack2<T>(e[6], e[7])};
-                }
-        };
-        // p = 2^(s - m) with the current m, issued without waiting for the test;
-        // final unless some row's reference point moves in this block.
-        exps();
-        if (__ballot(trig) != 0) {
-            // Rare: full row max (the row's 16-lane groups), move m, rescale O
-            // and l, exps again -- the same values as deciding before the exps.
+            float lmax[QT];
+            bool trig = false;
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) {
-                float mx = lmax[qt];
-                mx = __builtin_elementwise_maximum(mx, __shfl_xor(mx, 16, 64));
-                mx = __builtin_elementwise_maximum(mx, __shfl_xor(mx, 32, 64));
-                const float top = mx;
-                if constexpr (MODE == 4) mx -= m[qt];
-                const bool move = mset[qt] ? (mx > LAZY) : (mx != -INFINITY);
-                const float delta = move ? mx : 0.f;
-                const float alpha = (move && mset[qt]) ? __builtin_amdgcn_exp2f(-delta) : 1.0f;
-                if constexpr (MODE == 4) m[qt] = move ? top : m[qt];
-                else m[qt] += delta;
-                mset[qt] = mset[qt] || move;
-                thr[qt] = mset[qt] ? LAZY : -INFINITY;
+                const int qa = q0 + qt * 16 + l16;
+                if constexpr (MODE == 4) {
+                    if (!need_mask) {
+#pragma unroll
+                        for (int kt = 0; kt < NKT; ++kt) s[qt][kt] *= c;
+                    } else {
+                        const bool diag = a.mask == nullptr && a.bias == nullptr && k0 + BKV <= a.Skv;
+#pragma unroll
+                        for (int kt = 0; kt < NKT; ++kt) {
+                            const int key = k0 + kt * 16 + g * 4;
+                            if (diag) math_scores4_diag(a, s[qt][kt], qa, key);
+                            else math_scores4(a, s[qt][kt], min(qa, a.Sq - 1), qa, key, seen[qt]);
+                        }
+                    }
+                } else if (need_mask) {
+#pragma unroll
+                    for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            float x = s[qt][kt][r];
+                            const int key = k0 + kt * 16 + g * 4 + r;
+                            bool vis = key < a.Skv;
+                            if (MODE == 1) vis = vis && (key <= qa + off);
+                            if (MODE == 3) {
+                                if (staged) {
+                                    const uint32_t w = reinterpret_cast<const uint32_t*>(sM + mslot(kb) * MSTG)
+                                        [((qa - qb * BQ) * BKV + kt * 16 + g * 4) >> 2];
+                                    vis = ((w >> (8 * r)) & 0xffu) != 0u;
+                                } else if (vis && qa < a.Sq) {
+                                    vis = a.mask[(int64_t)qa * a.mask_ld + key] != 0;
+                                }
+                            }
+                            if (MODE == 2 && vis && qa < a.Sq) {
+                                if (a.mask != nullptr) vis = a.mask[(int64_t)qa * a.mask_ld + key] != 0;
+                                // bias is added after scaling: log2 units, like the scores
+                                if (vis && a.bias != nullptr)
+                                    x += a.bias[(int64_t)qa * a.brs + (int64_t)key * a.bcs] * LOG2E;
+                            }
+                            s[qt][kt][r] = vis ? x : -INFINITY;
+                        }
+                }
+                // IEEE maximum (NaN-propagating) instead of fmaxf: gfx950's v_maximum3_f32
+                // takes the MFMA results as they are, where fmaxf first canonicalises
+                // every input (one extra VALU op per score); same value for any non-NaN row
+                float mx = -INFINITY;
 #pragma unroll
                 for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
-                    for (int r = 0; r < 4 && MODE != 4; ++r) s[qt][kt][r] -= delta;
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) o[qt][dt] *= alpha;
-                lsum[qt] *= alpha;
+                    for (int r = 0; r < 4; ++r) mx = __builtin_elementwise_maximum(mx, s[qt][kt][r]);
+                lmax[qt] = mx;
+                // the reference point of a row moves (set on its first visible block,
+                // afterwards only for a block max far above it) iff one of its lanes sees this
+                if constexpr (MODE == 4) trig = trig || mx - m[qt] > thr[qt];
+                else trig = trig || mx > thr[qt];
             }
+            auto exps = [&]() {
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+                    for (int kk = 0; kk < NKT / 2; ++kk) {
+                        float e[8];
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            // MODE 4 keeps the scores themselves: next to a hidden key's
+                            // -1e9, s - m would lose a visible score's digits
+                            const float z = MODE == 4 ? m[qt] : 0.f;
+                            e[r] = __builtin_amdgcn_exp2f(s[qt][2 * kk][r] - z);
+                            e[4 + r] = __builtin_amdgcn_exp2f(s[qt][2 * kk + 1][r] - z);
+                        }
+                        pk[qt][kk] = u32x4{pack2<T>(e[0], e[1]), pack2<T>(e[2], e[3]), pack2<T>(e[4], e[5]),
+                                           pack2<T>(e[6], e[7])};
+                    }
+            };
+            // p = 2^(s - m) with the current m, issued without waiting for the test;
+            // final unless some row's reference point moves in this block.
             exps();
-        }
+            if (__ballot(trig) != 0) {
+                // Rare: full row max (the row's 16-lane groups), move m, rescale O
+                // and l, exps again -- the same values as deciding before the exps.
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt) {
+                    float mx = lmax[qt];
+                    mx = __builtin_elementwise_maximum(mx, __shfl_xor(mx, 16, 64));
+                    mx = __builtin_elementwise_maximum(mx, __shfl_xor(mx, 32, 64));
+                    const float top = mx;
+                    if constexpr (MODE == 4) mx -= m[qt];
+                    const bool move = mset[qt] ? (mx > LAZY) : (mx != -INFINITY);
+                    const float delta = move ? mx : 0.f;
+                    const float alpha = (move && mset[qt]) ? __builtin_amdgcn_exp2f(-delta) : 1.0f;
+                    if constexpr (MODE == 4) m[qt] = move ? top : m[qt];
+                    else m[qt] += delta;
+                    mset[qt] = mset[qt] || move;
+                    thr[qt] = mset[qt] ? LAZY : -INFINITY;
+#pragma unroll
+                    for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+                        for (int r = 0; r < 4 && MODE != 4; ++r) s[qt][kt][r] -= delta;
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) o[qt][dt] *= alpha;
+                    lsum[qt] *= alpha;
+                }
+                exps();
+            }
         }
         const u32x4* cV = sV + (kb & 1) * STG + grp * BKV * KCH;
 #pragma unroll

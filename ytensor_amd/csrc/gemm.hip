@@ -9,10 +9,12 @@
 //    B[k][n]) stays [k][n] in LDS and its fragments are read with the gfx950
 //    transposing read ds_read_b64_tr_b16, so nothing is transposed in registers.
 //  * Tiles move global -> LDS by direct-to-LDS DMA (global_load_lds_dwordx4):
-//    no VGPR staging. Two stages for the 256 x 256 tile (one k step in flight),
-//    a 4-deep ring for the smaller tiles. The bytes each CU can pull through its
-//    vector-memory path (~28 B/clk) are close to what 256 x 256 MFMA work
-//    consumes, so the 256 x 256 tile is the only one that keeps up at 4096^3.
+//    no VGPR staging. Two stages where the tile fills the LDS (256 x 256) or two
+//    workgroups share a CU (128 x 128 of four waves), three at 256 x 128 and 128 x 64,
+//    a 4-deep ring for 64 x 64, 64 x 32 and the one-per-CU 128 x 128 of eight waves. The
+//    bytes each CU can pull through its vector-memory path (~28 B/clk) are close to what
+//    256 x 256 MFMA work consumes, so the 256 x 256 tile is the only one that keeps up
+//    at 4096^3.
 //  * LDS swizzles were chosen by measuring gfx950's LDS read rate per pattern
 //    (see swz_dma / nn_blk): fragment reads are bank-conflict free.
 //  * Inside a k step the A fragments stream through a 3-register ring read two
