@@ -16,7 +16,7 @@ the kernels are launched on):
                   causal mask as bytes, and fp32 (the reference flash backend's dtype)
   attn_decode     configs[3] decode attention (GB/s of K/V read)
   rmsnorm_rope    fused RMSNorm+RoPE on configs[2] shapes at S=8192 (GB/s)
-  attn_math       the MATH attention backend (materialised scores) at S=2048, and
+  attn_math       the MATH attention backend at S=2048, and
                   a causal masked matmul at 4096^3
   qwen3_0p6b      configs[4] shape: 512-token prefill + greedy decode tok/s (a KV
                   ring sized to the run, and the reference's max_position_embeddings

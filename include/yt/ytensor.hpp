@@ -43,7 +43,7 @@
 // names a CPU implementation (Naive, Eigen, AVX2, FLASH_AVX2) runs the HIP
 // kernels too -- a call site such as the Qwen3 example's attention, which asks
 // for FLASH_AVX2 (example/qwen3/src/qwen3.cpp:256-264), needs no edit. MATH
-// runs the materialised-score path (ythip_attn_math).
+// runs ythip_attn_math (the scores in memory only where one launch does not take the call).
 //
 // Compile with a C++20 host compiler, -I<repo>/include -I/opt/rocm/include
 // -D__HIP_PLATFORM_AMD__, and link libythip.so and libamdhip64.so.
