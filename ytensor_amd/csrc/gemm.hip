@@ -10,8 +10,9 @@
 //    transposing read ds_read_b64_tr_b16, so nothing is transposed in registers.
 //  * Tiles move global -> LDS by direct-to-LDS DMA (global_load_lds_dwordx4):
 //    no VGPR staging. Two stages where the tile fills the LDS (256 x 256) or two
-//    workgroups share a CU (128 x 128 of four waves), three at 256 x 128 and 128 x 64,
-//    a 4-deep ring for 64 x 64, 64 x 32 and the one-per-CU 128 x 128 of eight waves. The
+//    workgroups share a CU (128 x 128 of four waves), three at 256 x 128 and where two 128 x 64
+//    share one, a 4-deep ring for 64 x 64, 64 x 32 and the one-per-CU 128 x 64 and 128 x 128 of
+//    eight waves. The
 //    bytes each CU can pull through its vector-memory path (~28 B/clk) are close to what
 //    256 x 256 MFMA work consumes, so the 256 x 256 tile is the only one that keeps up
 //    at 4096^3.
@@ -1127,9 +1128,9 @@ hipError_t launch_dma(const GemmArgs& a, bool nn, int batch, hipStream_t s) {
     // stages: passes over the 256 CUs times BM + BN rows a k step. The smallest wins,
     // the smaller tile when even (its ramp is shorter). Measured on bf16, the rule's
     // tile against the one of a rule by tile counts that stood here: 2048^3 NN 24.0 /
-    // 31.3 us, 2400^3 40.5 / 62.9, 1536^3 16.2 / 19.1, 512 x 6144 x 1024 NT 12.2 / 12.8
-    // (weights from HBM 13.8 / 16.4), 512 x 4096 x 1024 NT 9.5 / 9.6 (10.3 / 12.0), 2048 x
-    // 1024 x 3072 NT 23.4 / 24.6 (25.1 / 29.5). A ring deeper than 4 steps loses at
+    // 31.3 us, 2400^3 40.5 / 62.9, 1536^3 16.2 / 19.1, 2048 x 1024 x 3072 NT 23.4 / 24.6
+    // (weights from HBM 25.1 / 29.5); as graph nodes 512 x 6144 x 1024 NT 10.9 / 10.1 (12.8 / 15.1),
+    // 512 x 4096 x 1024 NT 8.3 / 8.0 (9.7 / 11.0). A ring deeper than 4 steps loses at
     // every size (512 x 1024 x 3072: 13.6, 8 deep 14.8, 12 deep 17.6 us).
     const int64_t c0 = cost(64, 32), c1 = cost(64, 64), c2 = cost(128, 64), c3 = cost(128, 128);
     // The 256-wide tiles of a small matrix in a batch share little of the XCDs' L2s, and lose
@@ -1140,7 +1141,14 @@ hipError_t launch_dma(const GemmArgs& a, bool nn, int batch, hipStream_t s) {
     const int64_t best = std::min(std::min(std::min(c0, c1), std::min(c2, c3)), c4);
     if (c0 == best) return launch_dma_tile<T, TO, 64, 32, 2, 1, 4>(a, nn, batch, s);
     if (c1 == best) return launch_dma_tile<T, TO, 64, 64, 2, 2, 4>(a, nn, batch, s);
-    if (c2 == best) return launch_dma_tile<T, TO, 128, 64, 2, 2, 3>(a, nn, batch, s);
+    if (c2 == best) {
+        // one per CU: eight waves and a deep ring, as four waves with two steps in flight leave
+        // the CU waiting. Two resident 64 x 64 tiles / one 128 x 64 of four waves / of eight, NT, weights
+        // from HBM: 200 x 6144 x 1024 10.1 / 10.2 / 8.8 us, 448 x 4096 x 1024 11.0 / 10.2 / 9.0; weights that
+        // stay cached: 7.2 / 8.8 / 7.9 and 7.6 / 9.1 / 8.2
+        if (tiles(128, 64) <= 256) return launch_dma_tile<T, TO, 128, 64, 4, 2, 4>(a, nn, batch, s);
+        return launch_dma_tile<T, TO, 128, 64, 2, 2, 3>(a, nn, batch, s);
+    }
     if (c3 == best) {
         // one per CU: eight waves and a deep ring; several: two resident per CU
         // (3072^3: 75.9 us, 80.2 with the deep ring)
