@@ -115,8 +115,11 @@ __global__ __launch_bounds__(64 * W) void attn_any_kernel(AttnArgs a) {
     // the mask word of four keys is read where it fits; without a mask, or with
     // fewer keys than four, a constant stands in for it
     const bool words = a.mask != nullptr && a.Skv >= 4;
-    const uint8_t* mrow =
-        words ? a.mask + (int64_t)qr * a.mask_ld : reinterpret_cast<const uint8_t*>(&no_mask_word);
+    // (in the global address space by name: the choice of two origins would be read by flat
+    // loads, which wait for every load in flight -- bf16, d = 128, 2048 keys 76 us, 84 flat)
+    using global_word = const __attribute__((address_space(1))) u32_any*;
+    using global_byte = const __attribute__((address_space(1))) uint8_t*;
+    const global_byte mrow = words ? (global_byte)(a.mask + (int64_t)qr * a.mask_ld) : (global_byte)&no_mask_word;
 
     // One block's operands. The next block's K is loaded as soon as the scores have
     // used this one's, its V after the output product: each load has the other
@@ -133,7 +136,7 @@ __global__ __launch_bounds__(64 * W) void attn_any_kernel(AttnArgs a) {
         const int k0 = first_key(i);
 #pragma unroll
         for (int kt = 0; kt < NKT; ++kt)
-            mw[kt] = *reinterpret_cast<const u32_any*>(mrow + (words ? min(k0 + 16 * kt + 4 * g, a.Skv - 4) : 0));
+            mw[kt] = *(global_word)(mrow + (words ? min(k0 + 16 * kt + 4 * g, a.Skv - 4) : 0));
 #pragma unroll
         for (int kt = 0; kt < NKT; ++kt) {
             const int64_t row = ko + (int64_t)min(k0 + 16 * kt + r, a.Skv - 1) * a.ks2;
