@@ -981,3 +981,25 @@ def test_prefill_any_layout_long_keys(yt, Skv, layout):
     vis = torch.arange(Skv, device="cuda")[None, :] <= torch.arange(Sq, device="cuda")[:, None] + off
     want = _sdpa64(q[0], k[0], v[0], 1.0 / math.sqrt(D), vis, bias)
     assert ((out[0].double() - want).abs() <= 1e-5 * float(v.abs().max())).all()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("kv", [1, 17, 32, 33, 64, 65, 512, 513])
+@pytest.mark.parametrize("D,Dv", [(8, 8), (64, 64), (80, 72), (128, 128), (200, 130)])
+def test_prefill_any_layout_many_rows(yt, D, Dv, kv, dtype):
+    """Enough query blocks (1026 workgroups) for one wave each, at both sides of the key counts
+    where that is taken, no mask, causal and bytes, against float64. Bound as in
+    test_prefill_any_layout."""
+    td = TORCH_DT[dtype]
+    g = torch.Generator(device="cuda").manual_seed(D + kv)
+    Sq = 8205
+    op = lambda r, c: torch.randn(1, 2, r, c + 1, device="cuda", generator=g).to(td)[..., 1:]  # noqa: E731
+    q, k, v = op(Sq, D), op(kv, D), op(kv, Dv)
+    i, j = torch.arange(Sq, device="cuda")[:, None], torch.arange(kv, device="cuda")[None, :]
+    drop = torch.rand(Sq, kv, device="cuda", generator=g) < 0.3
+    drop[7] = True
+    ulp = {"f32": 0.0, "bf16": 2.0 ** -8}[dtype]
+    for mask, vis in [(None, torch.ones_like(drop)), (("diag", -2000), j <= i - 2000), (~drop, ~drop)]:
+        out = yt.scaled_dot_product_attention(q, k, v, 0.0, mask=mask)
+        want = _sdpa64(q[0], k[0], v[0], 1.0 / math.sqrt(D), vis, None)
+        assert ((out[0].double() - want).abs() <= 1e-5 * float(v.double().abs().max()) + ulp * want.abs()).all()

@@ -14,13 +14,14 @@
 //     else 4 loads (contiguous over the 16 lanes r when keys do);
 //   O^T += V^T . P^T: lane (r, g) holds V[key 4 g + j][d = 16 t + r]: 16 bytes
 //     along the keys when they run contiguously, else 4 loads over d.
-// The W waves of a workgroup share the same 16 queries and each take a run of the
-// visible key blocks, with an online softmax of their own; they are merged through
-// LDS at the end. That keeps every SIMD busy at a few hundred queries and
-// evens out causal rows. 8 heads x 256 queries x 1024 keys, d = 64, transposed
-// cache, byte mask, fp32: 323 us one wave per query before, 26 us here (8.5 us of
-// it the 64 MB that the 128 workgroups read from L2, 7.5 us matrix work on the 128
-// CUs they cover); 16 heads x 1024 x 80 bf16 causal 2311 -> 127 us.
+// The W waves of a workgroup (eight, four at the largest head dims, or one: see
+// launch_any) share the same 16 queries and each take a run of the visible key
+// blocks, with an online softmax of their own; they are merged through LDS at the end.
+// That keeps every SIMD busy at a few hundred queries and evens out causal rows. 8
+// heads x 256 queries x 1024 keys, d = 64, transposed cache, byte mask, fp32: 323 us
+// one wave per query before, 26 us here (8.5 us of it the 64 MB that the 128
+// workgroups read from L2, 7.5 us matrix work on the 128 CUs they cover); 16 heads x
+// 1024 x 80 bf16 causal 2311 -> 127 us.
 
 #include <algorithm>
 
@@ -362,9 +363,9 @@ __global__ __launch_bounds__(64 * W) void attn_any_kernel(AttnArgs a) {
 
 namespace {
 
-template <class T, int NB>
+template <class T, int NB, int W>
 hipError_t launch_full(const AttnArgs& a, const dim3 grid, hipStream_t s) {
-    constexpr int NKT = NB <= 4 ? 2 : 1, W = 8;  // what the registers hold at two waves a SIMD
+    constexpr int NKT = NB <= 4 ? 2 : 1;  // what the registers hold at two waves a SIMD
     const bool kd = a.ks3 == 1, vk = a.vs2 == 1 && a.Skv >= 4;
     if (kd && vk) attn_any_kernel<T, NB, true, true, true, W, NKT><<<grid, 64 * W, 0, s>>>(a);
     else if (kd) attn_any_kernel<T, NB, true, true, false, W, NKT><<<grid, 64 * W, 0, s>>>(a);
@@ -385,11 +386,23 @@ template <class T>
 hipError_t launch_any(const AttnArgs& a, hipStream_t s) {
     const dim3 grid((unsigned)((int64_t)((a.Sq + 15) / 16) * a.B * a.Hq));
     const int d = std::max(a.D, a.Dv);
-    if (a.D == 64 && a.Dv == 64) return launch_full<T, 4>(a, grid, s);
-    if (a.D == 128 && a.Dv == 128) return launch_full<T, 8>(a, grid, s);
-    if (d <= 64) return launch_part<T, 4, 8>(a, grid, s);
-    if (d <= 128) return launch_part<T, 8, 8>(a, grid, s);
-    return launch_part<T, 16, 4>(a, grid, s);  // 64 KB of O tiles in LDS
+    // One wave a workgroup where the queries fill the chip by themselves, or the keys are one or
+    // two blocks: of eight most would idle, and all pay the merge. Many keys stay with eight,
+    // which read a block's K and V from L2 together, and under a mask, where rows see different
+    // numbers of keys, the eight even them out: there the line lies lower. Eight waves / one, us:
+    // 2048 workgroups, fp32, no mask: d 8, 16 keys 57 / 23; d 80, 16 keys 106 / 27; d 128, 128
+    // keys 89 / 44; bf16 d 64, 512 keys 125 / 85; bf16 d 128 transposed, 1024 keys 353 / 362,
+    // 2048 keys 643 / 712. Causal, fp32, d 80, 128 keys: one wave takes 0.47 of eight's time,
+    // 512 keys 1.11.
+    const bool masked = a.causal || a.mask != nullptr;
+    const unsigned wgs = grid.x;
+    const int top = wgs < 1024 ? 32 : !masked || wgs >= 8192 ? 512 : wgs >= 2048 ? 128 : 64;
+    const bool one = a.Skv <= top;
+    if (a.D == 64 && a.Dv == 64) return one ? launch_full<T, 4, 1>(a, grid, s) : launch_full<T, 4, 8>(a, grid, s);
+    if (a.D == 128 && a.Dv == 128) return one ? launch_full<T, 8, 1>(a, grid, s) : launch_full<T, 8, 8>(a, grid, s);
+    if (d <= 64) return one ? launch_part<T, 4, 1>(a, grid, s) : launch_part<T, 4, 8>(a, grid, s);
+    if (d <= 128) return one ? launch_part<T, 8, 1>(a, grid, s) : launch_part<T, 8, 8>(a, grid, s);
+    return one ? launch_part<T, 16, 1>(a, grid, s) : launch_part<T, 16, 4>(a, grid, s);  // 64 KB of O tiles in LDS
 }
 
 }  // namespace
